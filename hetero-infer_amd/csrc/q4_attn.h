@@ -3,16 +3,26 @@
 //
 // hetero/cpu_model.py:233-252 for one query token: per query head,
 // s = (q . k_t) * scale over the positions t <= pos, p = exp(s - max s),
-// o = (sum p_t v_t) / (sum p_t).  Workgroup (chunk, kv head) takes 64
-// positions and the G = nh / nkv query heads that share the kv head:
+// o = (sum p_t v_t) / (sum p_t).  Workgroup (part, kv head) takes a run of
+// 64-position chunks and the G = nh / nkv query heads that share the kv head:
 // wave g is query head g -- for the scores and the softmax lane j takes
-// position j of the chunk (all in registers), for the weighted sum of v
+// position j of a chunk (all in registers), for the weighted sum of v
 // lane i the dimensions 2i, 2i + 1.  Each wave writes its head's partial
 // result (max m, sum l, unnormalised o) and arrives at the head's counter;
-// the wave of the last chunk to arrive merges the head's parts
-// (o = sum_c e^(m_c - M) o_c / sum_c e^(m_c - M) l_c, the o sum in chunk
+// the wave of the last part to arrive merges the head's parts
+// (o = sum_c e^(m_c - M) o_c / sum_c e^(m_c - M) l_c, the o sum in part
 // order, the l sum a fixed lane tree), so there is no second launch.  The
-// result does not depend on which chunk arrives last.
+// result does not depend on which part arrives last.
+//
+// Parts.  A part is one chunk while the cache has at most attn_max_parts()
+// chunks (every chunk's loads in flight together); past that the grid stays
+// there and a workgroup walks ceil(chunks / parts) consecutive chunks with an
+// online softmax, the next chunk's rows in flight while the current one is
+// computed.  The merge is one wave per head and pays a device-scope round
+// trip per 32 parts, so what bounded long contexts was the number of parts,
+// not bytes: with a part per chunk and the merge's later loads one at a time,
+// 12345 positions (193 parts, 25 MB, 28 heads on 4 kv heads) took 63 us, and
+// take 17.5 in parts of four chunks; 32700 positions 173 and 29 us.
 #pragma once
 
 #include "q4_common.h"
@@ -27,7 +37,9 @@ constexpr int kMaxChunks = 1024;        // cap <= 65536
 constexpr int kAttnThreads = 64 * kMaxG;   // a wave per query head
 constexpr int kAttnCounters = 512;      // arrival counters after the partials (one per query head)
 constexpr int kCounterStride = 32;      // words between counters: each on its own 128-byte line
-constexpr int kMergeBatch = 36;         // chunks merged per round of loads (2304 positions in one round)
+constexpr int kMaxParts = 128;          // parts of a query head at most: two (m, l) per lane in the merge
+constexpr int kMergeBatch = 36;         // parts merged in the first round of loads (2304 positions in one round)
+constexpr int kMergeMore = 32;          // parts of each later round
 constexpr int kAttnCoherent = 16;       // cache policy sc1: device-scope stores and loads of the parts
 
 __device__ __forceinline__ uint16_t attn_f2h(float f) {
@@ -49,7 +61,7 @@ struct AttnArgs {
     uint16_t* kc;
     uint16_t* vc;
     const int64_t* pos;
-    float* part;             // [nh][n_chunks][d + 2], then kAttnCounters arrival counters
+    float* part;             // [nh][n_chunks][d + 2] (the parts first), then kAttnCounters arrival counters
     float* out;              // [nh][d]
     int nh, nkv, d, cap, n_chunks;
     float scale;
@@ -60,16 +72,32 @@ struct AttnArgs {
     const float* sin_t;
 };
 
+// Parts per query head at most (the grid's x): one workgroup per CU over the
+// kv heads, but at least 64 and at most kMaxParts.  More workgroups per CU
+// only share the vector ALUs and LDS that the chunks are bound by, and leave
+// more parts to merge: 28 heads on 4 kv heads at 12345 positions take 17.5 us
+// with 64 parts, 20.2 with 128 (9000: 15.0 and 18.8, 32700: 29.0 and 31.9);
+// 8 kv heads take 20.5 us with 32 parts and 19.8 with 64.  The same for a
+// stage's whole life, so a captured launch fits every position.
+inline int attn_max_parts(int nkv) {
+    const int p = 256 / nkv;
+    return p < 64 ? 64 : p > kMaxParts ? kMaxParts : p;
+}
+
 // ROPE: q, k and v are the raw projection outputs; the workgroup applies
 // the biases and the rotary embedding to its G query heads (as
 // rope_kv_kernel does), and the one whose chunk holds the position also
 // rotates the new key, writes the new key and value rows to the cache and
-// takes them from registers instead of the cache.  G: query heads per kv
+// takes them from registers instead of the cache.  part: this workgroup's
+// part of max_parts (the grid's x; at most kMaxParts and a.n_chunks).
+// RUNS: the cache holds more than max_parts chunks, so a part may be a run
+// of them; without it a part is one chunk, and the loop and its rescaling
+// are not compiled in (they cost the one-chunk kernel 0.3 of 8.3 us).  G: query heads per kv
 // head, D: head_dim (32, 64 or 128; a.d), template parameters so that the
 // loops over them unroll and their LDS reads are issued together.  Called
 // by the kAttnThreads threads of the workgroup.
-template <bool ROPE, int G, int D>
-__device__ __forceinline__ void attn_decode(const AttnArgs& a, int chunk, int kvh, char* lds) {
+template <bool ROPE, bool RUNS, int G, int D>
+__device__ __forceinline__ void attn_decode(const AttnArgs& a, int part, int max_parts, int kvh, char* lds) {
     static_assert(D == 32 || D == 64 || D == 128, "head_dim 32, 64 or 128");
     constexpr int NT = kAttnThreads;
     constexpr int KV = kChunk * (kMaxD / 8) / NT;            // uint4 of K (and of V) per thread at d = 128
@@ -85,34 +113,40 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, int chunk, int kv
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // uniform: the wave's resources stay scalar
     const int64_t pos = *a.pos;
-    const int c0 = chunk * kChunk;
     const int64_t lim = pos + 1 < cap ? pos + 1 : cap;      // positions [0, lim)
-    if (lim <= c0) return;                                   // past the position: no part, no arrival
-    const int valid = lim - c0 >= kChunk ? kChunk : static_cast<int>(lim - c0);
-    const int n_act = static_cast<int>((lim + kChunk - 1) / kChunk);   // chunks that arrive
+    if (lim <= 0) return;
+    const int chunks = static_cast<int>((lim + kChunk - 1) / kChunk);
+    const int per = RUNS ? (chunks + max_parts - 1) / max_parts : 1;   // chunks of a part
+    const int n_act = (chunks + per - 1) / per;              // parts that arrive
+    if (part >= n_act) return;                               // past the position: no part, no arrival
+    const int first = part * per, past = first + per < chunks ? first + per : chunks;
     constexpr int du4 = d >> 3;                              // uint4 (8 fp16) per row
-    // the chunk's new row (the position) comes from registers, not the cache
-    const bool fresh = ROPE && pos >= c0 && pos < c0 + kChunk && pos < cap;
-    const int frow = fresh ? static_cast<int>(pos - c0) : -1;
-    // every load up front: q, the chunk's K and V rows, unconditional,
-    // through resources that end with the rows to read: rows past `valid`
-    // (and a fresh row) read 0 without an access
-    {
-        const int nkv4 = (fresh ? valid - 1 : valid) * du4;
+    // the new row (the position) comes from registers, not the cache; it is
+    // in the last chunk of the last part
+    const bool fresh = ROPE && past == chunks && pos >= 0 && pos < cap;
+    const int fchunk = fresh ? chunks - 1 : -1;
+    const int frow = fresh ? static_cast<int>(pos) & (kChunk - 1) : -1;
+    uint4 kv[KV], vv[KV];
+    uint16_t fh1 = 0, fh2 = 0;                               // the fresh row's values of this thread
+    // every load of the first chunk up front: q, the chunk's K and V rows,
+    // unconditional, through resources that end with the rows to read: rows
+    // past the position (and a fresh row) read 0 without an access
+    auto load_kv = [&](int c) {
+        const int c0 = c * kChunk;
+        const int valid = lim - c0 >= kChunk ? kChunk : static_cast<int>(lim - c0);
+        const int nkv4 = (c == fchunk ? valid - 1 : valid) * du4;
         const __amdgpu_buffer_rsrc_t kr =
             buf_rsrc(a.kc + (static_cast<size_t>(kvh) * cap + c0) * d, static_cast<uint32_t>(nkv4) * 16u);
         const __amdgpu_buffer_rsrc_t vr =
             buf_rsrc(a.vc + (static_cast<size_t>(kvh) * cap + c0) * d, static_cast<uint32_t>(nkv4) * 16u);
-        uint4 kv[KV], vv[KV];
-        uint16_t fh1 = 0, fh2 = 0;                           // the fresh row's values of this thread
-        auto load_kv = [&]() {
 #pragma unroll
-            for (int r = 0; r < KV; r++) {
-                const uint32_t off = static_cast<uint32_t>(r * NT + tid) * 16u;
-                kv[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(kr, off, 0, 0));
-                vv[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(vr, off, 0, 0));
-            }
-        };
+        for (int r = 0; r < KV; r++) {
+            const uint32_t off = static_cast<uint32_t>(r * NT + tid) * 16u;
+            kv[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(kr, off, 0, 0));
+            vv[r] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(vr, off, 0, 0));
+        }
+    };
+    {
         if constexpr (ROPE) {
             // hetero/cpu_model.py:156-157 (bias) and :195-204 (RoPE), the same
             // fp32 operations as rope_kv_kernel
@@ -143,7 +177,7 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, int chunk, int kv
                     nvb = a.bias[(nh + nkv) * d + e];
                 }
             }
-            load_kv();
+            load_kv(first);
             float* qf = reinterpret_cast<float*>(&q_s[0][0]);
 #pragma unroll
             for (int r = 0; r < QR; r++) {
@@ -174,20 +208,30 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, int chunk, int kv
             const int nq4 = G * d / 4;
             float4 qv = make_float4(0.f, 0.f, 0.f, 0.f);
             if (tid < nq4) qv = reinterpret_cast<const float4*>(a.q + static_cast<size_t>(kvh * G) * d)[tid];
-            load_kv();
+            load_kv(first);
             if (tid < nq4) q_s[tid / (d / 4)][tid % (d / 4)] = qv;
         }
+    }
+    const int g = wave;                                      // this wave's query head (uniform)
+    const int h = kvh * G + g;
+    const int stride = d + 2;
+    const int i = lane;
+    constexpr int dp = d >> 1;
+    constexpr float kNegInf = -__builtin_inff();
+    float m = kNegInf, l = 0.0f, o0 = 0.0f, o1 = 0.0f;       // the part so far
+    for (int c = first; RUNS ? c < past : c == first; c++) {
         // all 64 rows but a fresh one: the rows past the ones read (past the
         // position) hold 0, so the output loop needs no bound
+        const int fr = c == fchunk ? frow : -1;
 #pragma unroll
         for (int r = 0; r < KV; r++) {
             const int e = r * NT + tid;
-            if (e < kChunk * du4 && e / du4 != frow) {
+            if (e < kChunk * du4 && e / du4 != fr) {
                 k_s[e / du4][e % du4] = kv[r];
                 v_s[e / du4][e % du4] = vv[r];
             }
         }
-        if (fresh) {
+        if (c == fchunk) {
             const int half = d >> 1;
             uint16_t* kl = reinterpret_cast<uint16_t*>(&k_s[frow][0]);
             uint16_t* vl = reinterpret_cast<uint16_t*>(&v_s[frow][0]);
@@ -198,79 +242,91 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, int chunk, int kv
                 vl[tid - half] = fh1;
             }
         }
-    }
-    __syncthreads();
-    const int g = wave;                                      // this wave's query head (uniform)
-    const int h = kvh * G + g;
-    const int stride = d + 2;
-    const int i = lane;
-    constexpr int dp = d >> 1;
-    if (g >= G) return;
-    {
-        // scores: lane j = position c0 + j, the dimensions in four
-        // interleaved partial sums
-        const int j = lane;
-        float acc[4] = {0.f, 0.f, 0.f, 0.f};
+        if (RUNS && c + 1 < past) load_kv(c + 1);
+        __syncthreads();
+        if (g < G) {
+            // scores: lane j = position 64 c + j, the dimensions in four
+            // interleaved partial sums
+            const int j = lane;
+            const int valid = lim - c * kChunk >= kChunk ? kChunk : static_cast<int>(lim - c * kChunk);
+            float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < du4; c++) {
-            const uint4 kk = k_s[j][c];
-            const float4 qa = q_s[g][2 * c], qb = q_s[g][2 * c + 1];
-            acc[0] = __builtin_fmaf(qa.x, attn_h2f(static_cast<uint16_t>(kk.x)), acc[0]);
-            acc[1] = __builtin_fmaf(qa.y, attn_h2f(static_cast<uint16_t>(kk.x >> 16)), acc[1]);
-            acc[2] = __builtin_fmaf(qa.z, attn_h2f(static_cast<uint16_t>(kk.y)), acc[2]);
-            acc[3] = __builtin_fmaf(qa.w, attn_h2f(static_cast<uint16_t>(kk.y >> 16)), acc[3]);
-            acc[0] = __builtin_fmaf(qb.x, attn_h2f(static_cast<uint16_t>(kk.z)), acc[0]);
-            acc[1] = __builtin_fmaf(qb.y, attn_h2f(static_cast<uint16_t>(kk.z >> 16)), acc[1]);
-            acc[2] = __builtin_fmaf(qb.z, attn_h2f(static_cast<uint16_t>(kk.w)), acc[2]);
-            acc[3] = __builtin_fmaf(qb.w, attn_h2f(static_cast<uint16_t>(kk.w >> 16)), acc[3]);
-        }
-        const float dot = __fadd_rn(__fadd_rn(acc[0], acc[1]), __fadd_rn(acc[2], acc[3]));
-        // softmax over the chunk (lane = position; position c0 is visible, so
-        // m is finite)
-        const float sc = j < valid ? __fmul_rn(dot, a.scale) : -__builtin_inff();
-        const float m = wave_max(sc);
-        const float p = j < valid ? expf(__fsub_rn(sc, m)) : 0.0f;
-        const float l = wave_sum(p);
-        p_s[g][j] = p;
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-        // unnormalised output: lane i = dimensions 2i, 2i + 1; positions in
-        // order (p is 0 and the V row is 0 past the valid positions); stored
-        // at device scope
-        float* my = a.part + (static_cast<size_t>(h) * n_chunks + chunk) * stride;
-        const __amdgpu_buffer_rsrc_t pr = buf_rsrc(my, static_cast<uint32_t>(stride) * 4u);
-        using u32x2 = unsigned int __attribute__((ext_vector_type(2)));
-        if (i < dp) {
-            const uint32_t* vw = reinterpret_cast<const uint32_t*>(&v_s[0][0]);
-            constexpr int kRowW = kRowU4 * 4;
+            for (int e = 0; e < du4; e++) {
+                const uint4 kk = k_s[j][e];
+                const float4 qa = q_s[g][2 * e], qb = q_s[g][2 * e + 1];
+                acc[0] = __builtin_fmaf(qa.x, attn_h2f(static_cast<uint16_t>(kk.x)), acc[0]);
+                acc[1] = __builtin_fmaf(qa.y, attn_h2f(static_cast<uint16_t>(kk.x >> 16)), acc[1]);
+                acc[2] = __builtin_fmaf(qa.z, attn_h2f(static_cast<uint16_t>(kk.y)), acc[2]);
+                acc[3] = __builtin_fmaf(qa.w, attn_h2f(static_cast<uint16_t>(kk.y >> 16)), acc[3]);
+                acc[0] = __builtin_fmaf(qb.x, attn_h2f(static_cast<uint16_t>(kk.z)), acc[0]);
+                acc[1] = __builtin_fmaf(qb.y, attn_h2f(static_cast<uint16_t>(kk.z >> 16)), acc[1]);
+                acc[2] = __builtin_fmaf(qb.z, attn_h2f(static_cast<uint16_t>(kk.w)), acc[2]);
+                acc[3] = __builtin_fmaf(qb.w, attn_h2f(static_cast<uint16_t>(kk.w >> 16)), acc[3]);
+            }
+            const float dot = __fadd_rn(__fadd_rn(acc[0], acc[1]), __fadd_rn(acc[2], acc[3]));
+            // softmax over the chunk (lane = position; position 64 c is
+            // visible, so the maximum is finite)
+            const float sc = j < valid ? __fmul_rn(dot, a.scale) : kNegInf;
+            const float mc = wave_max(sc);
+            const float p = j < valid ? expf(__fsub_rn(sc, mc)) : 0.0f;
+            const float lc = wave_sum(p);
+            p_s[g][j] = p;
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+            // unnormalised output: lane i = dimensions 2i, 2i + 1; positions
+            // in order (p is 0 and the V row is 0 past the valid positions)
             float a0 = 0.0f, a1 = 0.0f;
-            // 16 positions' V words and p values per round, loaded together
+            if (i < dp) {
+                const uint32_t* vw = reinterpret_cast<const uint32_t*>(&v_s[0][0]);
+                constexpr int kRowW = kRowU4 * 4;
+                // 16 positions' V words and p values per round, loaded together
 #pragma unroll
-            for (int s0 = 0; s0 < kChunk; s0 += 16) {
-                uint32_t w2[16];
-                float4 p4[4];
+                for (int s0 = 0; s0 < kChunk; s0 += 16) {
+                    uint32_t w2[16];
+                    float4 p4[4];
 #pragma unroll
-                for (int t = 0; t < 16; t++) w2[t] = vw[(s0 + t) * kRowW + i];
+                    for (int t = 0; t < 16; t++) w2[t] = vw[(s0 + t) * kRowW + i];
 #pragma unroll
-                for (int k = 0; k < 4; k++) p4[k] = *reinterpret_cast<const float4*>(&p_s[g][s0 + 4 * k]);
+                    for (int k = 0; k < 4; k++) p4[k] = *reinterpret_cast<const float4*>(&p_s[g][s0 + 4 * k]);
 #pragma unroll
-                for (int t = 0; t < 16; t++) {
-                    const float4 q4 = p4[t >> 2];
-                    const float pv = (t & 3) == 0 ? q4.x : (t & 3) == 1 ? q4.y : (t & 3) == 2 ? q4.z : q4.w;
-                    a0 = __builtin_fmaf(pv, attn_h2f(static_cast<uint16_t>(w2[t])), a0);
-                    a1 = __builtin_fmaf(pv, attn_h2f(static_cast<uint16_t>(w2[t] >> 16)), a1);
+                    for (int t = 0; t < 16; t++) {
+                        const float4 q4 = p4[t >> 2];
+                        const float pv = (t & 3) == 0 ? q4.x : (t & 3) == 1 ? q4.y : (t & 3) == 2 ? q4.z : q4.w;
+                        a0 = __builtin_fmaf(pv, attn_h2f(static_cast<uint16_t>(w2[t])), a0);
+                        a1 = __builtin_fmaf(pv, attn_h2f(static_cast<uint16_t>(w2[t] >> 16)), a1);
+                    }
                 }
             }
-            __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(a0), __float_as_uint(a1)}, pr,
-                                                  (2 + 2 * i) * 4u, 0, kAttnCoherent);
+            if (!RUNS || c == first) {
+                m = mc; l = lc; o0 = a0; o1 = a1;
+            } else {
+                // the part so far and this chunk, each scaled to the larger maximum
+                const float mn = fmaxf(m, mc);
+                const float so = expf(__fsub_rn(m, mn)), sn = expf(__fsub_rn(mc, mn));
+                l = __builtin_fmaf(lc, sn, __fmul_rn(l, so));
+                o0 = __builtin_fmaf(a0, sn, __fmul_rn(o0, so));
+                o1 = __builtin_fmaf(a1, sn, __fmul_rn(o1, so));
+                m = mn;
+            }
         }
+        if (RUNS && c + 1 < past) __syncthreads();                   // the chunk's rows are read: the next ones may land
+    }
+    if (g >= G) return;
+    {
+        // the part, stored at device scope
+        float* my = a.part + (static_cast<size_t>(h) * n_chunks + part) * stride;
+        const __amdgpu_buffer_rsrc_t pr = buf_rsrc(my, static_cast<uint32_t>(stride) * 4u);
+        using u32x2 = unsigned int __attribute__((ext_vector_type(2)));
+        if (i < dp)
+            __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(o0), __float_as_uint(o1)}, pr,
+                                                  (2 + 2 * i) * 4u, 0, kAttnCoherent);
         if (lane == 0)
             __builtin_amdgcn_raw_buffer_store_b64(u32x2{__float_as_uint(m), __float_as_uint(l)}, pr, 0u, 0,
                                                   kAttnCoherent);
         __builtin_amdgcn_s_waitcnt(0x0F70);                  // vmcnt(0): this wave's part is stored
     }
-    // the query head's arrival: one per chunk, the last merges (each wave
+    // the query head's arrival: one per part, the last merges (each wave
     // on its own: no workgroup barrier after the staging)
     unsigned* count = reinterpret_cast<unsigned*>(a.part + static_cast<size_t>(nh) * n_chunks * stride) +
                       h * kCounterStride;
@@ -284,59 +340,62 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, int chunk, int kv
     if (!__builtin_amdgcn_readfirstlane(last)) return;
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     {
-    // the merge of query head h: lane c takes the (m, l) of chunks c,
-    // c + 64, ...: the maximum M over all chunks, the weights e^(m_c - M)
+    // the merge of query head h: lane c takes the (m, l) of parts c and
+    // c + 64: the maximum M over all parts, the weights e^(m_c - M)
     // and the lane tree of the w_c l_c; lane i then adds w_c o_c for its
-    // dimensions 2i, 2i + 1 in chunk order, w_c read from lane c.  The first
-    // kMergeBatch chunks' o and the first 64 chunks' (m, l) are loaded in
-    // one round; loads past the arrived chunks read 0 and their weights are
-    // 0, so they add exactly nothing.
+    // dimensions 2i, 2i + 1 in part order, w_c read from lane c.  The first
+    // kMergeBatch parts' o and the (m, l) are loaded in one round, the
+    // others kMergeMore a round; loads past the arrived parts read 0 and
+    // their weights are 0, so they add exactly nothing.
     const float* ph = a.part + static_cast<size_t>(h) * n_chunks * stride;
     const __amdgpu_buffer_rsrc_t hr = buf_rsrc(ph, static_cast<uint32_t>(n_act * stride) * 4u);
-    auto ld_ml = [&](int c) {                    // (m, l) of chunk c; (0, 0) past the arrived chunks
+    auto ld_ml = [&](int c) {                    // (m, l) of part c; (0, 0) past the arrived parts
         return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(
                                               hr, static_cast<uint32_t>(c * stride) * 4u, 0, kAttnCoherent));
     };
-    auto ld_o = [&](int c) {                     // o[2i], o[2i + 1] of chunk c
+    auto ld_o = [&](int c) {                     // o[2i], o[2i + 1] of part c
         return __builtin_bit_cast(float2, __builtin_amdgcn_raw_buffer_load_b64(
                                               hr, static_cast<uint32_t>(c * stride + 2 + 2 * i) * 4u, 0,
                                               kAttnCoherent));
     };
+    static_assert(kMaxParts == 128, "the merge holds two parts' (m, l) per lane");
     float2 ob[kMergeBatch];
 #pragma unroll
     for (int c = 0; c < kMergeBatch; c++) ob[c] = ld_o(c);
-    const float2 ml0 = ld_ml(lane);
-    float mloc = lane < n_act ? ml0.x : -__builtin_inff();
-    for (int c = lane + 64; c < n_act; c += 64) mloc = fmaxf(mloc, ld_ml(c).x);
-    const float M = wave_max(mloc);
-    auto weight = [&](float2 ml, int c) {
-        return c < n_act && ml.x != -__builtin_inff() ? expf(__fsub_rn(ml.x, M)) : 0.0f;
+    const float2 ml0 = ld_ml(lane), ml1 = ld_ml(lane + 64);
+    const float m0 = lane < n_act ? ml0.x : -__builtin_inff(), m1 = lane + 64 < n_act ? ml1.x : -__builtin_inff();
+    const float M = wave_max(fmaxf(m0, m1));
+    auto weight = [&](float mc) { return mc != -__builtin_inff() ? expf(__fsub_rn(mc, M)) : 0.0f; };
+    const float w0 = weight(m0), w1 = weight(m1);    // lane c: the weights of parts c and c + 64
+    const float lloc = n_act > 64 ? __builtin_fmaf(ml1.y, w1, __fmul_rn(ml0.y, w0)) : __fmul_rn(ml0.y, w0);
+    auto wt = [&](int c) {                           // c a constant after unrolling
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c < 64 ? w0 : w1), c & 63));
     };
-    float w = weight(ml0, lane);                 // lane c: the weight of chunk c (of this round of 64)
-    float lloc = __fmul_rn(ml0.y, w);
-    float o0 = 0.0f, o1 = 0.0f;
+    float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll
     for (int c = 0; c < kMergeBatch; c++) {
-        const float wc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), c));
-        o0 = __builtin_fmaf(ob[c].x, wc, o0);
-        o1 = __builtin_fmaf(ob[c].y, wc, o1);
+        const float wc = wt(c);
+        s0 = __builtin_fmaf(ob[c].x, wc, s0);
+        s1 = __builtin_fmaf(ob[c].y, wc, s1);
     }
-    for (int c = kMergeBatch; c < n_act; c++) {
-        if (c % 64 == 0) {                       // the next round of 64 chunks' weights
-            const float2 ml = ld_ml(c + lane);
-            w = weight(ml, c + lane);
-            lloc = __builtin_fmaf(ml.y, w, lloc);
+#pragma unroll
+    for (int base = kMergeBatch; base < kMaxParts; base += kMergeMore) {
+        if (base < n_act) {
+#pragma unroll
+            for (int t = 0; t < kMergeMore && base + t < kMaxParts; t++) ob[t] = ld_o(base + t);
+#pragma unroll
+            for (int t = 0; t < kMergeMore && base + t < kMaxParts; t++) {
+                const float wc = wt(base + t);
+                s0 = __builtin_fmaf(ob[t].x, wc, s0);
+                s1 = __builtin_fmaf(ob[t].y, wc, s1);
+            }
         }
-        const float wc = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), c % 64));
-        const float2 o = ld_o(c);
-        o0 = __builtin_fmaf(o.x, wc, o0);
-        o1 = __builtin_fmaf(o.y, wc, o1);
     }
     const float L = wave_sum(lloc);
     if (i < dp) {
         float* dst = a.out + static_cast<size_t>(h) * d + 2 * i;
-        dst[0] = __fdiv_rn(o0, L);
-        dst[1] = __fdiv_rn(o1, L);
+        dst[0] = __fdiv_rn(s0, L);
+        dst[1] = __fdiv_rn(s1, L);
     }
     }
 }

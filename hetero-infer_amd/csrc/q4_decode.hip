@@ -207,19 +207,19 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const float* __restrict__
 }
 
 // ---------------------------------------------------------- attention ---
-// attn_decode of q4_attn.h as one launch over grid (chunk, kv head).
-template <bool ROPE, int G, int D>
+// attn_decode of q4_attn.h as one launch over grid (part, kv head).
+template <bool ROPE, bool RUNS, int G, int D>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) char lds[kAttnLdsBytes];
-    attn_decode<ROPE, G, D>(a, blockIdx.x, blockIdx.y, lds);
+    attn_decode<ROPE, RUNS, G, D>(a, blockIdx.x, gridDim.x, blockIdx.y, lds);
 }
 
-template <bool ROPE, int D>
+template <bool ROPE, bool RUNS, int D>
 void launch_attention_d(int G, dim3 grid, hipStream_t st, const AttnArgs& a) {
     switch (G) {
 #define Q4_ATTN_CASE(g)                                                                                      \
     case g:                                                                                                  \
-        hipLaunchKernelGGL((attn_decode_kernel<ROPE, g, D>), grid, dim3(kAttnThreads), 0, st, a);          \
+        hipLaunchKernelGGL((attn_decode_kernel<ROPE, RUNS, g, D>), grid, dim3(kAttnThreads), 0, st, a);      \
         break;
         Q4_ATTN_CASE(1) Q4_ATTN_CASE(2) Q4_ATTN_CASE(3) Q4_ATTN_CASE(4)
         Q4_ATTN_CASE(5) Q4_ATTN_CASE(6) Q4_ATTN_CASE(7) Q4_ATTN_CASE(8)
@@ -228,12 +228,17 @@ void launch_attention_d(int G, dim3 grid, hipStream_t st, const AttnArgs& a) {
     }
 }
 
-// head_dim 32, 64 or 128 (the callers check)
+// head_dim 32, 64 or 128 (the callers check); a workgroup per part and kv
+// head: a part is one chunk while the cache has no more chunks than
+// attn_max_parts, else a run of chunks (q4_attn.h)
 template <bool ROPE>
-void launch_attention(int G, dim3 grid, hipStream_t st, const AttnArgs& a) {
-    if (a.d == 128) launch_attention_d<ROPE, 128>(G, grid, st, a);
-    else if (a.d == 64) launch_attention_d<ROPE, 64>(G, grid, st, a);
-    else launch_attention_d<ROPE, 32>(G, grid, st, a);
+void launch_attention(hipStream_t st, const AttnArgs& a) {
+    const int G = a.nh / a.nkv, most = attn_max_parts(a.nkv);
+    const bool runs = a.n_chunks > most;
+    const dim3 grid(runs ? most : a.n_chunks, a.nkv);
+    if (a.d == 128) runs ? launch_attention_d<ROPE, true, 128>(G, grid, st, a) : launch_attention_d<ROPE, false, 128>(G, grid, st, a);
+    else if (a.d == 64) runs ? launch_attention_d<ROPE, true, 64>(G, grid, st, a) : launch_attention_d<ROPE, false, 64>(G, grid, st, a);
+    else runs ? launch_attention_d<ROPE, true, 32>(G, grid, st, a) : launch_attention_d<ROPE, false, 32>(G, grid, st, a);
 }
 
 // ---------------------------------------------------------------- argmax ---
@@ -489,7 +494,7 @@ int q4_attention_dev(const float* q, const uint16_t* k_cache, const uint16_t* v_
     hipStream_t st = static_cast<hipStream_t>(stream);
     const AttnArgs a{q, const_cast<uint16_t*>(k_cache), const_cast<uint16_t*>(v_cache), pos, scratch, out, n_heads,
                      n_kv, head_dim, cap, n_chunks, scale, nullptr, nullptr, nullptr, nullptr, nullptr};
-    launch_attention<false>(n_heads / n_kv, dim3(n_chunks, n_kv), st, a);
+    launch_attention<false>(st, a);
     return check_launch("q4_attention_dev");
 }
 
@@ -509,7 +514,7 @@ int q4_attention_rope_dev(const float* q, const float* k, const float* v, const 
     hipStream_t st = static_cast<hipStream_t>(stream);
     const AttnArgs a{q, k_cache, v_cache, pos, scratch, out, n_heads, n_kv, head_dim, cap, n_chunks, scale,
                      k, v, bias, cos_t, sin_t};
-    launch_attention<true>(n_heads / n_kv, dim3(n_chunks, n_kv), st, a);
+    launch_attention<true>(st, a);
     return check_launch("q4_attention_rope_dev");
 }
 

@@ -138,9 +138,10 @@ long q4_attention_scratch_floats(int n_heads, int head_dim, int cap);
  * with the maximum subtracted, weighted sum of v; query head h uses kv head
  * h / (n_heads / n_kv)).  q [n_heads][d] fp32, caches fp16 [nkv][cap][d],
  * out [n_heads][d] fp32.  One launch: the context is split in chunks of 64
- * positions (one workgroup per kv head and chunk) whose partial softmax
- * results go to scratch (q4_attention_scratch_floats); for each query
- * head, the last chunk to finish merges the head's parts.  head_dim 32, 64
+ * positions (one workgroup per kv head and chunk, or per run of chunks once
+ * the cache holds more than 64 chunks, 128 up to 2 kv heads) whose partial
+ * softmax results go to scratch (q4_attention_scratch_floats); for each query
+ * head, the last workgroup to finish merges the head's parts.  head_dim 32, 64
  * or 128; at most 8 query heads per kv head, at most 512 query heads;
  * cap <= 65536. */
 int q4_attention_dev(const float* q, const uint16_t* k_cache, const uint16_t* v_cache, const int64_t* pos,

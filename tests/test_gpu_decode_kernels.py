@@ -193,6 +193,57 @@ def test_attention(torch, lib, nh, nkv):
         assert oracle.normwise_rel(out.cpu().numpy(), ref) < ATTN_TOL, p
 
 
+@pytest.mark.parametrize("nh,nkv,d,parts", [(28, 4, 128, 64), (8, 8, 128, 64), (4, 2, 64, 128), (32, 32, 32, 64)])
+def test_attention_parts_of_several_chunks(torch, lib, nh, nkv, d, parts):
+    """Contexts on both sides of one, two and three 64-position chunks per
+    part (the grid stays at `parts` workgroups per kv head): the float64
+    softmax within the bar of the shorter contexts, counters back at zero,
+    repeated calls the same bits; and the one-launch bias + RoPE + cache
+    write form, whose new row sits in the last chunk of the last part,
+    equal to the separate calls bit for bit."""
+    rng = np.random.default_rng(19)
+    edge = parts * 64
+    cap = 2 * edge + 100
+    scale = float(np.float32(d ** -0.5))
+    dev = torch.device("cuda")
+    kc_np = rng.normal(0, 1, (nkv, cap, d)).astype(np.float16)
+    vc_np = rng.normal(0, 1, (nkv, cap, d)).astype(np.float16)
+    q_np = rng.normal(0, 1, nh * d).astype(np.float32)
+    kc, vc, tq = (torch.from_numpy(a).to(dev) for a in (kc_np, vc_np, q_np))
+    k, v = (torch.from_numpy(rng.normal(0, 1, nkv * d).astype(np.float32)).to(dev) for _ in range(2))
+    bias = torch.from_numpy(rng.normal(0, 0.1, (nh + 2 * nkv) * d).astype(np.float32)).to(dev)
+    ang = torch.arange(cap, dtype=torch.float32, device=dev)[:, None] * torch.linspace(1, 1e-4, d // 2, device=dev)
+    cos, sin = torch.cos(ang).contiguous(), torch.sin(ang).contiguous()
+    out = torch.empty(nh * d, device=dev)
+    scratch = torch.zeros(lib.q4_attention_scratch_floats(nh, d, cap), device=dev)
+
+    def attend(q, kk, vv, pos):
+        rc = lib.q4_attention_dev(q.data_ptr(), kk.data_ptr(), vv.data_ptr(), pos.data_ptr(), out.data_ptr(),
+                                  scratch.data_ptr(), nh, nkv, d, cap, scale, sp(torch))
+        assert rc == 0, q4.last_error(lib)
+        return out.clone()
+
+    for p in (edge - 1, edge, edge + 64, edge + 65, 2 * edge - 1, 2 * edge, cap - 1):
+        pos = torch.tensor([p], dtype=torch.int64, device=dev)
+        first = attend(tq, kc, vc, pos)
+        ref = attention_ref(q_np, kc_np, vc_np, p, nh, nkv, scale)
+        assert oracle.normwise_rel(first.cpu().numpy(), ref) < ATTN_TOL, p
+        assert torch.equal(first, attend(tq, kc, vc, pos)), p
+        assert int(scratch[-512 * 32:].view(torch.int32).abs().sum().item()) == 0, p
+        k1, v1, k2, v2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
+        qo = torch.empty(nh * d, device=dev)
+        rc = lib.q4_rope_kv_dev(tq.data_ptr(), k.data_ptr(), v.data_ptr(), bias.data_ptr(), cos.data_ptr(),
+                                sin.data_ptr(), pos.data_ptr(), k1.data_ptr(), v1.data_ptr(), qo.data_ptr(), nh, nkv,
+                                d, cap, sp(torch))
+        assert rc == 0, q4.last_error(lib)
+        two = attend(qo, k1, v1, pos)
+        rc = lib.q4_attention_rope_dev(tq.data_ptr(), k.data_ptr(), v.data_ptr(), bias.data_ptr(), cos.data_ptr(),
+                                       sin.data_ptr(), pos.data_ptr(), k2.data_ptr(), v2.data_ptr(), out.data_ptr(),
+                                       scratch.data_ptr(), nh, nkv, d, cap, scale, sp(torch))
+        assert rc == 0, q4.last_error(lib)
+        assert torch.equal(two, out) and torch.equal(k1, k2) and torch.equal(v1, v2), p
+
+
 def test_attention_long_context(torch, lib):
     """Contexts past one round of the merge's loads (36 chunks of 64
     positions): up to 79 chunks, the ones past the first round merged by
