@@ -1,5 +1,6 @@
-// Small-M GEMV on the int8 matrix cores (up to 8 activation rows, gs 64; the
-// library takes it from 3 rows, below which the streaming kernel is faster).
+// Small-M GEMV on the int8 matrix cores (up to 16 activation rows, gs 64; the
+// library takes it from kMfMinRows rows, below which the streaming kernel is
+// faster).
 //
 // The arithmetic is the reference's x86 path of kernel/q4gemv.c:232-301 for
 // every row of x: x quantised to int16 once per row (:244-270), an exact
@@ -9,63 +10,67 @@
 // steps stay in the order above, so the result is bit-identical to the
 // streaming kernel and to the reference.
 //
-// Integer dots.  v_mfma_i32_32x32x32_i8 takes A (32 x 32, int8) from x and
-// B (32 x 32, int8) from the weights.  A row of A is one byte plane of one
-// activation row; the 32 columns of B are 32 weight rows.  xq = 256 * xh + xl
-// with xh the signed high byte and xl the unsigned low byte; A carries
-// xl ^ 0x80 (= xl - 128, a signed byte) and xh, plus two rows of ones, so
-//   idot = D[xl] + 256 * D[xh] + 128 * D[ones]          (exact in int32)
-// Weights are 0..15, already valid signed bytes: the low and high nibbles of
-// each packed word go to two MFMAs (even and odd k), and the A operand holds
-// the matching even/odd bytes of x.  A rows: 0..7 xl of activation rows
-// 0..7, 8..15 xh (loaded), 16 and 20 ones (made in registers), the rest
-// zero, which puts every plane an output needs into the same lane of D.
+// Integer dots.  One v_mfma_i32_16x16x64_i8 covers a group: A (16 x 64, int8)
+// is one byte plane of x, B (64 x 16) the group's nibbles of 16 weight rows.
+// xq = 256 * xh + xl with xh the signed high byte and xl the unsigned low
+// byte; A carries xl ^ 0x80 (= xl - 128, a signed byte) and xh, and a third
+// MFMA with A = 1 gives the nibbles' sum, so
+//   idot = D[xl] + 256 * D[xh] + 128 * D[1]          (exact in int32)
+// Up to 8 rows of x (MB = 8) both planes share one A: row 2 m + p is plane p
+// of activation row m; 9..16 rows (MB = 16) take an A per plane.  Either way
+// a lane of D holds both planes of its activation rows.
+// A lane's 16 bytes of B are two packed words: even nibbles, odd nibbles of
+// each; the order of k inside a group is free as long as A matches.
 //
-// Work split.  A workgroup owns a tile of 32 weight rows (16 when 32-row
-// tiles would leave CUs idle; PAIR: 32 gate rows and the same 32 up rows,
-// one A operand for both) and runs S waves over K
-// in windows of kMfRing*S groups, kMfRing consecutive groups per wave, each
-// wave streaming its groups through a register ring of kMfRing (the next
-// window's loads are in flight while the window's terms are chained).  Each group's
-// fp32 term goes to an LDS table; after a barrier one lane per (activation
-// row, weight row) adds the window's terms in ascending group order.  The K
-// split keeps enough waves in flight for the 3584-row shapes; the ordered
-// chain keeps it exact.
+// Vector-memory results return in issue order, so a wave that also loads the
+// x operand (1 to 4 times the bytes of its weights, from the L2) holds few
+// weights in flight and waits for them behind x.  The waves of a workgroup
+// therefore have separate jobs:
+//   * 8 compute waves load nothing but weights, into a register ring, and
+//     take everything else from LDS;
+//   * one copy wave moves the x operand and the group sums into LDS by
+//     global->LDS copies ahead of their window, another the scales and biases;
+//   * MB / 4 chain waves add the terms in group order, a window behind.
+// A workgroup owns a tile of 16 weight rows (PAIR: 16 gate rows and the same
+// 16 up rows, one x operand for both) and walks K in windows of 16 groups,
+// two groups per compute wave; workgroups are persistent over tiles, so the
+// ring never drains between them.  A compute wave writes its groups' fp32
+// terms to an LDS table (two buffers), and after the window's one barrier a
+// lane per (weight row, activation row) adds the window's terms in ascending
+// group order.  All the matrices of a grouped call are one launch.
 //
-// Loads per pair of groups and wave: per matrix two loads of 16 rows x 64
-// contiguous bytes (the two groups of each row; 32-byte pieces per row made
-// twice the L2 requests), turned into the B operands of the two groups by
-// v_permlane16_swap and v_permlane32_swap; per group the A operand (the 32
-// lanes of rows 0..15, 32 bytes each) and the xsum of the lane's four
-// activation rows.  Scales and biases come once per window: the lane's
-// row, 8 groups in 16 bytes (the window's kMfRing of them used), scales in
-// k-half 0 and biases in k-half 1, exchanged across the halves (when the
-// group count is a multiple of 8; else one 2-byte load each per group).
+// Measured (Qwen2.5-7B shapes, graph replays, against the earlier form: x
+// operand in the register ring, a launch per matrix and per 8 rows): MLP
+// block 61.5 -> 50.5 us at 3..8 rows, 115 -> 64 at 16; q/k/v at 16 rows 57
+// -> 15; down_proj at 16 rows 49 -> 25.  What bounds it now is a window's
+// instructions and LDS traffic: with the copies and the weights' loads taken
+// out it still needs 0.5 us a window (0.75 paired) where the weights alone
+// need 0.43 (0.86), and the two overlap only in part across the barrier.
+// Measured and not kept: 12 compute waves (24 groups a window), two
+// workgroups per CU, a deeper ring.
 #pragma once
 
 #include "q4_common.h"
 
 namespace q4k {
 
-// groups per wave and window (ring: 2 slots of 2 groups).  8 groups (4
-// slots) measured slower: q_proj at 8 rows 11.45 against 10.9 us, the MLP
-// block 61.6 against 61.2 us -- fewer loads queued per CU wait less.
-constexpr int kMfRing = 4;
-constexpr int kMfArows = 16;        // A rows stored per (group, k-half): xl 0..7, xh 8..15
+constexpr int kMfRowsMax = 16;               // activation rows of one launch
 
-// x of up to 8 rows, prepared for the small-M MFMA kernel.  Grid (P, 8):
+// x of M <= MB rows, prepared for the small-M kernel.  Grid (P, MB):
 // workgroup (p, m) takes row slot m (slots >= M write zeros) and the p-th
 // slice of its groups.  The fp32 steps are xprep_kernel's:
-//   xa[((g*2 + h)*16 + r)*8 + s]  uint32: A row r, k-half h of group g;
-//                                 s 0..3 even-k bytes of words 4h..4h+3 of
-//                                 the group, 4..7 the odd-k bytes
-//   xsum_t[g*8 + m], xscale[m]
+//   xa      MB = 16: per group 2 KiB, plane p (low, high) at 1024 p: lane
+//           (q, m) = 16 q + m, 16 bytes; MB = 8: 1 KiB, lane 16 q + 2 m + p.
+//           Word j of the group is half j & 1 of quarter q = (j >> 2) |
+//           (j & 2): its even-k bytes, then its odd-k bytes.
+//   xsum_t[g * MB + m], xscale[m]
 // Every workgroup of a row stages the whole row in LDS by 16-byte loads all
 // issued at once (one memory round trip) and takes its amax; the group sums
 // and the quantisation of its slice then read LDS.
 constexpr int kMfPrepMaxK = 32768;           // floats of one x row staged in LDS
+template <int MB>
 __global__ __launch_bounds__(1024) void xprep_mf_kernel(const float* __restrict__ x, int M, int n_in,
-                                                        uint32_t* __restrict__ xa, float* __restrict__ xsum_t,
+                                                        uint2* __restrict__ xa, float* __restrict__ xsum_t,
                                                         float* __restrict__ xscale_out) {
     extern __shared__ float4 xrow4[];                            // [n_in / 4]
     const int m = blockIdx.y;
@@ -73,13 +78,16 @@ __global__ __launch_bounds__(1024) void xprep_mf_kernel(const float* __restrict_
     const int G = n_in >> 6;
     const int gs = (G + gridDim.x - 1) / gridDim.x;              // groups per slice
     const int g0 = blockIdx.x * gs, g1 = g0 + gs < G ? g0 + gs : G;
+    // the 8 bytes (even k, odd k) of word j of the row in plane p
+    auto at = [&](int j, int p) -> uint2& {
+        const int g = j >> 3, q = ((j >> 2) & 1) | (j & 2), s = j & 1;
+        const size_t lane = MB == 16 ? static_cast<size_t>(g * 2 + p) * 64 + q * 16 + m
+                                     : static_cast<size_t>(g) * 64 + q * 16 + 2 * m + p;
+        return xa[lane * 2 + s];
+    };
     if (m >= M) {
-        for (int i = g0 * 16 + tid; i < g1 * 16; i += nt) {
-            const int s = i & 7, gh = i >> 3;
-            xa[(static_cast<size_t>(gh) * kMfArows + m) * 8 + s] = 0u;
-            xa[(static_cast<size_t>(gh) * kMfArows + 8 + m) * 8 + s] = 0u;
-        }
-        for (int g = g0 + tid; g < g1; g += nt) xsum_t[static_cast<size_t>(g) * 8 + m] = 0.0f;
+        for (int j = g0 * 8 + tid; j < g1 * 8; j += nt) at(j, 0) = at(j, 1) = make_uint2(0u, 0u);
+        for (int g = g0 + tid; g < g1; g += nt) xsum_t[static_cast<size_t>(g) * MB + m] = 0.0f;
         if (tid == 0 && blockIdx.x == 0) xscale_out[m] = 1.0f;
         return;
     }
@@ -134,7 +142,7 @@ __global__ __launch_bounds__(1024) void xprep_mf_kernel(const float* __restrict_
             s = __fadd_rn(s, q.z);
             s = __fadd_rn(s, q.w);
         }
-        xsum_t[static_cast<size_t>(g) * 8 + m] = s;
+        xsum_t[static_cast<size_t>(g) * MB + m] = s;
     }
     __syncthreads();
     const float inv = s_inv;
@@ -152,302 +160,400 @@ __global__ __launch_bounds__(1024) void xprep_mf_kernel(const float* __restrict_
             if (n & 1) { lo |= xlb << sh; ho |= xhb << sh; }
             else       { le |= xlb << sh; he |= xhb << sh; }
         }
-        const int g = j >> 3, h = (j >> 2) & 1, wd = j & 3;
-        uint32_t* base = xa + static_cast<size_t>(g * 2 + h) * kMfArows * 8;
-        base[m * 8 + wd] = le ^ 0x80808080u;
-        base[m * 8 + 4 + wd] = lo ^ 0x80808080u;
-        base[(8 + m) * 8 + wd] = he;
-        base[(8 + m) * 8 + 4 + wd] = ho;
+        at(j, 0) = make_uint2(le ^ 0x80808080u, lo ^ 0x80808080u);
+        at(j, 1) = make_uint2(he, ho);
     }
 }
-
-// One ring slot: a pair of consecutive groups.
-template <bool PAIR>
-struct MfSlot {
-    uint4 w[PAIR ? 2 : 1][2];   // per matrix: rows 0..15 and 16..31 of the tile, 64 bytes of each row
-                                //   (the pair's two groups) over four lanes; permuted into B at use
-    uint4 xe[2], xo[2];         // per group: A operand, even and odd k
-    float4 xs[2];               // per group: xsum of activation rows 4h..4h+3
-    uint32_t s[PAIR ? 2 : 1][2], b[PAIR ? 2 : 1][2];   // per matrix and group without SB8 (fp16, low half)
-};
 
 typedef int mf_v4i __attribute__((ext_vector_type(4)));
-typedef int mf_v16i __attribute__((ext_vector_type(16)));
 
-// Weight-side arguments: one matrix, or (PAIR) gate in 0 and up in 1.
+// The matrices of one launch, sharing x: matrix k's 16-row tiles are tiles
+// tile0[k] .. tile0[k + 1] - 1.  PAIR: gate in 0 and up in 1, n[0] rows each,
+// tiles tile0[0] .. tile0[1] - 1, out[0].
 struct MfMats {
-    const uint32_t* w[2];
-    const uint16_t* s[2];
-    const uint16_t* b[2];
+    const uint32_t* w[4];
+    const uint16_t* s[4];
+    const uint16_t* b[4];
+    float* out[4];
+    int n[4];
+    int tile0[5];
 };
 
-__device__ __forceinline__ mf_v4i lo_nibbles(const uint4& w) {
-    return {static_cast<int>(w.x & 0x0F0F0F0Fu), static_cast<int>(w.y & 0x0F0F0F0Fu),
-            static_cast<int>(w.z & 0x0F0F0F0Fu), static_cast<int>(w.w & 0x0F0F0F0Fu)};
-}
-__device__ __forceinline__ mf_v4i hi_nibbles(const uint4& w) {
-    return {static_cast<int>((w.x >> 4) & 0x0F0F0F0Fu), static_cast<int>((w.y >> 4) & 0x0F0F0F0Fu),
-            static_cast<int>((w.z >> 4) & 0x0F0F0F0Fu), static_cast<int>((w.w >> 4) & 0x0F0F0F0Fu)};
+// B of one group: two packed words, each its even then its odd nibbles.
+__device__ __forceinline__ mf_v4i mf_nibbles(uint32_t a, uint32_t b) {
+    return {static_cast<int>(a & 0x0F0F0F0Fu), static_cast<int>((a >> 4) & 0x0F0F0F0Fu),
+            static_cast<int>(b & 0x0F0F0F0Fu), static_cast<int>((b >> 4) & 0x0F0F0F0Fu)};
 }
 
-// [a0 a1 a2 a3], [b0 b1 b2 b3] (quarters of 16 lanes) -> [a0 b0 a1 b1],
-// [a2 b2 a3 b3]: the odd quarters of the first swap with the even quarters
-// of the second, then the upper halves of the first with the lower halves
-// of the second.
-__device__ __forceinline__ void pair_permute(uint32_t i0, uint32_t i1, uint32_t& b0, uint32_t& b1) {
-    const auto pq = __builtin_amdgcn_permlane16_swap(i0, i1, false, false);    // [a0 b0 a2 b2], [a1 b1 a3 b3]
-    const auto r = __builtin_amdgcn_permlane32_swap(pq[0], pq[1], false, false);
-    b0 = r[0];
-    b1 = r[1];
+// The waves of a workgroup meet once per window.  Each makes its own LDS
+// accesses and copies complete before it (a compute or chain wave its LDS
+// accesses, not the weights in flight; the copy wave the copies of the next
+// window), which a fence would do by waiting for everything.
+__device__ __forceinline__ void mf_barrier() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
+constexpr int kMfWaitLds = 0xC07F;                               // s_waitcnt lgkmcnt(0)
+constexpr int mf_wait_copies(int n) {                            // s_waitcnt vmcnt(n), at most the counter's 63
+    return n > 63 ? 0xCF7F : 0x0F70 | (n & 15) | ((n >> 4) << 14);
 }
 
-// fp16 k of the 8 packed in a uint4 (k = 0..7, wave-uniform)
-__device__ __forceinline__ uint32_t half_of(const uint4& v, int k) {
-    const uint32_t d = k < 2 ? v.x : k < 4 ? v.y : k < 6 ? v.z : v.w;
-    return (k & 1) ? d >> 16 : d & 0xFFFFu;
-}
+// Sizes of an instance.  EVEN: an even group count and 4-byte aligned scales
+// and biases, copied two groups at a time; else one at a time, zero-extended.
+// The ring's depth hardly matters (2, 4 and 8 windows within 2 %: the copies
+// and the compute of a window set the pace, not the weights), so it is kept
+// short: every slot is a copy of the loop's code.
+constexpr int kMfWaves = 8;                                       // compute waves
+template <bool PAIR, int MB, bool EVEN>
+struct MfShape {
+    static constexpr int NM = PAIR ? 2 : 1;
+    static constexpr int win = 2 * kMfWaves;                      // groups per window
+    static constexpr int chain = MB / 4;                          // chain waves: 16 MB lanes
+    static constexpr int threads = 64 * (kMfWaves + chain + 2);
+    static constexpr int depth = PAIR && MB == 16 ? 2 : 4;        // windows of weights in a wave's ring (128 VGPRs)
+    static constexpr int xslots = PAIR && MB == 16 ? 2 : 3;       // windows of x in LDS (160 KB)
+    static constexpr int sbslots = PAIR && MB == 16 ? 6 : 8;      // and of scales and biases
+    static constexpr int xbytes = win * MB * 128;                 // x operand of a window
+    static constexpr int xcopies = xbytes / 1024 + 1;             // and its group sums (up to a KiB)
+    static constexpr int sbcopies = (EVEN ? 4 : 8) * NM;
+    static constexpr int sbbytes = sbcopies * 256;
+    static constexpr int tbytes = NM * win * 16 * MB * 4;         // terms of a window
+    static constexpr int xs0 = xslots * xbytes, sb0 = xs0 + xslots * 1024, t0 = sb0 + sbslots * sbbytes;
+    static constexpr int lds = t0 + 2 * tbytes;
+};
 
-// out[m][row] for m < M (PAIR: h[m][row] = SiLU(gate) * up), row stride ldo.
-// Grid: one workgroup per tile of TR rows; block: 64 * S threads (S = 4 or
-// 8: with the x operand in the ring, two waves per SIMD).
-// SB8: the group count is a multiple of 8 (scales/biases by window).
-// TR: weight rows per tile, 32, or 16 (B columns 16..31 dead) to spread a
-// matrix of few rows over twice the workgroups.
-template <bool PAIR, int S, bool SB8, int TR>
-__global__ __launch_bounds__(64 * S) void gemv_mfma_kernel(MfMats mt, int N, int K, int M,
-                                                         const uint32_t* __restrict__ xa,
-                                                         const float* __restrict__ xsum_t,
-                                                         const float* __restrict__ xscale,
-                                                         float* __restrict__ out, int ldo) {
-    constexpr int NM = PAIR ? 2 : 1;
-    static_assert(S == 4 || S == 8, "the chain lanes are waves 0..3; the ring fits two waves per SIMD");
-    constexpr int GW = kMfRing * S;
-    // terms of one window, [NM][GW][8 activation rows][32 weight rows]: a
-    // term store (fixed group and row of x) and a chain load (fixed group)
-    // touch 32 consecutive floats per half wave, so no bank conflict past
-    // the two halves
-    extern __shared__ float tbl[];
-    const int tid = threadIdx.x;
-    const int lane = tid & 63, j = lane & 31, h = lane >> 5;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int G = K >> 6;
-    const int nwin = (G + GW - 1) / GW;
-    const uint32_t rowb = static_cast<uint32_t>(K) >> 1;          // bytes of a weight row
-
-    // the lane's weight row; rows past N read 0 and are not stored
-    static_assert(TR == 32 || (TR == 16 && !PAIR), "16-row tiles for one matrix");
-    const int row = blockIdx.x * TR + j;
-    const bool live = row < N && j < TR;
-    __amdgpu_buffer_rsrc_t rw[NM], rs[NM], rb[NM];
+// The copy wave's copies (plain device functions: the copy builtin in a
+// lambda of the kernel keeps the compiler from emitting the host stub).
+template <int MB, int WIN>
+__device__ __forceinline__ void mf_copy_x(char* x_s, char* xs_s, const __amdgpu_buffer_rsrc_t rx,
+                                          const __amdgpu_buffer_rsrc_t rxs, int t, int lane) {
+    typedef __attribute__((address_space(3))) void* lds_ptr;
+    constexpr int XB = WIN * MB * 128;
+    const uint32_t base = static_cast<uint32_t>(t) * XB + static_cast<uint32_t>(lane) * 16u;
 #pragma unroll
-    for (int k = 0; k < NM; k++) {
-        rw[k] = buf_rsrc(mt.w[k], static_cast<uint32_t>(N) * rowb);
-        rs[k] = buf_rsrc(mt.s[k], static_cast<uint32_t>(N) * G * 2u);
-        rb[k] = buf_rsrc(mt.b[k], static_cast<uint32_t>(N) * G * 2u);
-    }
-    const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xa, static_cast<uint32_t>(G) * 2u * kMfArows * 32u);
-    const __amdgpu_buffer_rsrc_t rxs = buf_rsrc(xsum_t, static_cast<uint32_t>(G) * 32u);
-    // per-lane offsets at group 0, each below 2^31 (the host checks the
-    // matrix sizes), and a dead bit OR-ed in after the group's offset is
-    // added: rows past N and the A rows not stored read 0 without an access.
-    // A group past the last one adds 2^31 itself; the sum of two in-range
-    // parts never reaches 2^32.
-    // Weight loads: lane l reads row (l % 16) (+16 for the second load) at
-    // byte 16 * (l / 16) of the pair's 64 bytes.
-    const int lrow = blockIdx.x * TR + (lane & 15);
-    const uint32_t olw = static_cast<uint32_t>(lrow < N ? lrow : 0) * rowb + static_cast<uint32_t>(lane >> 4) * 16u;
-    const uint32_t deadw0 = lrow < N ? 0u : kOutOfRange, deadw1 = lrow + 16 < N ? 0u : kOutOfRange;
-    const uint32_t row16 = 16u * rowb;
-    const uint32_t rowc = live ? static_cast<uint32_t>(row) : 0u;
-    const uint32_t og = rowc * static_cast<uint32_t>(G) * 2u;
-    const uint32_t dead = live ? 0u : kOutOfRange;
-    const uint32_t ox = static_cast<uint32_t>(h * kMfArows + (j & 15)) * 32u;
-    const uint32_t deadx = j < kMfArows ? 0u : kOutOfRange;
-    const uint32_t onesv = (j == 16 || j == 20) ? 0x01010101u : 0u;   // A rows 16 and 20
-    const uint32_t oxs = static_cast<uint32_t>(h) * 16u;
+    for (int i = 0; i < XB / 1024; i++)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr)(x_s + i * 1024), 16, base + i * 1024u, 0, 0, 0);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        rxs, (lds_ptr)xs_s, 16, static_cast<uint32_t>(t) * (WIN * MB * 4) + static_cast<uint32_t>(lane) * 16u, 0, 0, 0);
+}
 
-    // slot of groups (g, g + 1), g even
-    auto load = [&](MfSlot<PAIR>& sl, int g) {
-        const bool gv = g < G;                                       // uniform
-        const uint32_t dw = gv ? static_cast<uint32_t>(g) * 32u : kOutOfRange;
-        __builtin_amdgcn_sched_barrier(0);
-        // default cache policy: the 64 bytes a lane group reads share their
-        // 128-byte line with the row's next pair, read by the next slot
+// A window's scales (copies 0 .. n/2 - 1) and biases of one tile: EVEN, word
+// (group pair p, row r) at 4 (16 p + r); else word (group g, row r).
+// Groups past G and rows past the tile read 0 (or, within the tile, a value
+// that no term uses).
+template <bool EVEN, int WIN>
+__device__ __forceinline__ void mf_copy_sb(char* s_s, const __amdgpu_buffer_rsrc_t rs, const __amdgpu_buffer_rsrc_t rb,
+                                           int G, int t, int lane) {
+    typedef __attribute__((address_space(3))) void* lds_ptr;
+    constexpr int n = EVEN ? WIN / 8 : WIN / 4, size = EVEN ? 4 : 2;
+    const uint32_t off = static_cast<uint32_t>(lane & 15) * G * 2u + static_cast<uint32_t>(t) * (WIN * 2u) +
+                         static_cast<uint32_t>(lane >> 4) * size;
 #pragma unroll
-        for (int k = 0; k < NM; k++) {
-            sl.w[k][0] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw[k], (olw + dw) | deadw0, 0, 0));
-            if constexpr (TR == 32)
-                sl.w[k][1] = __builtin_bit_cast(
-                    uint4, __builtin_amdgcn_raw_buffer_load_b128(rw[k], (olw + row16 + dw) | deadw1, 0, 0));
-            else
-                sl.w[k][1] = make_uint4(0u, 0u, 0u, 0u);
+    for (int i = 0; i < n; i++) {
+        if constexpr (EVEN) {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)(s_s + i * 256), 4, off + i * 16u, 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr)(s_s + (n + i) * 256), 4, off + i * 16u, 0, 0, 0);
+        } else {
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr)(s_s + i * 256), 2, off + i * 8u, 0, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr)(s_s + (n + i) * 256), 2, off + i * 8u, 0, 0, 0);
         }
+    }
+}
+
+// Matrix of a tile (wave-uniform): a chain of selects over the arguments.
+__device__ __forceinline__ int mf_matrix(const MfMats& mt, int tile) {
+    return (tile >= mt.tile0[1]) + (tile >= mt.tile0[2]) + (tile >= mt.tile0[3]);
+}
+
+// out[k][m][row] for m < M (PAIR: h[m][row] = SiLU(gate) * up).  Grid: up to
+// one workgroup per tile, persistent; block: MfShape::threads.
+template <bool PAIR, int MB, bool EVEN>
+__global__ __launch_bounds__((MfShape<PAIR, MB, EVEN>::threads)) void gemv_mfma_kernel(
+    MfMats mt, int tiles, int K, int M, const uint32_t* __restrict__ xa, const float* __restrict__ xsum_t,
+    const float* __restrict__ xscale) {
+    using S = MfShape<PAIR, MB, EVEN>;
+    constexpr int NM = S::NM, WIN = S::win, W = kMfWaves, MPL = MB / 4;   // MPL: activation rows per lane of D
+    extern __shared__ __attribute__((aligned(16))) char mf_lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int G = K >> 6, nwin = (G + WIN - 1) / WIN;
+    const int mine = (tiles - static_cast<int>(blockIdx.x) + static_cast<int>(gridDim.x) - 1) / static_cast<int>(gridDim.x);
+    const int iters = mine * nwin;                               // windows of this workgroup
+    const int meets = (iters + S::depth - 1) / S::depth * S::depth;   // barriers before the last
+    const uint32_t rowb = static_cast<uint32_t>(K) >> 1;         // bytes of a weight row
+    // rows [row0, row0 + 16) of matrix k as a buffer of `stride` bytes a row
+    // (past the last tile: empty)
+    auto rows_of = [&](const void* p, int k, int row0, uint32_t stride, bool live) {
+        int rows = mt.n[PAIR ? 0 : k] - row0;
+        rows = !live || rows < 0 ? 0 : rows > 16 ? 16 : rows;
+        return buf_rsrc(static_cast<const char*>(p) + static_cast<size_t>(row0) * stride,
+                        static_cast<uint32_t>(rows) * stride);
+    };
+
+    if (wave < W) {
+        // ---- compute waves: groups 2 wave, 2 wave + 1 of each window
+        const int q = lane >> 4, col = lane & 15;
+        // xscale of the lane's activation rows, by scalar loads: a vector load
+        // would count among the ring's loads in every wait of the loop.  Bit
+        // masks, not selects, which become one load at a per-lane index.
+        float xsc[MPL];
 #pragma unroll
-        for (int e = 0; e < 2; e++) {
-            const bool ge = g + e < G;                               // uniform
-            const uint32_t dg = ge ? static_cast<uint32_t>(g + e) * 2u : kOutOfRange;
-            const uint32_t dx = ge ? static_cast<uint32_t>(g + e) * (2u * kMfArows * 32u) : kOutOfRange;
-            const uint32_t dxs = ge ? static_cast<uint32_t>(g + e) * 32u : kOutOfRange;
-            if constexpr (!SB8) {
+        for (int i = 0; i < MPL; i++) {
+            uint32_t v = 0;
 #pragma unroll
-                for (int k = 0; k < NM; k++) {
-                    sl.s[k][e] = __builtin_amdgcn_raw_buffer_load_b16(rs[k], (og + dg) | dead, 0, 0);
-                    sl.b[k][e] = __builtin_amdgcn_raw_buffer_load_b16(rb[k], (og + dg) | dead, 0, 0);
+            for (int k = 0; k < 4; k++) v |= __float_as_uint(xscale[MPL * k + i]) & (q == k ? ~0u : 0u);
+            xsc[i] = __uint_as_float(v);
+        }
+        uint4 ring[S::depth][NM];
+        int lt = 0, ltile = blockIdx.x;                          // window and tile of the next load
+        __amdgpu_buffer_rsrc_t rw[NM];                           // its rows
+        auto tile_rows = [&]() {
+            const bool live = ltile < tiles;
+            const int k = PAIR || !live ? 0 : mf_matrix(mt, ltile);
+            const int row0 = live ? (ltile - mt.tile0[k]) * 16 : 0;
+#pragma unroll
+            for (int e = 0; e < NM; e++) rw[e] = rows_of(mt.w[PAIR ? e : k], k, row0, rowb, live);
+        };
+        const uint32_t lw = static_cast<uint32_t>(col) * rowb + static_cast<uint32_t>(q) * 16u;
+        auto load = [&](uint4 (&r)[NM]) {
+            if (lt == 0) tile_rows();
+            const int g = lt * WIN + 2 * wave;
+            const uint32_t off = lw + (g < G ? static_cast<uint32_t>(g) * 32u : kOutOfRange);
+            __builtin_amdgcn_sched_barrier(0);
+            // default cache policy: a row's 128-byte line is shared with the
+            // next wave's groups
+#pragma unroll
+            for (int e = 0; e < NM; e++)
+                r[e] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rw[e], off, 0, 0));
+            __builtin_amdgcn_sched_barrier(0);
+            if (++lt == nwin) {
+                lt = 0;
+                ltile += gridDim.x;
+            }
+        };
+        const mf_v4i ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101}, zero = {};
+        // the LDS operands of a window: A per group and plane, the group sums
+        // of the lane's activation rows, scales and biases (fp16 words)
+        struct Ops {
+            mf_v4i a[2][MB / 8];
+            float xs[2][MPL];
+            uint32_t s[NM][EVEN ? 1 : 2], b[NM][EVEN ? 1 : 2];
+        };
+        int xslot = 0, sslot = 0, tslot = 0;                     // of the next operands; of the next terms
+        auto operands = [&](Ops& o) {
+            const char* x_s = mf_lds + xslot * S::xbytes + wave * (2 * MB * 128) + lane * 16;
+            const char* xs_s = mf_lds + S::xs0 + xslot * 1024 + (2 * wave * MB + MPL * q) * 4;
+            const char* s_s = mf_lds + S::sb0 + sslot * S::sbbytes + ((EVEN ? 1 : 2) * wave * 16 + col) * 4;
+#pragma unroll
+            for (int g = 0; g < 2; g++) {
+#pragma unroll
+                for (int p = 0; p < MB / 8; p++)
+                    o.a[g][p] = *reinterpret_cast<const mf_v4i*>(x_s + (g * (MB / 8) + p) * 1024);
+#pragma unroll
+                for (int i = 0; i < MPL; i++) o.xs[g][i] = reinterpret_cast<const float*>(xs_s + g * MB * 4)[i];
+            }
+#pragma unroll
+            for (int e = 0; e < NM; e++)
+#pragma unroll
+                for (int g = 0; g < (EVEN ? 1 : 2); g++) {
+                    o.s[e][g] = *reinterpret_cast<const uint32_t*>(s_s + e * (S::sbbytes / NM) + g * 64);
+                    o.b[e][g] = *reinterpret_cast<const uint32_t*>(s_s + e * (S::sbbytes / NM) + S::sbbytes / (2 * NM) + g * 64);
                 }
-            }
-            sl.xe[e] = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rx, (ox + dx) | deadx, 0, 0));
-            sl.xo[e] = __builtin_bit_cast(uint4,
-                                          __builtin_amdgcn_raw_buffer_load_b128(rx, (ox + dx + 16u) | deadx, 0, 0));
-            sl.xs[e] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rxs, oxs + dxs, 0, 0));
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // SB8: 8 groups of scales (k-half 0) or biases (k-half 1) of the lane's
-    // row in 16 bytes, from the window's first group of the wave
-    auto load_sb = [&](uint4 (&sb)[NM], int g) {
-        const bool gv = g < G;                                       // uniform
-        const uint32_t dg = gv ? static_cast<uint32_t>(g) * 2u : kOutOfRange;
-        __builtin_amdgcn_sched_barrier(0);
-        // both loads on every lane, the other half's through a dead offset:
-        // no divergent branch around a load
-        const uint32_t ds = h == 0 ? dead : kOutOfRange, db = h == 0 ? kOutOfRange : dead;
+            xslot = xslot + 1 == S::xslots ? 0 : xslot + 1;
+            sslot = sslot + 1 == S::sbslots ? 0 : sslot + 1;
+        };
+        auto window = [&](const Ops& o, const uint4 (&r)[NM]) {
+            // lane (row, quarter q) holds words 4q .. 4q + 3 of the pair's 16:
+            // swapping the upper half of one register with the lower half of
+            // another leaves one group in each, its words in the order of
+            // xprep_mf_kernel
+            char* t_s = mf_lds + S::t0 + tslot * S::tbytes + (2 * wave * 16 + col) * (MB * 4) + q * (MPL * 4);
 #pragma unroll
-        for (int k = 0; k < NM; k++) {
-            const uint4 a = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rs[k], (og + dg) | ds, 0, 0));
-            const uint4 c = __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rb[k], (og + dg) | db, 0, 0));
-            sb[k] = make_uint4(a.x | c.x, a.y | c.y, a.z | c.z, a.w | c.w);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-
-    // xscale of the lane's four activation rows (4h .. 4h+3): the eight
-    // values by scalar loads (uniform addresses), picked per k-half.  A
-    // vector load here would be one more vector-memory result the loop
-    // header's wait accounting merges with the ring, and the first group of
-    // every window then waited for the whole ring.
-    float xsc[4];
-    {
-        // a bit mask, not a select: a select of the two loads became one
-        // load at a per-lane index, i.e. an array in scratch memory
-        const uint32_t hm = 0u - static_cast<uint32_t>(h);
+            for (int e = 0; e < NM; e++) {
+                const auto p0 = __builtin_amdgcn_permlane32_swap(r[e].x, r[e].z, false, false);
+                const auto p1 = __builtin_amdgcn_permlane32_swap(r[e].y, r[e].w, false, false);
+                mf_v4i d0[2], dh[2], d1[2];
 #pragma unroll
-        for (int mm = 0; mm < 4; mm++)
-            xsc[mm] = __uint_as_float((__float_as_uint(xscale[4 + mm]) & hm) | (__float_as_uint(xscale[mm]) & ~hm));
-    }
-
-    constexpr int kSlots = kMfRing / 2;
-    MfSlot<PAIR> ring[kSlots];
-    uint4 sb_next[NM];
-    const int g_wave = wave * kMfRing;                               // the wave's first group of a window
-    if constexpr (SB8) load_sb(sb_next, g_wave);
+                for (int g = 0; g < 2; g++) {
+                    const mf_v4i b = mf_nibbles(p0[g], p1[g]);
+                    d1[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, b, zero, 0, 0, 0);
+                    d0[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(o.a[g][0], b, zero, 0, 0, 0);
+                    if constexpr (MB == 16) dh[g] = __builtin_amdgcn_mfma_i32_16x16x64_i8(o.a[g][1], b, zero, 0, 0, 0);
+                }
 #pragma unroll
-    for (int d = 0; d < kSlots; d++) load(ring[d], g_wave + 2 * d);
-
-    // chain lanes: waves 0..3, activation row 2*wave + h, weight row j
-    const int cm = 2 * wave + h;
-    const bool chain = wave < 4 && 2 * wave < M;                     // uniform
-    float acc[NM];
+                for (int g = 0; g < 2; g++) {
+                    const float sc = h2f(static_cast<uint16_t>(EVEN ? o.s[e][0] >> (16 * g) : o.s[e][g]));
+                    const float bi = h2f(static_cast<uint16_t>(EVEN ? o.b[e][0] >> (16 * g) : o.b[e][g]));
+                    float term[MPL];
 #pragma unroll
-    for (int k = 0; k < NM; k++) acc[k] = 0.0f;
-    for (int t = 0; t < nwin; t++) {
-        const int g0 = t * GW + g_wave;
-        // this window's scales and biases: own half plus the other half's
-        uint4 sv[NM], bv[NM];
-        if constexpr (SB8) {
-#pragma unroll
-            for (int k = 0; k < NM; k++) {
-                uint4 other;
-                other.x = __shfl_xor(sb_next[k].x, 32);
-                other.y = __shfl_xor(sb_next[k].y, 32);
-                other.z = __shfl_xor(sb_next[k].z, 32);
-                other.w = __shfl_xor(sb_next[k].w, 32);
-                sv[k] = h == 0 ? sb_next[k] : other;
-                bv[k] = h == 0 ? other : sb_next[k];
-            }
-            load_sb(sb_next, g0 + GW);
-        }
-#pragma unroll
-        for (int d = 0; d < kSlots; d++) {
-            const MfSlot<PAIR>& sl = ring[d];
-            // B operands of the slot's two groups: from [a0 a1 a2 a3] (rows
-            // 0..15) and [b0 b1 b2 b3] (rows 16..31), quarters of 16 lanes,
-            // to [a0 b0 a1 b1] (first group) and [a2 b2 a3 b3] (second)
-            mf_v4i bw[NM][2][2];                                     // [matrix][group][even, odd k]
-#pragma unroll
-            for (int k = 0; k < NM; k++) {
-                uint4 b0, b1;
-                pair_permute(sl.w[k][0].x, sl.w[k][1].x, b0.x, b1.x);
-                pair_permute(sl.w[k][0].y, sl.w[k][1].y, b0.y, b1.y);
-                pair_permute(sl.w[k][0].z, sl.w[k][1].z, b0.z, b1.z);
-                pair_permute(sl.w[k][0].w, sl.w[k][1].w, b0.w, b1.w);
-                bw[k][0][0] = lo_nibbles(b0);
-                bw[k][0][1] = hi_nibbles(b0);
-                bw[k][1][0] = lo_nibbles(b1);
-                bw[k][1][1] = hi_nibbles(b1);
-            }
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const uint4 xe = make_uint4(sl.xe[e].x | onesv, sl.xe[e].y | onesv, sl.xe[e].z | onesv,
-                                            sl.xe[e].w | onesv);
-                const uint4 xo = make_uint4(sl.xo[e].x | onesv, sl.xo[e].y | onesv, sl.xo[e].z | onesv,
-                                            sl.xo[e].w | onesv);
-                const mf_v4i ae = __builtin_bit_cast(mf_v4i, xe), ao = __builtin_bit_cast(mf_v4i, xo);
-                const float xs4[4] = {sl.xs[e].x, sl.xs[e].y, sl.xs[e].z, sl.xs[e].w};
-                const int gi = 2 * d + e;                            // group of the wave's 8
-                const int gl = wave * kMfRing + gi;                  // group within the window
-#pragma unroll
-                for (int k = 0; k < NM; k++) {
-                    mf_v16i D = {};
-                    D = __builtin_amdgcn_mfma_i32_32x32x32_i8(ae, bw[k][e][0], D, 0, 0, 0);
-                    D = __builtin_amdgcn_mfma_i32_32x32x32_i8(ao, bw[k][e][1], D, 0, 0, 0);
-                    uint32_t sraw, braw;
-                    if constexpr (SB8) {
-                        sraw = half_of(sv[k], gi);
-                        braw = half_of(bv[k], gi);
-                    } else {
-                        sraw = sl.s[k][e];
-                        braw = sl.b[k][e];
-                    }
-                    const float sc = h2f(static_cast<uint16_t>(sraw)), bi = h2f(static_cast<uint16_t>(braw));
-                    float* tk = tbl + (k * GW + gl) * 256;
-#pragma unroll
-                    for (int mm = 0; mm < 4; mm++) {
+                    for (int i = 0; i < MPL; i++) {
                         // kernel/q4gemv.c:173-180 with xq = 256 xh + (xl' + 128)
-                        const int32_t idot = D[mm] + D[4 + mm] * 256 + D[8] * 128;
-                        const float dot = __fmul_rn(xsc[mm], static_cast<float>(idot));
-                        const float bx = __fmul_rn(bi, xs4[mm]);
-                        tk[(4 * h + mm) * 32 + j] = __fmaf_rn(sc, dot, bx);
+                        const int32_t lo = MB == 16 ? d0[g][i] : d0[g][2 * (i & 1)];
+                        const int32_t hi = MB == 16 ? dh[g][i] : d0[g][2 * (i & 1) + 1];
+                        const int32_t idot = lo + hi * 256 + d1[g][0] * 128;
+                        const float dot = __fmul_rn(xsc[i], static_cast<float>(idot));
+                        term[i] = __fmaf_rn(sc, dot, __fmul_rn(bi, o.xs[g][i]));
                     }
+                    char* to = t_s + (e * WIN + g) * (16 * MB * 4);
+                    if constexpr (MB == 16)
+                        *reinterpret_cast<float4*>(to) = make_float4(term[0], term[1], term[2], term[3]);
+                    else
+                        *reinterpret_cast<float2*>(to) = make_float2(term[0], term[1]);
                 }
             }
-            load(ring[d], g0 + GW + 2 * d);                          // the next window's pair
-        }
-        __syncthreads();
-        if (chain) {
-            const int n = G - t * GW < GW ? G - t * GW : GW;
+            tslot ^= 1;
+        };
+        // whole rings, the first one only filled: the loads go out (past the
+        // last window: empty) on every path, so that the waits for the ring
+        // never assume a skipped load.  A window's LDS operands are read
+        // while the window before is computed.  (One site for each slot's
+        // load: code that runs cold costs about 0.4 us per KB.)
+        Ops ops[2];
+        static_assert(S::depth % 2 == 0, "the operands alternate");
+#pragma unroll 1
+        for (int it = -S::depth; it < iters; it += S::depth)
 #pragma unroll
-            for (int k = 0; k < NM; k++) {
-                const float* tp = tbl + k * GW * 256 + cm * 32 + j;
-                float a = acc[k];
-                int g = 0;
-                for (; g + 8 <= n; g += 8) {
-                    float v[8];
-#pragma unroll
-                    for (int i = 0; i < 8; i++) v[i] = tp[(g + i) * 256];
-#pragma unroll
-                    for (int i = 0; i < 8; i++) a = __fadd_rn(a, v[i]);
+            for (int d = 0; d < S::depth; d++) {
+                if (it >= 0) {                                   // uniform
+                    if (d == 0 && it == 0) {
+                        mf_barrier();                            // window 0 is in LDS
+                        operands(ops[0]);
+                        __builtin_amdgcn_s_waitcnt(kMfWaitLds);
+                    }
+                    mf_barrier();                                // window it + d + 1 is in LDS
+                    operands(ops[(d + 1) & 1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    if (it + d < iters) window(ops[d & 1], ring[d]);
                 }
-                for (; g < n; g++) a = __fadd_rn(a, tp[g * 256]);
-                acc[k] = a;
+                load(ring[d]);
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_s_waitcnt(kMfWaitLds);          // the terms are in LDS
             }
-        }
-        __syncthreads();
+        mf_barrier();
+        return;
     }
-    if (!chain || !live || cm >= M) return;
-    if constexpr (PAIR)
-        out[static_cast<size_t>(cm) * ldo + row] = silu_mul(acc[0], acc[1]);
-    else
-        out[static_cast<size_t>(cm) * ldo + row] = acc[0];
+
+    if (wave < W + S::chain) {
+        // ---- chain waves: lane (weight row col, activation row m)
+        const int t = (wave - W) * 64 + lane, col = t / MB, m = t % MB;
+        float acc[NM];
+#pragma unroll
+        for (int e = 0; e < NM; e++) acc[e] = 0.0f;
+        int win = 0, tile = blockIdx.x;
+        mf_barrier();
+        mf_barrier();
+        for (int it = 0; it < iters; it++) {
+            mf_barrier();                                        // window it's terms are in the table
+            const float* tp = reinterpret_cast<const float*>(mf_lds + S::t0 + (it & 1) * S::tbytes) + t;
+            const int n = G - win * WIN < WIN ? G - win * WIN : WIN;
+            float v[NM][WIN];
+#pragma unroll
+            for (int e = 0; e < NM; e++)
+#pragma unroll
+                for (int g = 0; g < WIN; g++) v[e][g] = tp[(e * WIN + g) * (16 * MB)];
+            __builtin_amdgcn_s_waitcnt(kMfWaitLds);              // read before the next barrier
+            if (n == WIN) {
+#pragma unroll
+                for (int g = 0; g < WIN; g++)
+#pragma unroll
+                    for (int e = 0; e < NM; e++) acc[e] = __fadd_rn(acc[e], v[e][g]);
+            } else {
+#pragma unroll
+                for (int g = 0; g < WIN; g++)
+#pragma unroll
+                    for (int e = 0; e < NM; e++)
+                        if (g < n) acc[e] = __fadd_rn(acc[e], v[e][g]);
+            }
+            if (++win == nwin) {
+                const int k = PAIR ? 0 : mf_matrix(mt, tile);
+                const int row = (tile - mt.tile0[k]) * 16 + col, N = mt.n[k];
+                if (row < N && m < M) {
+                    float* o = mt.out[k] + static_cast<size_t>(m) * N + row;
+                    if constexpr (PAIR) *o = silu_mul(acc[0], acc[1]);
+                    else *o = acc[0];
+                }
+                win = 0;
+                tile += gridDim.x;
+#pragma unroll
+                for (int e = 0; e < NM; e++) acc[e] = 0.0f;
+            }
+        }
+#pragma unroll 1
+        for (int it = iters; it < meets; it++) mf_barrier();
+        return;
+    }
+
+    if (wave == W + S::chain) {
+        // ---- the x copy wave: a window's operand and group sums, up to
+        // xslots - 1 windows ahead of its use
+        const __amdgpu_buffer_rsrc_t rx = buf_rsrc(xa, static_cast<uint32_t>(G) * (MB * 128u));
+        const __amdgpu_buffer_rsrc_t rxs = buf_rsrc(xsum_t, static_cast<uint32_t>(G) * (MB * 4u));
+        int win = 0, slot = 0;                                   // of the next copy
+        auto copy = [&]() {
+            mf_copy_x<MB, WIN>(mf_lds + slot * S::xbytes, mf_lds + S::xs0 + slot * 1024, rx, rxs, win, lane);
+            slot = slot + 1 == S::xslots ? 0 : slot + 1;
+            win = win + 1 == nwin ? 0 : win + 1;
+        };
+#pragma unroll 1
+        for (int it = -S::xslots; it < iters; it++) {
+            if (it >= 0) {
+                if (it == 0) {
+                    __builtin_amdgcn_s_waitcnt(mf_wait_copies((S::xslots - 1) * S::xcopies));
+                    mf_barrier();                                // window 0
+                }
+                __builtin_amdgcn_s_waitcnt(mf_wait_copies((S::xslots - 2) * S::xcopies));
+                mf_barrier();                                    // window it + 1
+            }
+            copy();                                              // window it + xslots
+        }
+        __builtin_amdgcn_s_waitcnt(mf_wait_copies(0));           // none may land after the workgroup ends
+#pragma unroll 1
+        for (int it = iters; it <= meets; it++) mf_barrier();
+        return;
+    }
+
+    // ---- the scale copy wave: a window's scales and biases, up to sbslots - 1
+    // windows ahead (they come from HBM: in the x wave's queue they would hold back
+    // the x copies, which the L2 holds)
+    int win = 0, tile = blockIdx.x, slot = 0;                    // of the next copy
+    __amdgpu_buffer_rsrc_t rs[NM], rb[NM];
+    auto tile_rows = [&]() {
+        const bool live = tile < tiles;
+        const int k = PAIR || !live ? 0 : mf_matrix(mt, tile);
+        const int row0 = live ? (tile - mt.tile0[k]) * 16 : 0;
+#pragma unroll
+        for (int e = 0; e < NM; e++) {
+            rs[e] = rows_of(mt.s[PAIR ? e : k], k, row0, static_cast<uint32_t>(G) * 2u, live);
+            rb[e] = rows_of(mt.b[PAIR ? e : k], k, row0, static_cast<uint32_t>(G) * 2u, live);
+        }
+    };
+    auto copy = [&]() {
+        if (win == 0) tile_rows();
+#pragma unroll
+        for (int e = 0; e < NM; e++)
+            mf_copy_sb<EVEN, WIN>(mf_lds + S::sb0 + slot * S::sbbytes + e * (S::sbbytes / NM), rs[e], rb[e], G, win, lane);
+        slot = slot + 1 == S::sbslots ? 0 : slot + 1;
+        if (++win == nwin) {
+            win = 0;
+            tile += gridDim.x;
+        }
+    };
+#pragma unroll 1
+    for (int it = -S::sbslots; it < iters; it++) {
+        if (it >= 0) {
+            if (it == 0) {
+                __builtin_amdgcn_s_waitcnt(mf_wait_copies((S::sbslots - 1) * S::sbcopies));
+                mf_barrier();                                    // window 0
+            }
+            __builtin_amdgcn_s_waitcnt(mf_wait_copies((S::sbslots - 2) * S::sbcopies));
+            mf_barrier();                                        // window it + 1
+        }
+        copy();                                                  // window it + sbslots
+    }
+    __builtin_amdgcn_s_waitcnt(mf_wait_copies(0));
+#pragma unroll 1
+    for (int it = iters; it <= meets; it++) mf_barrier();
 }
 
 }  // namespace q4k

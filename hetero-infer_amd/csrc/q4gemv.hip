@@ -615,7 +615,7 @@ int ensure_ws(Workspace& ws, hipStream_t st, size_t words, size_t groups) {
     const size_t cw = words < 4096 ? 4096 : words, cg = groups < 1024 ? 1024 : groups;
     if (int rc = grow(ws, ws.planes, kWsPlanes, (ws.fixed ? words : cw) * sizeof(uint4), st, "x")) return rc;
     if (int rc = grow(ws, ws.xsum, kWsXsum, (ws.fixed ? groups : cg) * sizeof(float), st, "x")) return rc;
-    return grow(ws, ws.xscale, kWsXscale, kMaxM * sizeof(float), st, "x");
+    return grow(ws, ws.xscale, kWsXscale, q4k::kMfRowsMax * sizeof(float), st, "x");
 }
 
 template <int MR>
@@ -789,88 +789,100 @@ int gemv_split(const uint32_t* w, const uint16_t* s, const uint16_t* b, const fl
     return 0;
 }
 
-template <bool PAIR, int S, bool SB8, int TR>
-int launch_mfma_k(const q4k::MfMats& mt, int n, int n_in, int m, const Workspace& ws, float* out, hipStream_t st) {
-    auto kern = q4k::gemv_mfma_kernel<PAIR, S, SB8, TR>;
-    constexpr size_t lds = (PAIR ? 2 : 1) * 256 * q4k::kMfRing * S * sizeof(float);
+template <bool PAIR, int MB, bool EVEN>
+int launch_mfma_k(const q4k::MfMats& mt, int tiles, int n_in, int m, const Workspace& ws, hipStream_t st) {
+    using S = q4k::MfShape<PAIR, MB, EVEN>;
+    static_assert(S::lds <= static_cast<int>(kStreamLdsMax), "the LDS of one CU");
+    auto kern = q4k::gemv_mfma_kernel<PAIR, MB, EVEN>;
     static std::atomic<uint64_t> lds_raised{0};
-    if (int rc = q4k::raise_lds_limit(reinterpret_cast<const void*>(kern), lds, lds_raised)) return rc;
-    const int tiles = (n + TR - 1) / TR;
-    hipLaunchKernelGGL(kern, dim3(tiles), dim3(64 * S), lds, st, mt, n, n_in, m,
-                       reinterpret_cast<const uint32_t*>(ws.planes), ws.xsum, ws.xscale, out, n);
+    if (int rc = q4k::raise_lds_limit(reinterpret_cast<const void*>(kern), S::lds, lds_raised)) return rc;
+    // workgroups are persistent over their tiles: no more than are resident
+    static std::atomic<int> resident{0};
+    int per_cu = resident.load(std::memory_order_relaxed);
+    if (!per_cu) {
+        HIP_TRY(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(kern), S::threads,
+                                                             S::lds));
+        if (per_cu < 1) per_cu = 1;
+        resident.store(per_cu, std::memory_order_relaxed);
+    }
+    const int most = per_cu * num_cus();
+    hipLaunchKernelGGL(kern, dim3(tiles < most ? tiles : most), dim3(S::threads), S::lds, st, mt, tiles, n_in, m,
+                       reinterpret_cast<const uint32_t*>(ws.planes), ws.xsum, ws.xscale);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(Q4_EHIP, "mfma gemv launch: %s", hipGetErrorString(e));
-    return 1;
-}
-
-template <bool PAIR, bool SB8>
-int launch_mfma_s(const q4k::MfMats& mt, int n, int n_in, int m, const Workspace& ws, float* out, hipStream_t st) {
-    // One workgroup per CU holds a fixed number of weight bytes in flight
-    // (the register ring), so the workgroups must cover the CUs: 16-row
-    // tiles of 8 waves when 32-row tiles would leave CUs idle (one matrix of
-    // 3584 rows: 224 tiles), 32-row tiles of 8 waves while they do not fill
-    // the CUs twice, else 4 waves.
-    const int tiles = (n + 31) / 32, cus = num_cus();
-    if constexpr (!PAIR)
-        if (tiles < cus) return launch_mfma_k<PAIR, 8, SB8, 16>(mt, n, n_in, m, ws, out, st);
-    return tiles < 2 * cus ? launch_mfma_k<PAIR, 8, SB8, 32>(mt, n, n_in, m, ws, out, st)
-                           : launch_mfma_k<PAIR, 4, SB8, 32>(mt, n, n_in, m, ws, out, st);
-}
-
-// Rows of x from which the matrix-core path is used.  Its cost does not
-// depend on the row count; the streaming kernel's grows with it (Qwen2.5-7B
-// MLP block: 60 us at 2 rows and 80 us at 3-4 rows streaming, 64 us on the
-// matrix cores; q_proj about even at 3-4 rows).
-constexpr int kMfMinRows = 3;
-
-// Small-M GEMV on the int8 matrix cores (q4_mfma_m.h): kMfMinRows <= m <= kMaxM,
-// gs 64, n_in <= 32768, x 16-byte aligned, every byte offset into the
-// matrix below 2^31.  PAIR: mt holds gate and up, out receives
-// SiLU(gate) * up.  x is prepared into the stream's workspace by
-// xprep_mf_kernel.  Returns 1 if it launched, 0 if the shape is not one it
-// takes, <0 on error.
-bool mfma_takes(int m, int n, int n_in, int gs, const float* x) {
-    if (m < kMfMinRows || m > kMaxM || gs != 64 || n_in <= 0 || n <= 0 || n_in > q4k::kMfPrepMaxK) return false;
-    if (reinterpret_cast<uintptr_t>(x) & 15) return false;
-    // (n + 32 rows: a tile's second weight load starts 16 rows past the first)
-    const long G = n_in / 64;
-    return static_cast<long>(n + 32) * (n_in / 2) < (1L << 31) && static_cast<long>(n) * G * 2 < (1L << 31);
-}
-
-// x of m rows quantised into the stream's workspace for the matrix-core
-// kernel (xprep_mf_kernel); every later launch on the stream reads it.
-int mfma_prep(const float* x, int m, int n_in, hipStream_t st, Workspace& ws) {
-    const long G = n_in / 64;
-    int rc = ensure_ws(ws, st, static_cast<size_t>(G) * 2 * q4k::kMfArows * 2, static_cast<size_t>(G) * 8);
-    if (rc) return rc;
-    static std::atomic<uint64_t> prep_raised{0};
-    if ((rc = q4k::raise_lds_limit(reinterpret_cast<const void*>(q4k::xprep_mf_kernel),
-                                   q4k::kMfPrepMaxK * sizeof(float), prep_raised)))
-        return rc;
-    // each row's groups in slices of at least 32 over up to 8 workgroups
-    // (every workgroup of a row reads the whole row for its amax)
-    const int slices = static_cast<int>(G / 32 < 1 ? 1 : (G / 32 > 8 ? 8 : G / 32));
-    hipLaunchKernelGGL(q4k::xprep_mf_kernel, dim3(slices, kMaxM), dim3(1024), static_cast<size_t>(n_in) * sizeof(float),
-                       st, x, m, n_in, reinterpret_cast<uint32_t*>(ws.planes), ws.xsum, ws.xscale);
-    HIP_TRY(hipGetLastError());
     return 0;
 }
 
-// The matrix-core GEMV on x prepared by mfma_prep.  Returns 1 (launched) or <0.
-int mfma_main(const q4k::MfMats& mt, bool pair, float* out, int m, int n, int n_in, hipStream_t st,
-              const Workspace& ws) {
-    const bool sb8 = (n_in / 64) % 8 == 0;
-    if (pair) return sb8 ? launch_mfma_s<true, true>(mt, n, n_in, m, ws, out, st)
-                         : launch_mfma_s<true, false>(mt, n, n_in, m, ws, out, st);
-    return sb8 ? launch_mfma_s<false, true>(mt, n, n_in, m, ws, out, st)
-               : launch_mfma_s<false, false>(mt, n, n_in, m, ws, out, st);
+// Rows of x from which the matrix-core path is used.  Its cost does not
+// depend on the row count (up to 8); the streaming kernel's grows with it.
+// Qwen2.5-7B MLP block: streaming 57 us at 2 rows and 80 at 3-4, matrix cores
+// 50.5; q_proj at 2 rows 7.7 us streaming, 10.2 on the matrix cores.
+constexpr int kMfMinRows = 3;
+
+// Small-M GEMV on the int8 matrix cores (q4_mfma_m.h): kMfMinRows to
+// kMfRowsMax rows, gs 64, n_in <= 32768, x 16-byte aligned.
+bool mfma_takes(int m, int n_in, int gs, const float* x) {
+    return m >= kMfMinRows && m <= q4k::kMfRowsMax && gs == 64 && n_in > 0 && n_in <= q4k::kMfPrepMaxK &&
+           !(reinterpret_cast<uintptr_t>(x) & 15);
 }
 
-int gemv_mfma(const q4k::MfMats& mt, bool pair, const float* x, float* out, int m, int n, int n_in, int gs,
-              hipStream_t st, Workspace& ws) {
-    if (!mfma_takes(m, n, n_in, gs, x)) return 0;
-    if (int rc = mfma_prep(x, m, n_in, st, ws)) return rc;
-    return mfma_main(mt, pair, out, m, n, n_in, st, ws);
+// Rows of the next block of a call with `left` rows to go: up to 16 where
+// the matrix cores take them, else up to kMaxM.
+int block_rows(int left, int n_in, int gs, const float* x) {
+    if (left > kMaxM && mfma_takes(q4k::kMfRowsMax, n_in, gs, x))
+        return left < q4k::kMfRowsMax ? left : q4k::kMfRowsMax;
+    return left < kMaxM ? left : kMaxM;
+}
+
+// The matrix-core GEMV of m rows (mfma_takes) over up to kMaxMats matrices
+// that share x: x quantised into the stream's workspace (xprep_mf_kernel),
+// then one launch.  pair: matrices 0 and 1 are gate and up, out[0] receives
+// SiLU(gate) * up.
+int gemv_mfma(int count, const uint32_t* const* w, const uint16_t* const* s, const uint16_t* const* b,
+              float* const* out, const int* n_out, bool pair, const float* x, int m, int n_in, hipStream_t st,
+              Workspace& ws) {
+    q4k::MfMats mt{};
+    uintptr_t sb = 0;
+    int tiles = 0;
+    static_assert(kMaxMats == 4, "MfMats holds four matrices");
+    for (int k = 0; k < kMaxMats; k++) {
+        const int kk = k < count ? k : count - 1;
+        mt.w[k] = w[kk]; mt.s[k] = s[kk]; mt.b[k] = b[kk]; mt.out[k] = out[kk];
+        mt.n[k] = n_out[kk];
+        mt.tile0[k] = tiles;
+        if (k < (pair ? 1 : count)) tiles += (n_out[k] + 15) / 16;
+        sb |= reinterpret_cast<uintptr_t>(s[kk]) | reinterpret_cast<uintptr_t>(b[kk]);
+    }
+    mt.tile0[kMaxMats] = tiles;
+    if (tiles == 0) return 0;
+    const int G = n_in / 64, mb = m > 8 ? 16 : 8;
+    // sized for 16 rows from the first call on (so that a later capture of a
+    // call with more rows finds its workspace), except for the fixed scratch
+    const int wsb = ws.fixed ? mb : 16;
+    int rc = ensure_ws(ws, st, static_cast<size_t>(G) * wsb * 8, static_cast<size_t>(G) * wsb);
+    if (rc) return rc;
+    // each row's groups in slices of at least 32 over up to 8 workgroups
+    // (every workgroup of a row reads the whole row for its amax)
+    const int slices = G / 32 < 1 ? 1 : (G / 32 > 8 ? 8 : G / 32);
+    static std::atomic<uint64_t> raised8{0}, raised16{0};
+    auto prep = mb == 16 ? q4k::xprep_mf_kernel<16> : q4k::xprep_mf_kernel<8>;
+    if ((rc = q4k::raise_lds_limit(reinterpret_cast<const void*>(prep), q4k::kMfPrepMaxK * sizeof(float),
+                                   mb == 16 ? raised16 : raised8)))
+        return rc;
+    hipLaunchKernelGGL(prep, dim3(slices, mb), dim3(1024), static_cast<size_t>(n_in) * sizeof(float), st, x, m, n_in,
+                       reinterpret_cast<uint2*>(ws.planes), ws.xsum, ws.xscale);
+    HIP_TRY(hipGetLastError());
+    const bool even = G % 2 == 0 && !(sb & 3);
+    if (pair) {
+        if (mb == 16) return even ? launch_mfma_k<true, 16, true>(mt, tiles, n_in, m, ws, st)
+                                  : launch_mfma_k<true, 16, false>(mt, tiles, n_in, m, ws, st);
+        return even ? launch_mfma_k<true, 8, true>(mt, tiles, n_in, m, ws, st)
+                    : launch_mfma_k<true, 8, false>(mt, tiles, n_in, m, ws, st);
+    }
+    if (mb == 16) return even ? launch_mfma_k<false, 16, true>(mt, tiles, n_in, m, ws, st)
+                              : launch_mfma_k<false, 16, false>(mt, tiles, n_in, m, ws, st);
+    return even ? launch_mfma_k<false, 8, true>(mt, tiles, n_in, m, ws, st)
+                : launch_mfma_k<false, 8, false>(mt, tiles, n_in, m, ws, st);
 }
 
 // ROWS of the reference build being replaced (kernel/build.sh:7, -DROWS):
@@ -923,7 +935,7 @@ int multi_tails(int count, const uint32_t* const* w, const uint16_t* const* scal
 int gemv_rows_int(const uint32_t* w, const uint16_t* s, const uint16_t* b, const float* x,
                   float* out, int m, int n_out, int n_in, int gs, hipStream_t st, Workspace& ws);
 
-// GEMV of m (<= kMaxM) rows already on the device, as the reference build
+// GEMV of m (block_rows) rows already on the device, as the reference build
 // with ROWS = rows_block() computes it: the integer path, then the tail rows.
 int gemv_rows(const uint32_t* w, const uint16_t* s, const uint16_t* b, const float* x,
               float* out, int m, int n_out, int n_in, int gs, hipStream_t st, Workspace& ws) {
@@ -931,16 +943,11 @@ int gemv_rows(const uint32_t* w, const uint16_t* s, const uint16_t* b, const flo
     return tail_rows(w, s, b, x, out, m, n_out, n_in, gs, st);
 }
 
-// The integer path for every row: the matrix cores for kMfMinRows..8 rows,
-// else fused when possible.
+// The integer path for every row: the matrix cores where they take the
+// rows, else fused when possible.
 int gemv_rows_int(const uint32_t* w, const uint16_t* s, const uint16_t* b, const float* x,
                   float* out, int m, int n_out, int n_in, int gs, hipStream_t st, Workspace& ws) {
-    if (m >= kMfMinRows) {
-        const q4k::MfMats mt{{w, w}, {s, s}, {b, b}};
-        const int rc = gemv_mfma(mt, false, x, out, m, n_out, n_in, gs, st, ws);
-        if (rc < 0) return rc;
-        if (rc == 1) return 0;
-    }
+    if (mfma_takes(m, n_in, gs, x)) return gemv_mfma(1, &w, &s, &b, &out, &n_out, false, x, m, n_in, st, ws);
     MatList ml{};
     ml.w[0] = w; ml.s[0] = s; ml.b[0] = b; ml.out[0] = out; ml.n_out[0] = n_out;
     ml.row_begin[0] = 0;
@@ -1101,8 +1108,8 @@ int gemv_host(const uint32_t* w, const uint16_t* s, const uint16_t* b, const flo
     memcpy(d->pin_x, x, nx * sizeof(float));
     HIP_TRY(hipMemcpyAsync(d->dev_x, d->pin_x, nx * sizeof(float), hipMemcpyHostToDevice, d->stream));
     Workspace& ws = d->ws[d->stream];
-    for (int m0 = 0; m0 < m; m0 += kMaxM) {
-        const int mm = m - m0 < kMaxM ? m - m0 : kMaxM;
+    for (int m0 = 0, mm; m0 < m; m0 += mm) {
+        mm = block_rows(m - m0, n_in, gs, d->dev_x);
         rc = gemv_rows(r->w, r->s, r->b, d->dev_x + static_cast<size_t>(m0) * n_in,
                        d->dev_out + static_cast<size_t>(m0) * n_out, mm, n_out, n_in, gs,
                        d->stream, ws);
@@ -1160,7 +1167,7 @@ constexpr int kNoAllocMaxIn = 32768;
 constexpr size_t kScrPlanes = static_cast<size_t>(kMaxM) * (kNoAllocMaxIn / 8);   // uint4
 constexpr size_t kScrXsum = static_cast<size_t>(kMaxM) * (kNoAllocMaxIn / 64);    // floats
 constexpr size_t kScrXscale = 64;                                                  // floats
-static_assert(kScrPlanes >= static_cast<size_t>(kNoAllocMaxIn / 64) * 2 * q4k::kMfArows * 2,
+static_assert(kScrPlanes >= static_cast<size_t>(kNoAllocMaxIn / 64) * 64,
               "the matrix-core prep fits the planes");
 static __device__ __align__(256) uint4 scratch[kScrPlanes + (kScrXsum + kScrXscale) / 4];
 
@@ -1402,8 +1409,8 @@ int q4_gemv_dev(const uint32_t* w, const uint16_t* scales, const uint16_t* biase
         if ((rc = current_device(&dev))) return rc;
         ws = &g_dev[dev].ws[st];
     }
-    for (int m0 = 0; m0 < m; m0 += kMaxM) {
-        const int mm = m - m0 < kMaxM ? m - m0 : kMaxM;
+    for (int m0 = 0, mm; m0 < m; m0 += mm) {
+        mm = block_rows(m - m0, n_in, gs, x);
         rc = gemv_rows(w, scales, biases, x + static_cast<size_t>(m0) * n_in,
                        out + static_cast<size_t>(m0) * n_out, mm, n_out, n_in, gs, st, *ws);
         if (rc) return rc;
@@ -1449,46 +1456,47 @@ int q4_gemv_multi_dev(int count, const uint32_t* const* w, const uint16_t* const
     if (m == 0) return 0;
     if (!x) return fail(Q4_EARG, "null x");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    if (m < kMfMinRows) {  // one grouped streaming launch; more rows: a matrix-core launch per matrix
-        MatList ml{};
-        ml.row_begin[0] = 0;
-        for (int k = 0; k < kMaxMats; k++) {
-            const int kk = k < count ? k : count - 1;
-            ml.w[k] = w[kk]; ml.s[k] = scales[kk]; ml.b[k] = biases[kk]; ml.out[k] = out[kk];
-            ml.n_out[k] = k < count ? n_out[k] : 0;
-            ml.row_begin[k + 1] = ml.row_begin[k] + ml.n_out[k];
+    // blocks of rows: 3..16 on the matrix cores, one launch for every matrix
+    // with x quantised once; 1..2 rows as one grouped streaming launch; a
+    // shape that neither takes, a call per matrix
+    for (int m0 = 0, mm; m0 < m; m0 += mm) {
+        mm = block_rows(m - m0, n_in, gs, x);
+        const float* xm = x + static_cast<size_t>(m0) * n_in;
+        float* om[kMaxMats];
+        for (int k = 0; k < count; k++) om[k] = out[k] + static_cast<size_t>(m0) * n_out[k];
+        if (mfma_takes(mm, n_in, gs, xm)) {
+            Workspace* ws;
+            {
+                std::lock_guard<std::mutex> lock(g_mu);
+                int dev;
+                if ((rc = current_device(&dev))) return rc;
+                ws = &g_dev[dev].ws[st];
+            }
+            if ((rc = gemv_mfma(count, w, scales, biases, om, n_out, false, xm, mm, n_in, st, *ws))) return rc;
+            if ((rc = multi_tails(count, w, scales, biases, om, n_out, xm, mm, n_in, gs, st))) return rc;
+            continue;
         }
-        ml.count = count;
-        if (ml.row_begin[count] == 0) return 0;
-        rc = try_fused_m(ml, x, m, n_in, gs, st);
-        if (rc < 0) return rc;
-        if (rc == 1) return multi_tails(count, w, scales, biases, out, n_out, x, m, n_in, gs, st);
-    }
-    // 3..8 rows on the matrix cores: x prepared once for every matrix
-    bool all_mf = m <= kMaxM, any = false;
-    for (int k = 0; k < count && all_mf; k++) {
-        all_mf = n_out[k] == 0 || mfma_takes(m, n_out[k], n_in, gs, x);
-        any = any || n_out[k] > 0;
-    }
-    if (all_mf && any) {
-        Workspace* ws;
-        {
-            std::lock_guard<std::mutex> lock(g_mu);
-            int dev;
-            if ((rc = current_device(&dev))) return rc;
-            ws = &g_dev[dev].ws[st];
+        if (mm < kMfMinRows) {
+            MatList ml{};
+            ml.row_begin[0] = 0;
+            for (int k = 0; k < kMaxMats; k++) {
+                const int kk = k < count ? k : count - 1;
+                ml.w[k] = w[kk]; ml.s[k] = scales[kk]; ml.b[k] = biases[kk]; ml.out[k] = om[kk];
+                ml.n_out[k] = k < count ? n_out[k] : 0;
+                ml.row_begin[k + 1] = ml.row_begin[k] + ml.n_out[k];
+            }
+            ml.count = count;
+            if (ml.row_begin[count] == 0) return 0;
+            rc = try_fused_m(ml, xm, mm, n_in, gs, st);
+            if (rc < 0) return rc;
+            if (rc == 1) {
+                if ((rc = multi_tails(count, w, scales, biases, om, n_out, xm, mm, n_in, gs, st))) return rc;
+                continue;
+            }
         }
-        if ((rc = mfma_prep(x, m, n_in, st, *ws))) return rc;
-        for (int k = 0; k < count; k++) {
-            if (n_out[k] == 0) continue;
-            const q4k::MfMats mt{{w[k], w[k]}, {scales[k], scales[k]}, {biases[k], biases[k]}};
-            if ((rc = mfma_main(mt, false, out[k], m, n_out[k], n_in, st, *ws)) < 0) return rc;
-        }
-        return multi_tails(count, w, scales, biases, out, n_out, x, m, n_in, gs, st);
+        for (int k = 0; k < count; k++)
+            if ((rc = q4_gemv_dev(w[k], scales[k], biases[k], xm, om[k], mm, n_out[k], n_in, gs, stream))) return rc;
     }
-    for (int k = 0; k < count; k++)
-        if ((rc = q4_gemv_dev(w[k], scales[k], biases[k], x, out[k], m, n_out[k], n_in, gs, stream)))
-            return rc;
     return 0;
 }
 
@@ -1505,8 +1513,8 @@ int q4_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate_s, const ui
     if ((reinterpret_cast<uintptr_t>(gate_w) | reinterpret_cast<uintptr_t>(up_w)) & 15)
         return fail(Q4_EARG, "w must be 16-byte aligned");
     hipStream_t st = static_cast<hipStream_t>(stream);
-    for (int m0 = 0; m0 < m; m0 += kMaxM) {
-        const int mm = m - m0 < kMaxM ? m - m0 : kMaxM;
+    for (int m0 = 0, mm; m0 < m; m0 += mm) {
+        mm = block_rows(m - m0, n_in, gs, x);
         const float* xm = x + static_cast<size_t>(m0) * n_in;
         float* hm = h + static_cast<size_t>(m0) * n_inter;
         MatList ml{};
@@ -1520,7 +1528,7 @@ int q4_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate_s, const ui
         ml.count = 2;
         ml.mrows = mm;
         int done = 0;
-        if (mm >= kMfMinRows) {
+        if (mfma_takes(mm, n_in, gs, xm)) {
             Workspace* ws;
             {
                 std::lock_guard<std::mutex> lock(g_mu);
@@ -1528,9 +1536,12 @@ int q4_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate_s, const ui
                 if ((rc = current_device(&dev))) return rc;
                 ws = &g_dev[dev].ws[st];
             }
-            const q4k::MfMats mt{{gate_w, up_w}, {gate_s, up_s}, {gate_b, up_b}};
-            done = gemv_mfma(mt, true, xm, hm, mm, n_inter, n_in, gs, st, *ws);
-            if (done < 0) return done;
+            const uint32_t* pw[2] = {gate_w, up_w};
+            const uint16_t *ps[2] = {gate_s, up_s}, *pb[2] = {gate_b, up_b};
+            float* ph[2] = {hm, hm};
+            const int pn[2] = {n_inter, n_inter};
+            if ((rc = gemv_mfma(2, pw, ps, pb, ph, pn, true, xm, mm, n_in, st, *ws))) return rc;
+            done = 1;
         }
         if (!done && mm <= 2 && stream_takes(xm, n_in, gs)) {
             done = mm == 1 ? launch_stream_gs<1, true>(ml, xm, n_in, gs, st)

@@ -88,9 +88,10 @@ const char *q4_last_error(void);
  * that share a device and overlap in time must be issued on one stream: the
  * per-stream x workspace is reused by the next call on that stream. */
 
-/* Batched GEMV over m rows (any m >= 1; rows are processed eight at a time).
+/* Batched GEMV over m rows (any m >= 1; rows are processed up to 16 at a
+ * time, eight where the matrix cores do not take the shape).
  * Same arithmetic as q4_gemv.  x is [m][n_in], out is [m][n_out].  Blocks of
- * 3..8 rows with gs 64 run their integer dots on the int8 matrix cores, with
+ * 3..16 rows with gs 64 run their integer dots on the int8 matrix cores, with
  * x quantised into the per-stream workspace first; the workspace grows on
  * first use, so run the largest call once on a stream before capturing it
  * in a graph. */
@@ -112,8 +113,8 @@ int q4_gemv_noalloc_dev(const uint32_t *w, const uint16_t *scales, const uint16_
                         void *stream);
 
 /* Up to four matrices that share the activations x (q/k/v, gate/up) in one
- * launch (1..2 rows; 3..8 rows: x quantised once, then one matrix-core launch
- * per matrix): out[k] is [m][n_out[k]] = W_k x, each row bit-identical to
+ * launch per block of rows (1..2 rows; 3..16 rows: x quantised once, then one
+ * matrix-core launch): out[k] is [m][n_out[k]] = W_k x, each row bit-identical to
  * q4_gemv.
  * w, scales, biases, out and n_out are host arrays of `count` device
  * pointers / sizes.  No counterpart in the reference, whose caller makes one

@@ -346,6 +346,52 @@ def test_matrix_core_group_count_bounds(lib):
             assert_bit_exact(got.cpu().numpy(), want[:m], f"K={k_in} N={n_out} m={m}")
 
 
+@pytest.mark.parametrize("k_in,shapes", [
+    (64, (40, 16, 1)),                 # one group; tiles of 16 rows full, partial and of one row
+    (1024, (17, 1, 4100)),             # a whole window; more tiles than CUs
+    (1088, (300,)),                    # 17 groups (odd): scales one at a time, a window of one group
+    (3584, (3584, 512, 512)),          # 3.5 windows, 288 tiles: some workgroups walk two
+    (18944, (96, 33)),                 # the ring wraps twice
+    (32768, (20,)),                    # the longest row the prep stages
+])
+def test_matrix_core_up_to_16_rows(lib, k_in, shapes):
+    """3..16 rows in one launch over every matrix of a grouped call, and the
+    rows past 16 in a block of their own: bit-exact vs the oracle, also with
+    scales and biases at a 2-byte offset (copied one group at a time), and
+    the same bits from the one-matrix and the no-allocation entry points."""
+    import torch
+    o = oracle.Oracle()
+    rows = 19
+    mats_np = [synth.qlinear(900 + k_in + i, n, k_in, 64) for i, n in enumerate(shapes)]
+    x = synth.activations(901 + k_in, rows, k_in)
+    tx = torch.from_numpy(x).cuda()
+    want = [o.gemv_rows(w, s, b, x, 64) for w, s, b in mats_np]
+
+    def odd(a):                        # the same values 2 bytes past a 4-byte boundary
+        t = torch.zeros(a.size + 1, dtype=torch.int16, device="cuda")
+        t[1:] = torch.from_numpy(a.view(np.int16).reshape(-1)).cuda()
+        return t[1:].reshape(a.shape)
+
+    mats = [tuple(torch.from_numpy(a).cuda() for a in (w, s.view(np.int16), b.view(np.int16))) for w, s, b in mats_np]
+    mats2 = [(t[0], odd(s), odd(b)) for t, (_, s, b) in zip(mats, mats_np)]
+    for m in (3, 8, 9, 16, 17, 19):
+        print(f"up to 16 rows K={k_in} N={shapes} m={m}", flush=True)
+        xm = tx[:m].contiguous()
+        for group in (mats, mats2):
+            outs = q4.gemv_multi_dev(group, xm)
+            torch.cuda.synchronize()
+            for got, w in zip(outs, want):
+                assert_bit_exact(got.cpu().numpy(), w[:m], f"multi K={k_in} N={w.shape[1]} m={m}")
+        got = q4.gemv_dev(*mats[0], xm)
+        noalloc = torch.full_like(got, float("nan"))
+        rc = lib.q4_gemv_noalloc_dev(*(t.data_ptr() for t in mats[0]), xm.data_ptr(), noalloc.data_ptr(), m, shapes[0],
+                                     k_in, 64, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, q4.last_error(lib)
+        torch.cuda.synchronize()
+        assert_bit_exact(got.cpu().numpy(), want[0][:m], f"dev K={k_in} m={m}")
+        assert_bit_exact(noalloc.cpu().numpy(), want[0][:m], f"noalloc K={k_in} m={m}")
+
+
 def test_matrix_core_uneven_prep_slices(lib):
     """The matrix-core x prep splits each row's groups over up to 8
     workgroups in slices of ceil(G / slices): K = 6208 (97 groups, slices of

@@ -114,3 +114,20 @@ def test_gate_up_silu_rows_odd_group_count():
         h = h.cpu().numpy()
         for r in range(m):
             assert np.array_equal(h[r].view(np.uint32), ones[r].view(np.uint32)), f"m={m} row {r}"
+
+
+@pytest.mark.parametrize("hidden,inter", [(832, 100), (1024, 2816), (3584, 18944), (4160, 40)])
+def test_gate_up_silu_9_to_16_rows(hidden, inter):
+    """The fused gate/up tiles for 9..16 rows (one launch) and 17 and 18
+    (a block of 16, then one or two rows): each row bit-identical to its
+    one-row launch; odd and even group counts, a partial tile, tiles past one
+    per CU."""
+    import torch
+    (_, gt), (_, ut) = mats(640, inter, hidden), mats(641, inter, hidden)
+    tx = tensors(synth.activations(642, 18, hidden))[0]
+    ones = torch.cat([q4.gate_up_silu_dev(gt, ut, tx[r:r + 1].contiguous()) for r in range(18)])
+    for m in (9, 13, 16, 17, 18):
+        print(f"gate/up rows hidden={hidden} inter={inter} m={m}", flush=True)
+        h = q4.gate_up_silu_dev(gt, ut, tx[:m].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(h.view(torch.int32), ones[:m].view(torch.int32)), m
