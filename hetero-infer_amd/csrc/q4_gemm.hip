@@ -5,21 +5,36 @@
 // Workgroup tile BM x 256 (BM 256 or 128), NW waves in 2 x NW/2, each wave
 // (BM/2) x (512/NW) -- TM x TN MFMA tiles of 32 x 32.  One K step is 64 = one
 // quantisation group, so each weight row has one scale/bias pair per step.
-// Every operand reaches LDS by global->LDS copies (buffer_load ... lds, 16 or
-// 2 bytes a lane), into a ring of three stages, each holding one K step:
-//   * A: the bf16 copy of x, BM rows x 128 bytes, 16-byte chunk c of row r
-//     at r * 128 + (c ^ (r & 7)) * 16 (the XOR spreads a fragment read by 32
-//     rows over the banks);
-//   * B: the packed weights as they are in memory, 256 rows x 8 words;
-//   * the 256 rows' scales, then their biases, a zero-extended word each.
+// Every operand reaches LDS by global->LDS copies (buffer_load ... lds, 16,
+// 4 or 2 bytes a lane):
+//   * A: the bf16 copy of x, BM rows x 128 bytes, a ring of three K steps;
+//     16-byte chunk c of row r at r * 128 + (c ^ (r / 2 & 7)) * 16 (the XOR
+//     spreads a fragment read by 32 rows over the 64 banks, which hold two
+//     rows);
+//   * B: the packed weights as they are in memory, 256 rows x 64 bytes: two
+//     K steps at a time, two slots; chunk c of row r at c ^ (r / 4 & 3);
+//   * the 256 rows' scales and biases, SG groups at a time, two slots: SG = 8
+//     (16 bytes a row) where the group count and the pointers allow it, 2 (4
+//     bytes), else 1 (2 bytes, zero-extended).
+// What bounds the copies is their number of requests, not their bytes: with
+// 32 bytes of weights and 2-byte scales and biases per row and step, those
+// 2 x 256 + 256 requests of a step (A has 256, of 128 bytes) kept the L2 busy
+// and the non-temporal policy fetched a row's 128-byte line once per step.
+// Measured at 512 rows (graph replays, before -> after these copies, the bank
+// swizzle, byte selects in the dequant and the next step's operands read under
+// the last slice): gate/up + down of a prompt chunk 308 -> 270 us, down 111 ->
+// 94, o 45 -> 37, 1000 rows 546 -> 446; one 256-row tile per CU over K = 18944
+// takes 2.02 us a step, 1064 TFLOP/s (MFMAs and barriers alone 1.52 us).
 // B is dequantised in registers right before the MFMA that consumes it:
-// one packed word (word 2 ks + lane/32 of the row) is exactly one lane's
-// 8-value B fragment of K slice ks, and its value is bf16(fma(q, scale,
-// bias)) -- what q4_dequant_bf16_dev writes.  Staging B 4-bit keeps its LDS
+// one packed word (word ks + 4 (lane/32) of the row: a lane's four words of
+// a step are one 16-byte read) is exactly one lane's 8-value B fragment of K
+// slice ks, and its value is bf16(fma(q, scale, bias)) -- what
+// q4_dequant_bf16_dev writes.  Staging B 4-bit keeps its LDS
 // traffic a quarter of bf16's, and a dequantised word feeds TM MFMAs.
 // Pipeline: step k + 2's copies are issued while step k is multiplied; at
-// the top of a step each wave waits for its own copies of the step (the
-// next step's stay in flight) and one barrier publishes everyone's.
+// the top of step k each wave waits for its own copies of step k + 1, made
+// a step before, and one barrier publishes everyone's, so that step k can
+// read and dequantise the first operands of step k + 1 under its last MFMAs.
 // Every copy goes through a buffer resource bounded to the tile's rows:
 // rows past M or N and steps past the workgroup's K range read 0 and cost
 // no access.  Split-K: blockIdx.z takes steps [z kt_split, (z+1) kt_split)
@@ -36,9 +51,13 @@ namespace q4k {
 typedef __bf16 gemm_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float gemm_f32x16 __attribute__((ext_vector_type(16)));
 
-// One stage of the LDS ring: A (BM rows x 128 bytes), B (256 rows x 32
-// bytes), then the 256 rows' scales and biases (a word each).
-__host__ __device__ constexpr int w4_stage_bytes(int bm) { return bm * 128 + 8192 + 2048; }
+// LDS: three steps of A (BM rows x 128 bytes), two slots of B (256 rows x 64
+// bytes), two slots of scales, then biases (256 rows of SG values, at least a
+// word, each).
+__host__ __device__ constexpr int w4_row_bytes(int sg) { return sg == 8 ? 16 : 4; }
+__host__ __device__ constexpr int w4_b0(int bm) { return 3 * bm * 128; }
+__host__ __device__ constexpr int w4_s0(int bm) { return w4_b0(bm) + 2 * 16384; }
+__host__ __device__ constexpr int w4_lds_bytes(int bm, int sg) { return w4_s0(bm) + 2 * 512 * w4_row_bytes(sg); }
 
 __device__ __forceinline__ uint32_t w4_pack_bf16(float a, float b) {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -47,64 +66,70 @@ __device__ __forceinline__ uint32_t w4_pack_bf16(float a, float b) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(p, bf16x2v));
 }
 
-// The 8 values of one packed word (element e in bits 4e..4e+3), each
-// bf16(fma(q_e, s, b)), in element order.
-__device__ __forceinline__ gemm_bf16x8 w4_dequant8(uint32_t w, float s, float b) {
-    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;   // even / odd elements, a byte each
-    float v[8];
-#pragma unroll
-    for (int n = 0; n < 4; n++) {
-        v[2 * n] = __builtin_fmaf(static_cast<float>((lo >> (8 * n)) & 0xFFu), s, b);
-        v[2 * n + 1] = __builtin_fmaf(static_cast<float>((hi >> (8 * n)) & 0xFFu), s, b);
-    }
-    const uint4 p = make_uint4(w4_pack_bf16(v[0], v[1]), w4_pack_bf16(v[2], v[3]), w4_pack_bf16(v[4], v[5]),
-                               w4_pack_bf16(v[6], v[7]));
-    return __builtin_bit_cast(gemm_bf16x8, p);
+// The nibbles of a packed word as bytes: even elements in lo, odd in hi.
+// (Opaque to the compiler, which would fold the masks into a bit-field
+// extract per value instead of the byte selects of v_cvt_f32_ubyte0..3.)
+__device__ __forceinline__ void w4_bytes(uint32_t w, uint32_t& lo, uint32_t& hi) {
+    lo = w & 0x0F0F0F0Fu;
+    hi = (w >> 4) & 0x0F0F0F0Fu;
+    asm("" : "+v"(lo), "+v"(hi));
 }
 
-// The operands of one tile (M block mt, N block nt): buffer resources over
-// its rows of x, W, scales and biases.
+// Elements 2q and 2q + 1 of a word's bytes, each bf16(fma(q_e, s, b)).
+__device__ __forceinline__ uint32_t w4_dequant2(uint32_t lo, uint32_t hi, int q, float s, float b) {
+    return w4_pack_bf16(__builtin_fmaf(static_cast<float>((lo >> (8 * q)) & 0xFFu), s, b),
+                        __builtin_fmaf(static_cast<float>((hi >> (8 * q)) & 0xFFu), s, b));
+}
+
+// The operands of one tile (M block mt, N block nt): its rows of x, W, scales
+// and biases and their bytes (the bounds of the copies' resources); paired
+// tiles: the up matrix's rows too.
 struct W4Tile {
-    __amdgpu_buffer_rsrc_t xr, wr, sr, br;
-    __amdgpu_buffer_rsrc_t wr2, sr2, br2;    // paired tiles: the up matrix's rows
+    const uint16_t* x;
+    const uint32_t *w, *w2;
+    const uint16_t *s, *b, *s2, *b2;
+    uint32_t xbytes, wbytes, gbytes;
     int m0, n0;
 };
 
-// The copies of one K step (kt) into a stage of the LDS ring (a plain device
-// function: the copy builtin in a lambda of the kernel keeps the compiler
-// from emitting the kernel's host stub).  NW waves share them: A in 1 KiB
-// copies of 8 rows, B in 8 copies of 32 rows, the 256 scales and biases in
-// 4 copies of 64 rows each.  `live` false (a step past the workgroup's K
-// range) reads zeros without an access.
-template <int BM, int NW, bool PAIR>
-__device__ __forceinline__ void w4_issue(char* st, const W4Tile& t, const uint32_t* a_src, const uint32_t* b_src,
-                                         uint32_t g_src, int kt, bool live, int wave) {
+// Copy i of the up to w4_copies that a wave makes for K step k of its range,
+// `first` its first step (a plain device function: the copy builtin in a
+// lambda of the kernel keeps the compiler from emitting the kernel's host
+// stub).  NW waves share the copies: A in 1 KiB copies of 8 rows, B in 16
+// copies of 16 rows (on even steps, for two), the 256 scales and biases in 4
+// copies of 64 rows each (every SG steps).  The step's offset is the scalar
+// one.
+template <int BM, int NW>
+constexpr int w4_copies() { return BM / (8 * NW) + 16 / NW + (NW == 4 ? 2 : 1); }
+
+template <int BM, int NW, int SG, bool PAIR>
+__device__ __forceinline__ void w4_issue(int i, char* lds, const W4Tile& t, const uint32_t* a_src, const uint32_t* b_src,
+                                         uint32_t g_src, int k, int slot, bool first, int wave) {
     typedef __attribute__((address_space(3))) void* lds_ptr;
-    constexpr int A_DMA = BM / (8 * NW), B_DMA = 8 / NW;
+    constexpr int A_DMA = BM / (8 * NW), B_DMA = 16 / NW;
     static_assert(!PAIR || NW == 4, "paired tiles: waves 0-1 copy the gate rows, 2-3 the up rows");
-    const uint32_t dead = __builtin_amdgcn_readfirstlane(live ? 0u : kOutOfRange);
-    const __amdgpu_buffer_rsrc_t xr = t.xr;
-    const __amdgpu_buffer_rsrc_t wr = PAIR && wave >= 2 ? t.wr2 : t.wr;     // wave-uniform choice
-    const __amdgpu_buffer_rsrc_t sr = PAIR && wave >= 2 ? t.sr2 : t.sr;
-    const __amdgpu_buffer_rsrc_t br = PAIR && wave >= 2 ? t.br2 : t.br;
-#pragma unroll
-    for (int i = 0; i < A_DMA; i++)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_ptr)(st + (wave * A_DMA + i) * 1024), 16,
-                                                 a_src[i] + static_cast<uint32_t>(kt) * 128u + dead, 0, 0, 0);
-#pragma unroll
-    for (int q = 0; q < B_DMA; q++)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(wr, (lds_ptr)(st + BM * 128 + (B_DMA * wave + q) * 1024), 16,
-                                                 b_src[q] + static_cast<uint32_t>(kt) * 32u + dead, 0, 0, 2);
-    const uint32_t go = g_src + static_cast<uint32_t>(kt) * 2u + dead;
-    if constexpr (NW == 4) {
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_ptr)(st + BM * 128 + 8192 + wave * 256), 2, go, 0, 0, 0);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(br, (lds_ptr)(st + BM * 128 + 9216 + wave * 256), 2, go, 0, 0, 0);
-    } else {                                                       // waves 0-3 scales, 4-7 biases
-        if (wave < 4)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(sr, (lds_ptr)(st + BM * 128 + 8192 + wave * 256), 2, go, 0, 0, 0);
-        else
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(br, (lds_ptr)(st + BM * 128 + 9216 + (wave - 4) * 256), 2, go, 0,
-                                                     0, 0);
+    if (i < A_DMA) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(buf_rsrc(t.x, t.xbytes),
+                                                 (lds_ptr)(lds + slot * (BM * 128) + (wave * A_DMA + i) * 1024), 16,
+                                                 a_src[i], k * 128, 0, 0);
+    } else if (i < A_DMA + B_DMA) {
+        const int q = i - A_DMA;
+        if (first || (k & 1) == 0)
+            // default cache policy: a row's 128-byte line holds four steps
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                buf_rsrc(PAIR && wave >= 2 ? t.w2 : t.w, t.wbytes),                    // wave-uniform
+                (lds_ptr)(lds + w4_b0(BM) + (k >> 1 & 1) * 16384 + (B_DMA * wave + q) * 1024), 16, b_src[q],
+                (k >> 1) * 64, 0, 0);
+    } else if (first || k % SG == 0) {
+        // NW = 4: a copy of each per wave; NW = 8: waves 0-3 scales, 4-7 biases
+        const bool bias = NW == 4 ? i > A_DMA + B_DMA : wave >= 4;
+        const uint16_t* p = PAIR && wave >= 2 ? (bias ? t.b2 : t.s2) : (bias ? t.b : t.s);
+        const __amdgpu_buffer_rsrc_t r = buf_rsrc(p, t.gbytes);
+        constexpr int RB = w4_row_bytes(SG);
+        const lds_ptr to = (lds_ptr)(lds + w4_s0(BM) + ((k / SG & 1) * 512 + (bias ? 256 : 0) + (wave & 3) * 64) * RB);
+        if constexpr (SG == 8) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 16, g_src, k / 8 * 16, 0, 0);
+        else if constexpr (SG == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 4, g_src, k / 2 * 4, 0, 0);
+        else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 2, g_src, k * 2, 0, 0);
     }
 }
 
@@ -117,13 +142,13 @@ __device__ __forceinline__ W4Tile w4_tile(const uint16_t* xb, const uint32_t* w,
     t.n0 = nt * BN;
     const int G = K >> 6, wpr = K >> 3;
     const int mrows = M - t.m0 < BM ? M - t.m0 : BM, nrows = N - t.n0 < BN ? N - t.n0 : BN;
-    t.xr = buf_rsrc(xb + static_cast<size_t>(t.m0) * K, static_cast<uint32_t>(mrows * K) * 2u);
-    t.wr = buf_rsrc(w + static_cast<size_t>(t.n0) * wpr, static_cast<uint32_t>(nrows * wpr) * 4u);
-    t.sr = buf_rsrc(sc + static_cast<size_t>(t.n0) * G, static_cast<uint32_t>(nrows * G) * 2u);
-    t.br = buf_rsrc(bi + static_cast<size_t>(t.n0) * G, static_cast<uint32_t>(nrows * G) * 2u);
-    t.wr2 = t.wr;
-    t.sr2 = t.sr;
-    t.br2 = t.br;
+    t.x = xb + static_cast<size_t>(t.m0) * K;
+    t.w = t.w2 = w + static_cast<size_t>(t.n0) * wpr;
+    t.s = t.s2 = sc + static_cast<size_t>(t.n0) * G;
+    t.b = t.b2 = bi + static_cast<size_t>(t.n0) * G;
+    t.xbytes = static_cast<uint32_t>(mrows * K) * 2u;
+    t.wbytes = static_cast<uint32_t>(nrows * wpr) * 4u;
+    t.gbytes = static_cast<uint32_t>(nrows * G) * 2u;
     return t;
 }
 
@@ -138,45 +163,46 @@ __device__ __forceinline__ W4Tile w4_tile_pair(const uint16_t* xb, const GemmMat
     const int G = K >> 6, wpr = K >> 3;
     const int mrows = M - t.m0 < BM ? M - t.m0 : BM, nrows = N - t.n0 < 128 ? N - t.n0 : 128;
     const size_t wo = static_cast<size_t>(t.n0) * wpr, go = static_cast<size_t>(t.n0) * G;
-    const uint32_t wb = static_cast<uint32_t>(nrows * wpr) * 4u, gb = static_cast<uint32_t>(nrows * G) * 2u;
-    t.xr = buf_rsrc(xb + static_cast<size_t>(t.m0) * K, static_cast<uint32_t>(mrows * K) * 2u);
-    t.wr = buf_rsrc(gm.w[0] + wo, wb);
-    t.sr = buf_rsrc(gm.s[0] + go, gb);
-    t.br = buf_rsrc(gm.b[0] + go, gb);
-    t.wr2 = buf_rsrc(gm.w[1] + wo, wb);
-    t.sr2 = buf_rsrc(gm.s[1] + go, gb);
-    t.br2 = buf_rsrc(gm.b[1] + go, gb);
+    t.x = xb + static_cast<size_t>(t.m0) * K;
+    t.w = gm.w[0] + wo;
+    t.s = gm.s[0] + go;
+    t.b = gm.b[0] + go;
+    t.w2 = gm.w[1] + wo;
+    t.s2 = gm.s[1] + go;
+    t.b2 = gm.b[1] + go;
+    t.xbytes = static_cast<uint32_t>(mrows * K) * 2u;
+    t.wbytes = static_cast<uint32_t>(nrows * wpr) * 4u;
+    t.gbytes = static_cast<uint32_t>(nrows * G) * 2u;
     return t;
 }
 
-// Per-lane source offsets of a step's copies (step kt adds kt * 128, kt * 32
-// and kt * 2 bytes).  A: copy i of wave w moves rows 8 (w A_DMA + i) .. + 8,
-// lane -> (row, 16-byte chunk c), reading chunk c ^ (row & 7) of the row:
-// the stage holds row r's chunk c at r * 128 + (c ^ (r & 7)) * 16.  B: copy
-// q moves rows 32 (B_DMA w + q) .. + 32, two lanes per row.  Scales /
-// biases: one row per lane, a zero-extended word each.
+// Per-lane source offsets of a step's copies.  A: copy i of wave w moves rows
+// 8 (w A_DMA + i) .. + 8, lane -> (row, 16-byte position p), reading chunk
+// p ^ (row / 2 & 7) of the row.  B: copy q moves rows 16 (B_DMA w + q) .. +
+// 16, four lanes per row, reading chunk p ^ (row / 4 & 3).  Scales / biases:
+// one row per lane.
 template <int BM, int NW>
 struct W4Src {
     uint32_t a[BM / (8 * NW)];
-    uint32_t b[8 / NW];
+    uint32_t b[16 / NW];
     uint32_t g;
 };
 
 template <int BM, int NW, bool PAIR>
 __device__ __forceinline__ void w4_src(W4Src<BM, NW>& src, int K, int wave, int lane) {
-    constexpr int A_DMA = BM / (8 * NW), B_DMA = 8 / NW;
+    constexpr int A_DMA = BM / (8 * NW), B_DMA = 16 / NW;
     const int G = K >> 6, wpr = K >> 3;
 #pragma unroll
     for (int i = 0; i < A_DMA; i++) {
         const int r = (wave * A_DMA + i) * 8 + (lane >> 3), c = lane & 7;
-        src.a[i] = static_cast<uint32_t>(r * K + (c ^ (r & 7)) * 8) * 2u;
+        src.a[i] = static_cast<uint32_t>(r * K + (c ^ (r >> 1 & 7)) * 8) * 2u;
     }
 #pragma unroll
     for (int q = 0; q < B_DMA; q++) {
-        const int r = ((B_DMA * wave + q) * 32 + (lane >> 1)) & (PAIR ? 127 : 255);   // row of its matrix
-        src.b[q] = static_cast<uint32_t>(r * wpr + (lane & 1) * 4) * 4u;
+        const int r = (B_DMA * wave + q) * 16 + (lane >> 2);             // stage row
+        src.b[q] = static_cast<uint32_t>((r & (PAIR ? 127 : 255)) * wpr) * 4u + ((lane & 3) ^ (r >> 2 & 3)) * 16u;
     }
-    src.g = static_cast<uint32_t>(((PAIR ? wave & 1 : NW == 4 ? wave : wave & 3) * 64 + lane) * G) * 2u;
+    src.g = static_cast<uint32_t>(((PAIR ? wave & 1 : wave & 3) * 64 + lane) * G) * 2u;
 }
 
 // How NW waves split a BM x 256 tile: WM x WN waves of RW rows x WC
@@ -205,95 +231,110 @@ __device__ __forceinline__ int w4_brow(int wn, int j, int lane) {
 // K steps [k0, k0 + nk) of one tile into acc (which it adds to): the copy
 // pipeline starts and drains inside, and on return every wave is past its
 // last LDS read and no copy is in flight, so the next segment may reuse the
-// ring.
-template <int BM, int NW, bool PAIR = false>
+// LDS.
+template <int BM, int NW, int SG, bool PAIR = false>
 __device__ __forceinline__ void w4_segment(W4Acc<BM, NW>& acc, char* lds, const W4Tile& t, const W4Src<BM, NW>& src,
                                            int k0, int nk, int wave, int lane) {
     using L = W4Layout<BM, NW>;
     constexpr int WN = L::WN, WC = L::WC, RW = L::RW, TM = L::TM, TN = L::TN;
-    constexpr int A_DMA = BM / (8 * NW), B_DMA = 8 / NW;
-    constexpr int PER_STEP = A_DMA + B_DMA + (NW == 4 ? 2 : 1);    // copies per wave and step
-    constexpr int STAGE = w4_stage_bytes(BM);
+    constexpr int COPIES = w4_copies<BM, NW>(), A_DMA = BM / (8 * NW);
+    constexpr int NM = TM * TN, NPC = TN * 4;                      // MFMAs, dequant pieces per slice
     const int hb = lane >> 5;
     const int wm = wave / WN, wn = wave % WN;
-    w4_issue<BM, NW, PAIR>(lds, t, src.a, src.b, src.g, k0, 0 < nk, wave);
-    w4_issue<BM, NW, PAIR>(lds + STAGE, t, src.a, src.b, src.g, k0 + 1, 1 < nk, wave);
-    for (int it = 0; it < nk; it++) {
-        // step it's copies are done (only step it + 1's may be in flight)
-        __builtin_amdgcn_s_waitcnt(0x0F70 | PER_STEP);
-        // a bare barrier: every wave's copies of step it are in LDS and every
-        // wave is past step it - 1, whose stage step it + 2 refills (a fence
-        // would also wait for the copies of step it + 1)
-        __builtin_amdgcn_s_barrier();
-        w4_issue<BM, NW, PAIR>(lds + ((it + 2) % 3) * STAGE, t, src.a, src.b, src.g, k0 + it + 2, it + 2 < nk, wave);
-        const char* st = lds + (it % 3) * STAGE;
-        const uint16_t* As = reinterpret_cast<const uint16_t*>(st);
-        const uint32_t* Bs = reinterpret_cast<const uint32_t*>(st + BM * 128);
-        const uint32_t* Ss = reinterpret_cast<const uint32_t*>(st + BM * 128 + 8192);
-        const uint32_t* Ts = reinterpret_cast<const uint32_t*>(st + BM * 128 + 9216);
-        float sf[TN], bf[TN];
+    auto issue = [&](int i, int it) {
+        w4_issue<BM, NW, SG, PAIR>(i, lds, t, src.a, src.b, src.g, k0 + it, it % 3, it == 0, wave);
+    };
+    // the operands of slice ks of step it: lane half hb takes 16-byte chunk
+    // (8 values of x) and packed word 4 hb + ks of the 64
+    auto a_frag = [&](int it, int ks, int i) {
+        const int row = wm * RW + i * 32 + (lane & 31);
+        const int c = (4 * hb + ks) ^ (row >> 1 & 7);
+        return *reinterpret_cast<const gemm_bf16x8*>(lds + it % 3 * (BM * 128) + row * 128 + c * 16);
+    };
+    uint32_t bw[TN][4];                                            // the step's packed words of the lane
+    float sf[TN], bf[TN];                                          // its scale and bias
+    auto b_step = [&](int it) {
+        const int k = k0 + it;
+        const char* bs = lds + w4_b0(BM) + (k >> 1 & 1) * 16384;
+        constexpr int RB = w4_row_bytes(SG);
+        const char* ss = lds + w4_s0(BM) + (k / SG & 1) * (512 * RB) + k % SG * 2;
 #pragma unroll
         for (int j = 0; j < TN; j++) {
             const int row = w4_brow<PAIR, WC>(wn, j, lane);
-            sf[j] = h2f(static_cast<uint16_t>(Ss[row]));
-            bf[j] = h2f(static_cast<uint16_t>(Ts[row]));
+            const uint4 w = *reinterpret_cast<const uint4*>(bs + row * 64 + (((k & 1) * 2 + hb) ^ (row >> 2 & 3)) * 16);
+            bw[j][0] = w.x; bw[j][1] = w.y; bw[j][2] = w.z; bw[j][3] = w.w;
+            sf[j] = h2f(*reinterpret_cast<const uint16_t*>(ss + row * RB));
+            bf[j] = h2f(*reinterpret_cast<const uint16_t*>(ss + 256 * RB + row * RB));
         }
-        // four K slices of 16; slice ks + 1's operands are read while slice
-        // ks multiplies, and its dequant is spread over the last of slice
-        // ks's MFMAs (fences pin the order), so the VALU work runs under the
-        // matrix core instead of before it
-        constexpr int NM = TM * TN, NPC = TN * 4;                  // MFMAs, dequant pieces per slice
-        auto a_frag = [&](int ks, int i) {
-            const int row = wm * RW + i * 32 + (lane & 31);
-            const int c = (2 * ks + hb) ^ (row & 7);
-            return *reinterpret_cast<const gemm_bf16x8*>(As + row * 64 + c * 8);
-        };
-        auto b_word = [&](int ks, int j) { return Bs[w4_brow<PAIR, WC>(wn, j, lane) * 8 + 2 * ks + hb]; };
-        gemm_bf16x8 av[2][TM], bv[2][TN];
-        uint32_t bw[TN], blo[TN], bhi[TN], pk[TN][4];
+    };
+    gemm_bf16x8 av[2][TM], bv[2][TN];
 #pragma unroll
-        for (int j = 0; j < TN; j++) bv[0][j] = w4_dequant8(b_word(0, j), sf[j], bf[j]);
+    for (int i = 0; i < COPIES; i++) issue(i, 0);
+    if (nk > 1) {
 #pragma unroll
-        for (int i = 0; i < TM; i++) av[0][i] = a_frag(0, i);
+        for (int i = 0; i < COPIES; i++) issue(i, 1);
+        // step 1 made at least A_DMA copies
+        __builtin_amdgcn_s_waitcnt(0x0F70 | A_DMA);
+    } else
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+    __builtin_amdgcn_s_barrier();                                  // step 0 is in LDS
+    b_step(0);
+#pragma unroll
+    for (int i = 0; i < TM; i++) av[0][i] = a_frag(0, 0, i);
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+        uint32_t lo, hi, pk[4];
+        w4_bytes(bw[j][0], lo, hi);
+#pragma unroll
+        for (int q = 0; q < 4; q++) pk[q] = w4_dequant2(lo, hi, q, sf[j], bf[j]);
+        bv[0][j] = __builtin_bit_cast(gemm_bf16x8, make_uint4(pk[0], pk[1], pk[2], pk[3]));
+    }
+    for (int it = 0; it < nk; it++) {
+        // step it + 1's copies, a step old, are done
+        __builtin_amdgcn_s_waitcnt(0x0F70);
+        // a bare barrier: every wave's copies of step it + 1 are in LDS and
+        // every wave is past step it - 1, whose slots step it + 2 refills (a
+        // fence would also wait for the LDS reads in flight)
+        __builtin_amdgcn_s_barrier();
+        const bool more = it + 2 < nk;
+        // four K slices of 16; the next slice's operands (after the last, the
+        // next step's first) are read while this one multiplies, and its
+        // dequant is spread over the last of this slice's MFMAs (fences pin
+        // the order), so the VALU work runs under the matrix core instead of
+        // before it; the copies of step it + 2 go out between the first
+        // slice's MFMAs.  (Past the last step the reads find old values,
+        // which nothing uses.)
 #pragma unroll
         for (int ks = 0; ks < 4; ks++) {
-            const int cu = ks & 1, nx = cu ^ 1;
-            if (ks < 3) {
+            const int cu = ks & 1, nx = cu ^ 1, kn = (ks + 1) & 3;
+            if (ks == 3) b_step(it + 1);
 #pragma unroll
-                for (int j = 0; j < TN; j++) bw[j] = b_word(ks + 1, j);
-#pragma unroll
-                for (int i = 0; i < TM; i++) av[nx][i] = a_frag(ks + 1, i);
-            }
+            for (int i = 0; i < TM; i++) av[nx][i] = a_frag(ks < 3 ? it : it + 1, kn, i);
             __builtin_amdgcn_sched_barrier(0);
+            uint32_t blo[TN], bhi[TN], pk[TN][4];
 #pragma unroll
             for (int m = 0; m < NM; m++) {
                 const int i = m / TN, j = m % TN;
                 acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[cu][i], bv[cu][j], acc[i][j], 0, 0, 0);
-                if (ks < 3) {
-                    constexpr int M0 = NPC < NM ? NM - NPC : 0, NR = NM - M0;   // pieces in the last NR MFMAs
+                if (ks == 0 && more) {
 #pragma unroll
-                    for (int pc = m < M0 ? 0 : (m - M0) * NPC / NR; pc < (m < M0 ? 0 : (m - M0 + 1) * NPC / NR); pc++) {
-                        const int jj = pc / 4, q = pc % 4;
-                        if (q == 0) {
-                            blo[jj] = bw[jj] & 0x0F0F0F0Fu;          // even / odd elements, a byte each
-                            bhi[jj] = (bw[jj] >> 4) & 0x0F0F0F0Fu;
-                        }
-                        pk[jj][q] = w4_pack_bf16(
-                            __builtin_fmaf(static_cast<float>((blo[jj] >> (8 * q)) & 0xFFu), sf[jj], bf[jj]),
-                            __builtin_fmaf(static_cast<float>((bhi[jj] >> (8 * q)) & 0xFFu), sf[jj], bf[jj]));
-                        if (q == 3)
-                            bv[nx][jj] = __builtin_bit_cast(gemm_bf16x8,
-                                                            make_uint4(pk[jj][0], pk[jj][1], pk[jj][2], pk[jj][3]));
-                    }
+                    for (int c = m * COPIES / NM; c < (m + 1) * COPIES / NM; c++) issue(c, it + 2);
+                }
+                constexpr int M0 = NPC < NM ? NM - NPC : 0, NR = NM - M0;   // pieces in the last NR MFMAs
+#pragma unroll
+                for (int pc = m < M0 ? 0 : (m - M0) * NPC / NR; pc < (m < M0 ? 0 : (m - M0 + 1) * NPC / NR); pc++) {
+                    const int jj = pc / 4, q = pc % 4;
+                    if (q == 0) w4_bytes(bw[jj][kn], blo[jj], bhi[jj]);
+                    pk[jj][q] = w4_dequant2(blo[jj], bhi[jj], q, sf[jj], bf[jj]);
+                    if (q == 3)
+                        bv[nx][jj] = __builtin_bit_cast(gemm_bf16x8,
+                                                        make_uint4(pk[jj][0], pk[jj][1], pk[jj][2], pk[jj][3]));
                 }
                 __builtin_amdgcn_sched_barrier(0);
             }
         }
     }
-    // the last copies issued (past the segment) read nothing; wait for them,
-    // and for every wave's last LDS reads
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
+    __syncthreads();                                               // every wave's last LDS reads are done
 }
 
 // C tile: lane l, register v holds row 8 (v / 4) + 4 (l / 32) + v % 4,
@@ -362,7 +403,7 @@ __device__ __forceinline__ int gm_mat(const GemmMats& gm, int nt) {
 // Data-parallel: workgroup (mt, nt, z) computes K steps [z kt_split,
 // (z+1) kt_split) of tile (mt, nt): into its matrix's output, or (part)
 // into part + z M ldp at the matrix's columns.
-template <int BM, int NW>
+template <int BM, int NW, int SG>
 __global__ __launch_bounds__(64 * NW) void gemm_w4_kernel(const uint16_t* __restrict__ xb, GemmMats gm,
                                                           float* __restrict__ part, int M, int K, int kt_split,
                                                           int ldp) {
@@ -380,7 +421,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4_kernel(const uint16_t* __rest
     w4_src<BM, NW, false>(src, K, wave, lane);
     W4Acc<BM, NW> acc;
     w4_zero<BM, NW>(acc);
-    w4_segment<BM, NW>(acc, lds, t, src, kt0, nk, wave, lane);
+    w4_segment<BM, NW, SG>(acc, lds, t, src, kt0, nk, wave, lane);
     if (part)
         w4_store<BM, NW>(acc, part + static_cast<size_t>(blockIdx.z) * M * ldp + gm.col0[k], t, M, N, ldp, 0, wave,
                          lane);
@@ -392,7 +433,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4_kernel(const uint16_t* __rest
 // step: h[r][c] = bf16(SiLU(x W_gate^T) * (x W_up^T)), rounded to nearest
 // even -- the fp32 products of two gemm_w4_kernel calls through silu_mul,
 // then the bf16 rounding the down projection applies to its x.
-template <int BM, int NW>
+template <int BM, int NW, int SG>
 __global__ __launch_bounds__(64 * NW) void gemm_w4_pair_kernel(const uint16_t* __restrict__ xb, GemmMats gm,
                                                                uint16_t* __restrict__ h, int M, int K) {
     static_assert(BM == 256 && NW == 4, "paired tiles: 4 waves of 256 x (32 gate + 32 up) columns");
@@ -408,7 +449,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4_pair_kernel(const uint16_t* _
     w4_src<BM, NW, true>(src, K, wave, lane);
     W4Acc<BM, NW> acc;
     w4_zero<BM, NW>(acc);
-    w4_segment<BM, NW, true>(acc, lds, t, src, 0, K >> 6, wave, lane);
+    w4_segment<BM, NW, SG, true>(acc, lds, t, src, 0, K >> 6, wave, lane);
     const int col = t.n0 + wave * 32 + (lane & 31);
     if (col >= N) return;
 #pragma unroll
@@ -500,7 +541,7 @@ __device__ __forceinline__ void w4_store_pair_rows(const W4Acc<BM, NW>& acc, uin
 
 // Segment [it, stop) of a stream-K range (stop at most its tile's end).
 // NTL: tiles per block row (the N blocks of gm, or of the paired columns).
-template <int BM, int NW, bool PAIR>
+template <int BM, int NW, int SG, bool PAIR>
 __device__ __forceinline__ void w4_sk_segment(char* lds, const uint16_t* xb, const GemmMats& gm, float* part,
                                               uint16_t* hout, unsigned* flags, unsigned* errors, unsigned epoch,
                                               int M, int K, int NTL, const SkGroup& gp, long it, long stop,
@@ -525,7 +566,7 @@ __device__ __forceinline__ void w4_sk_segment(char* lds, const uint16_t* xb, con
     const W4Tile t = PAIR ? w4_tile_pair<BM>(xb, gm, M, N, K, tile / NTL, nt)
                           : w4_tile<BM>(xb, gm.w[mk], gm.s[mk], gm.b[mk], M, N, K, tile / NTL, nt - gm.nb0[mk]);
     w4_zero<BM, NW>(acc);
-    w4_segment<BM, NW, PAIR>(acc, lds, t, src, k0, nk, wave, lane);
+    w4_segment<BM, NW, SG, PAIR>(acc, lds, t, src, k0, nk, wave, lane);
     if (stop < tile_start + G) {
         const __amdgpu_buffer_rsrc_t pr =
             buf_rsrc(part + static_cast<size_t>(gp.phys(wg)) * (kSlotBytes / 4), kSlotBytes);
@@ -613,7 +654,7 @@ __device__ __forceinline__ void w4_sk_segment(char* lds, const uint16_t* xb, con
     }
 }
 
-template <int BM, int NW, bool PAIR>
+template <int BM, int NW, int SG, bool PAIR>
 __global__ __launch_bounds__(64 * NW) void gemm_w4_sk_kernel(const uint16_t* __restrict__ xb, GemmMats gm,
                                                              float* __restrict__ part, unsigned* __restrict__ flags,
                                                              unsigned* __restrict__ ctl, int M, int K, int nx,
@@ -646,7 +687,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4_sk_kernel(const uint16_t* __r
         for (long seg_end = end; seg_end > begin;) {
             const long tile_start = (seg_end - 1) / G * G;
             const long seg_start = tile_start > begin ? tile_start : begin;
-            w4_sk_segment<BM, NW, PAIR>(lds, xb, gm, part, hout, flags, errors, epoch, M, K, NTL, gp, seg_start,
+            w4_sk_segment<BM, NW, SG, PAIR>(lds, xb, gm, part, hout, flags, errors, epoch, M, K, NTL, gp, seg_start,
                                         seg_end, src, tid, wave, lane);
             seg_end = seg_start;
         }
@@ -665,16 +706,21 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4_sk_kernel(const uint16_t* __r
     }
 }
 
-template <int BM, int NW>
-size_t w4_lds_bytes() {
-    return static_cast<size_t>(3) * w4_stage_bytes(BM);
+// SG of a launch: the groups of scales and biases that one copy takes, by the
+// group count and the alignment of every matrix's scales and biases.
+int w4_groups(const GemmMats& gm, int K) {
+    const int G = K >> 6;
+    uintptr_t al = 0;
+    for (int k = 0; k < gm.count; k++)
+        al |= reinterpret_cast<uintptr_t>(gm.s[k]) | reinterpret_cast<uintptr_t>(gm.b[k]);
+    return G % 8 == 0 && !(al & 15) ? 8 : G % 2 == 0 && !(al & 3) ? 2 : 1;
 }
 
-template <int BM, int NW>
+template <int BM, int NW, int SG>
 int launch_w4(const uint16_t* xb, const GemmMats& gm, float* part, int M, int K, int S, int kt_split, int ldp,
               hipStream_t st) {
-    auto kern = gemm_w4_kernel<BM, NW>;
-    const size_t lds = w4_lds_bytes<BM, NW>();
+    auto kern = gemm_w4_kernel<BM, NW, SG>;
+    constexpr size_t lds = w4_lds_bytes(BM, SG);
     static std::atomic<uint64_t> lds_raised{0};
     if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kern), lds, lds_raised)) return rc;
     hipLaunchKernelGGL(kern, dim3((M + BM - 1) / BM, gm.nb0[gm.count], S), dim3(64 * NW), lds, st, xb, gm, part, M, K,
@@ -684,12 +730,12 @@ int launch_w4(const uint16_t* xb, const GemmMats& gm, float* part, int M, int K,
     return 0;
 }
 
-template <int BM, int NW, bool PAIR>
+template <int BM, int NW, int SG, bool PAIR>
 int launch_w4_sk(const uint16_t* xb, const GemmMats& gm, float* part, unsigned* flags, unsigned* ctl, int M, int K,
                  int P, int nx, uint16_t* hout, hipStream_t st) {
-    auto kern = gemm_w4_sk_kernel<BM, NW, PAIR>;
-    const size_t lds = w4_lds_bytes<BM, NW>();
-    static_assert(256 * 256 * 4 / kSkParts <= 3 * w4_stage_bytes(BM), "a part of a slot fits the LDS ring");
+    auto kern = gemm_w4_sk_kernel<BM, NW, SG, PAIR>;
+    constexpr size_t lds = w4_lds_bytes(BM, SG);
+    static_assert(256 * 256 * 4 / kSkParts <= lds, "a part of a slot fits the LDS");
     static std::atomic<uint64_t> lds_raised{0};
     if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kern), lds, lds_raised)) return rc;
     hipLaunchKernelGGL(kern, dim3(P), dim3(64 * NW), lds, st, xb, gm, part, flags, ctl, M, K, nx, hout);
@@ -698,9 +744,10 @@ int launch_w4_sk(const uint16_t* xb, const GemmMats& gm, float* part, unsigned* 
     return 0;
 }
 
-int gemm_w4_pair(const uint16_t* xb, const GemmMats& gm, uint16_t* h, int M, int K, hipStream_t st) {
-    auto kern = gemm_w4_pair_kernel<256, 4>;
-    const size_t lds = w4_lds_bytes<256, 4>();
+template <int SG>
+int launch_w4_pair(const uint16_t* xb, const GemmMats& gm, uint16_t* h, int M, int K, hipStream_t st) {
+    auto kern = gemm_w4_pair_kernel<256, 4, SG>;
+    constexpr size_t lds = w4_lds_bytes(256, SG);
     static std::atomic<uint64_t> lds_raised{0};
     if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kern), lds, lds_raised)) return rc;
     hipLaunchKernelGGL(kern, dim3((M + 255) / 256, (gm.n_out[0] + 127) / 128), dim3(256), lds, st, xb, gm, h, M, K);
@@ -709,22 +756,43 @@ int gemm_w4_pair(const uint16_t* xb, const GemmMats& gm, uint16_t* h, int M, int
     return 0;
 }
 
+int gemm_w4_pair(const uint16_t* xb, const GemmMats& gm, uint16_t* h, int M, int K, hipStream_t st) {
+    const int sg = w4_groups(gm, K);
+    return sg == 8 ? launch_w4_pair<8>(xb, gm, h, M, K, st)
+                   : sg == 2 ? launch_w4_pair<2>(xb, gm, h, M, K, st) : launch_w4_pair<1>(xb, gm, h, M, K, st);
+}
+
 int gemm_w4(const uint16_t* xb, const GemmMats& gm, float* part, int M, int K, int bm, int S, int kt_split, int ldp,
             hipStream_t st) {
     // 256-row tiles: 4 waves of 256 x 64 (a dequantised weight word feeds 8
     // MFMAs); 128-row tiles: 8 waves of 64 x 64
-    return bm == 256 ? launch_w4<256, 4>(xb, gm, part, M, K, S, kt_split, ldp, st)
-                     : launch_w4<128, 8>(xb, gm, part, M, K, S, kt_split, ldp, st);
+    const int sg = w4_groups(gm, K);
+    if (bm == 256)
+        return sg == 8 ? launch_w4<256, 4, 8>(xb, gm, part, M, K, S, kt_split, ldp, st)
+                       : sg == 2 ? launch_w4<256, 4, 2>(xb, gm, part, M, K, S, kt_split, ldp, st)
+                                 : launch_w4<256, 4, 1>(xb, gm, part, M, K, S, kt_split, ldp, st);
+    return sg == 8 ? launch_w4<128, 8, 8>(xb, gm, part, M, K, S, kt_split, ldp, st)
+                   : sg == 2 ? launch_w4<128, 8, 2>(xb, gm, part, M, K, S, kt_split, ldp, st)
+                             : launch_w4<128, 8, 1>(xb, gm, part, M, K, S, kt_split, ldp, st);
+}
+
+template <bool PAIR>
+int sk_by_groups(const uint16_t* xb, const GemmMats& gm, float* part, unsigned* flags, unsigned* ctl, uint16_t* h, int M,
+                 int K, int P, int nx, hipStream_t st) {
+    const int sg = w4_groups(gm, K);
+    return sg == 8 ? launch_w4_sk<256, 4, 8, PAIR>(xb, gm, part, flags, ctl, M, K, P, nx, h, st)
+                   : sg == 2 ? launch_w4_sk<256, 4, 2, PAIR>(xb, gm, part, flags, ctl, M, K, P, nx, h, st)
+                             : launch_w4_sk<256, 4, 1, PAIR>(xb, gm, part, flags, ctl, M, K, P, nx, h, st);
 }
 
 int gemm_w4_sk(const uint16_t* xb, const GemmMats& gm, float* part, unsigned* flags, unsigned* ctl, int M, int K,
                int P, int nx, hipStream_t st) {
-    return launch_w4_sk<256, 4, false>(xb, gm, part, flags, ctl, M, K, P, nx, nullptr, st);
+    return sk_by_groups<false>(xb, gm, part, flags, ctl, nullptr, M, K, P, nx, st);
 }
 
 int gemm_w4_sk_pair(const uint16_t* xb, const GemmMats& gm, float* part, unsigned* flags, unsigned* ctl, uint16_t* h,
                     int M, int K, int P, int nx, hipStream_t st) {
-    return launch_w4_sk<256, 4, true>(xb, gm, part, flags, ctl, M, K, P, nx, h, st);
+    return sk_by_groups<true>(xb, gm, part, flags, ctl, h, M, K, P, nx, st);
 }
 
 }  // namespace q4k

@@ -202,3 +202,34 @@ def test_gemm_bf16_multi(monkeypatch, m, n_in, n_outs, plans):
             assert oracle.normwise_rel(g, exact) < EXACT_OPERAND_TOL, (plan, n)
             assert torch.equal(got, again), (plan, n)
     _plan(monkeypatch, None)
+
+
+# Group counts that take each way of copying scales and biases (8 groups a
+# copy: G a multiple of 8; 2: even; 1: odd, or pointers off a 4-byte
+# boundary) and each start of a K range (even, odd, across an 8-group
+# boundary) in splits, stream-K ranges and whole tiles; the copies' two-step
+# and one-step tails; one row and a ragged last tile.
+@pytest.mark.parametrize("groups,plans", [(1, (None,)), (2, (None, "dp:256:2")), (3, ("dp:128:3", "dp:256:1")),
+                                          (7, ("dp:128:2", "sk:5")), (8, ("dp:256:2", "dp:128:3", "sk:5")),
+                                          (14, ("dp:256:3", "dp:128:2", "sk:9")), (17, ("dp:128:4", "sk:7")),
+                                          (24, ("dp:256:5", "dp:128:1", "sk:11"))])
+def test_gemm_bf16_group_copies(monkeypatch, groups, plans):
+    import torch
+    n_out, n_in = 300, 64 * groups
+    for m in (1, 70, 257):
+        (tw, ts, tb, tx), exact = _operands(900 + groups + m, m, n_out, n_in)
+        odd = []
+        for t in (ts, tb):                                     # the same values 2 bytes past a 4-byte boundary
+            o = torch.zeros(t.numel() + 1, dtype=t.dtype, device=t.device)
+            o[1:] = t.reshape(-1)
+            odd.append(o[1:].reshape(t.shape))
+        for plan in plans:
+            print(f"group copies G={groups} m={m} plan={plan}", flush=True)
+            _plan(monkeypatch, plan)
+            got = q4.gemm_bf16_dev(tw, ts, tb, tx)
+            one = q4.gemm_bf16_dev(tw, odd[0], odd[1], tx)
+            torch.cuda.synchronize()
+            assert oracle.normwise_rel(got.cpu().numpy(), exact) < EXACT_OPERAND_TOL
+            assert torch.equal(got, one), "the copies' width changed the result"
+    _plan(monkeypatch, None)
+    assert q4.prefill_errors() == 0
