@@ -368,7 +368,7 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, int part, int max
     auto weight = [&](float mc) { return mc != -__builtin_inff() ? expf(__fsub_rn(mc, M)) : 0.0f; };
     const float w0 = weight(m0), w1 = weight(m1);    // lane c: the weights of parts c and c + 64
     const float lloc = n_act > 64 ? __builtin_fmaf(ml1.y, w1, __fmul_rn(ml0.y, w0)) : __fmul_rn(ml0.y, w0);
-    auto wt = [&](int c) {                           // c a constant after unrolling
+    auto wt = [&](int c) {                           // c uniform
         return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c < 64 ? w0 : w1), c & 63));
     };
     float s0 = 0.0f, s1 = 0.0f;
@@ -378,17 +378,15 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, int part, int max
         s0 = __builtin_fmaf(ob[c].x, wc, s0);
         s1 = __builtin_fmaf(ob[c].y, wc, s1);
     }
+#pragma unroll 1
+    for (int base = kMergeBatch; base < n_act; base += kMergeMore) {
 #pragma unroll
-    for (int base = kMergeBatch; base < kMaxParts; base += kMergeMore) {
-        if (base < n_act) {
+        for (int t = 0; t < kMergeMore; t++) ob[t] = ld_o(base + t);
 #pragma unroll
-            for (int t = 0; t < kMergeMore && base + t < kMaxParts; t++) ob[t] = ld_o(base + t);
-#pragma unroll
-            for (int t = 0; t < kMergeMore && base + t < kMaxParts; t++) {
-                const float wc = wt(base + t);
-                s0 = __builtin_fmaf(ob[t].x, wc, s0);
-                s1 = __builtin_fmaf(ob[t].y, wc, s1);
-            }
+        for (int t = 0; t < kMergeMore; t++) {
+            const float wc = base + t < n_act ? wt(base + t) : 0.0f;
+            s0 = __builtin_fmaf(ob[t].x, wc, s0);
+            s1 = __builtin_fmaf(ob[t].y, wc, s1);
         }
     }
     const float L = wave_sum(lloc);

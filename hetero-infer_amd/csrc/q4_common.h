@@ -273,17 +273,17 @@ struct GemmMats {
     int count;
 };
 
-// The prefill GEMM (q4_gemm.hip), data-parallel: tiles of height bm (256 or
-// 128) over every block of gm, S splits of kt_split K steps.  part null:
+// The prefill GEMM (q4_gemm.hip), data-parallel: tiles of height bm (256, 192,
+// 128 or 64) over every block of gm, S splits of kt_split K steps.  part null:
 // each matrix's output directly; else split z into part + z M ldp at the
 // matrix's columns.
 int gemm_w4(const uint16_t* xb, const GemmMats& gm, float* part, int M, int K, int bm, int S, int kt_split, int ldp,
             hipStream_t st);
 
-// Paired gate/up form (q4_gemm.hip): matrices 0 and 1 of gm, both n_out[0]
-// rows, every K step in one workgroup, h[M][n_out[0]] = bf16(SiLU(x Wg^T) *
-// (x Wu^T)).
-int gemm_w4_pair(const uint16_t* xb, const GemmMats& gm, uint16_t* h, int M, int K, hipStream_t st);
+// Paired gate/up form (q4_gemm.hip), tiles of height bm: matrices 0 and 1 of
+// gm, both n_out[0] rows, every K step in one workgroup, h[M][n_out[0]] =
+// bf16(SiLU(x Wg^T) * (x Wu^T)).
+int gemm_w4_pair(const uint16_t* xb, const GemmMats& gm, uint16_t* h, int M, int K, int bm, hipStream_t st);
 
 // Stream-K form of the prefill GEMM: P workgroups in nx XCD groups (256 x
 // 256 tiles; P a multiple of nx, and P / nx at least a group's tile count,

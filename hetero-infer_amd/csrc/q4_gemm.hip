@@ -2,8 +2,8 @@
 // the MFMA: out[M][N] = bf16(x)[M][K] . bf16(dequant W)[N][K]^T, fp32
 // accumulation on v_mfma_f32_32x32x16_bf16.
 //
-// Workgroup tile BM x 256 (BM 256 or 128), NW waves in 2 x NW/2, each wave
-// (BM/2) x (512/NW) -- TM x TN MFMA tiles of 32 x 32.  One K step is 64 = one
+// Workgroup tile BM x 256 (BM 256, 192, 128 or 64), NW waves side by side, each
+// BM x 256/NW -- TM x TN MFMA tiles of 32 x 32.  One K step is 64 = one
 // quantisation group, so each weight row has one scale/bias pair per step.
 // Every operand reaches LDS by global->LDS copies (buffer_load ... lds, 16,
 // 4 or 2 bytes a lane):
@@ -22,9 +22,11 @@
 // and the non-temporal policy fetched a row's 128-byte line once per step.
 // Measured at 512 rows (graph replays, before -> after these copies, the bank
 // swizzle, byte selects in the dequant and the next step's operands read under
-// the last slice): gate/up + down of a prompt chunk 308 -> 270 us, down 111 ->
-// 94, o 45 -> 37, 1000 rows 546 -> 446; one 256-row tile per CU over K = 18944
-// takes 2.02 us a step, 1064 TFLOP/s (MFMAs and barriers alone 1.52 us).
+// the last slice, in 4 waves of 64 columns): gate/up + down of a prompt chunk
+// 308 -> 270 us, down 111 -> 94, o 45 -> 37, 1000 rows 546 -> 446; one 256-row
+// tile per CU over K = 18944 took 2.02 us a step, 1064 TFLOP/s (MFMAs and
+// barriers alone 1.52: the clock drops as the CUs fill).  8 waves of 32
+// columns: a lone tile's step 1.50 -> 1.31 us at 256 rows, 1.25 -> 1.09 at 192.
 // B is dequantised in registers right before the MFMA that consumes it:
 // one packed word (word ks + 4 (lane/32) of the row: a lane's four words of
 // a step are one 16-byte read) is exactly one lane's 8-value B fragment of K
@@ -41,9 +43,9 @@
 // and writes its partial sums to out + z M ldo.
 // Paired tiles (gate/up of the MLP): the tile's 256 weight rows are rows
 // [n0, n0 + 128) of the gate matrix, then the same rows of the up matrix,
-// and wave w's 64 columns are gate rows n0 + 32 w .. and the same up rows,
-// so one lane holds gate and up of every output it writes: the epilogue
-// stores bf16(SiLU(gate) * up), the down projection's bf16 operand.
+// and wave w's 32 columns are gate rows n0 + 16 w .. + 16 and the same up
+// rows: the epilogue brings a column's two sums into one lane and stores
+// bf16(SiLU(gate) * up), the down projection's bf16 operand.
 #include "q4_common.h"
 
 namespace q4k {
@@ -81,13 +83,14 @@ __device__ __forceinline__ uint32_t w4_dequant2(uint32_t lo, uint32_t hi, int q,
                         __builtin_fmaf(static_cast<float>((hi >> (8 * q)) & 0xFFu), s, b));
 }
 
-// The operands of one tile (M block mt, N block nt): its rows of x, W, scales
-// and biases and their bytes (the bounds of the copies' resources); paired
-// tiles: the up matrix's rows too.
+// What a wave copies of one tile (M block m0, N block n0): rows of x, of W and
+// of the scales or the biases, and their bytes (the bounds of the copies'
+// resources).  Paired tiles: waves 0..3 copy the gate rows of W, 4..7 the up
+// rows.
 struct W4Tile {
     const uint16_t* x;
-    const uint32_t *w, *w2;
-    const uint16_t *s, *b, *s2, *b2;
+    const uint32_t* w;
+    const uint16_t* g;
     uint32_t xbytes, wbytes, gbytes;
     int m0, n0;
 };
@@ -96,18 +99,17 @@ struct W4Tile {
 // `first` its first step (a plain device function: the copy builtin in a
 // lambda of the kernel keeps the compiler from emitting the kernel's host
 // stub).  NW waves share the copies: A in 1 KiB copies of 8 rows, B in 16
-// copies of 16 rows (on even steps, for two), the 256 scales and biases in 4
-// copies of 64 rows each (every SG steps).  The step's offset is the scalar
+// copies of 16 rows (on even steps, for two), 64 scales (waves 0..3) or biases
+// (4..7) each (every SG steps).  The step's offset is the scalar
 // one.
 template <int BM, int NW>
-constexpr int w4_copies() { return BM / (8 * NW) + 16 / NW + (NW == 4 ? 2 : 1); }
+constexpr int w4_copies() { return BM / (8 * NW) + 16 / NW + 1; }
 
 template <int BM, int NW, int SG, bool PAIR>
 __device__ __forceinline__ void w4_issue(int i, char* lds, const W4Tile& t, const uint32_t* a_src, const uint32_t* b_src,
                                          uint32_t g_src, int k, int slot, bool first, int wave) {
     typedef __attribute__((address_space(3))) void* lds_ptr;
     constexpr int A_DMA = BM / (8 * NW), B_DMA = 16 / NW;
-    static_assert(!PAIR || NW == 4, "paired tiles: waves 0-1 copy the gate rows, 2-3 the up rows");
     if (i < A_DMA) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(buf_rsrc(t.x, t.xbytes),
                                                  (lds_ptr)(lds + slot * (BM * 128) + (wave * A_DMA + i) * 1024), 16,
@@ -117,16 +119,13 @@ __device__ __forceinline__ void w4_issue(int i, char* lds, const W4Tile& t, cons
         if (first || (k & 1) == 0)
             // default cache policy: a row's 128-byte line holds four steps
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                buf_rsrc(PAIR && wave >= 2 ? t.w2 : t.w, t.wbytes),                    // wave-uniform
+                buf_rsrc(t.w, t.wbytes),
                 (lds_ptr)(lds + w4_b0(BM) + (k >> 1 & 1) * 16384 + (B_DMA * wave + q) * 1024), 16, b_src[q],
                 (k >> 1) * 64, 0, 0);
     } else if (first || k % SG == 0) {
-        // NW = 4: a copy of each per wave; NW = 8: waves 0-3 scales, 4-7 biases
-        const bool bias = NW == 4 ? i > A_DMA + B_DMA : wave >= 4;
-        const uint16_t* p = PAIR && wave >= 2 ? (bias ? t.b2 : t.s2) : (bias ? t.b : t.s);
-        const __amdgpu_buffer_rsrc_t r = buf_rsrc(p, t.gbytes);
+        const __amdgpu_buffer_rsrc_t r = buf_rsrc(t.g, t.gbytes);
         constexpr int RB = w4_row_bytes(SG);
-        const lds_ptr to = (lds_ptr)(lds + w4_s0(BM) + ((k / SG & 1) * 512 + (bias ? 256 : 0) + (wave & 3) * 64) * RB);
+        const lds_ptr to = (lds_ptr)(lds + w4_s0(BM) + ((k / SG & 1) * 512 + wave * 64) * RB);
         if constexpr (SG == 8) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 16, g_src, k / 8 * 16, 0, 0);
         else if constexpr (SG == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 4, g_src, k / 2 * 4, 0, 0);
         else __builtin_amdgcn_raw_ptr_buffer_load_lds(r, to, 2, g_src, k * 2, 0, 0);
@@ -135,7 +134,7 @@ __device__ __forceinline__ void w4_issue(int i, char* lds, const W4Tile& t, cons
 
 template <int BM>
 __device__ __forceinline__ W4Tile w4_tile(const uint16_t* xb, const uint32_t* w, const uint16_t* sc, const uint16_t* bi,
-                                          int M, int N, int K, int mt, int nt) {
+                                          int M, int N, int K, int mt, int nt, int wave) {
     constexpr int BN = 256;
     W4Tile t;
     t.m0 = mt * BM;
@@ -143,9 +142,8 @@ __device__ __forceinline__ W4Tile w4_tile(const uint16_t* xb, const uint32_t* w,
     const int G = K >> 6, wpr = K >> 3;
     const int mrows = M - t.m0 < BM ? M - t.m0 : BM, nrows = N - t.n0 < BN ? N - t.n0 : BN;
     t.x = xb + static_cast<size_t>(t.m0) * K;
-    t.w = t.w2 = w + static_cast<size_t>(t.n0) * wpr;
-    t.s = t.s2 = sc + static_cast<size_t>(t.n0) * G;
-    t.b = t.b2 = bi + static_cast<size_t>(t.n0) * G;
+    t.w = w + static_cast<size_t>(t.n0) * wpr;
+    t.g = (wave < 4 ? sc : bi) + static_cast<size_t>(t.n0) * G;
     t.xbytes = static_cast<uint32_t>(mrows * K) * 2u;
     t.wbytes = static_cast<uint32_t>(nrows * wpr) * 4u;
     t.gbytes = static_cast<uint32_t>(nrows * G) * 2u;
@@ -156,20 +154,16 @@ __device__ __forceinline__ W4Tile w4_tile(const uint16_t* xb, const uint32_t* w,
 // matrix 0 (gate) and matrix 1 (up) of gm.
 template <int BM>
 __device__ __forceinline__ W4Tile w4_tile_pair(const uint16_t* xb, const GemmMats& gm, int M, int N, int K, int mt,
-                                               int nt) {
+                                               int nt, int wave) {
     W4Tile t;
     t.m0 = mt * BM;
     t.n0 = nt * 128;
     const int G = K >> 6, wpr = K >> 3;
     const int mrows = M - t.m0 < BM ? M - t.m0 : BM, nrows = N - t.n0 < 128 ? N - t.n0 : 128;
-    const size_t wo = static_cast<size_t>(t.n0) * wpr, go = static_cast<size_t>(t.n0) * G;
+    const int up = wave & 2 ? 1 : 0;                               // rows 64 (wave & 3) .. of the 256 scales or biases
     t.x = xb + static_cast<size_t>(t.m0) * K;
-    t.w = gm.w[0] + wo;
-    t.s = gm.s[0] + go;
-    t.b = gm.b[0] + go;
-    t.w2 = gm.w[1] + wo;
-    t.s2 = gm.s[1] + go;
-    t.b2 = gm.b[1] + go;
+    t.w = (wave < 4 ? gm.w[0] : gm.w[1]) + static_cast<size_t>(t.n0) * wpr;
+    t.g = (wave < 4 ? (up ? gm.s[1] : gm.s[0]) : (up ? gm.b[1] : gm.b[0])) + static_cast<size_t>(t.n0) * G;
     t.xbytes = static_cast<uint32_t>(mrows * K) * 2u;
     t.wbytes = static_cast<uint32_t>(nrows * wpr) * 4u;
     t.gbytes = static_cast<uint32_t>(nrows * G) * 2u;
@@ -205,27 +199,27 @@ __device__ __forceinline__ void w4_src(W4Src<BM, NW>& src, int K, int wave, int 
     src.g = static_cast<uint32_t>(((PAIR ? wave & 1 : wave & 3) * 64 + lane) * G) * 2u;
 }
 
-// How NW waves split a BM x 256 tile: WM x WN waves of RW rows x WC
-// columns, TM x TN MFMA tiles of 32 x 32 each.  256-row tiles: 1 x 4 waves
-// of 256 x 64 -- each weight word is dequantised once and feeds 8 MFMAs
-// (a 2 x 2 split dequantises every word twice and measured 12% slower per
-// K step); 128-row tiles: 2 x 4 waves of 64 x 64.
+// How NW waves split a BM x 256 tile: side by side, each the tile's BM rows
+// x 256 / NW columns, TM x TN MFMA tiles of 32 x 32, so that every weight
+// word is dequantised once and feeds TM MFMAs (128 rows took 1.10 us a step in
+// 2 x 4 waves of 64 x 64, 0.88 side by side).  Two waves per SIMD, so that one
+// dequantises while the other multiplies.
 template <int BM, int NW>
 struct W4Layout {
-    static constexpr int WN = BM == 256 ? NW : NW / 2, WM = NW / WN;
-    static constexpr int RW = BM / WM, WC = 256 / WN;
+    static constexpr int RW = BM, WC = 256 / NW;
     static constexpr int TM = RW / 32, TN = WC / 32;
 };
 
 template <int BM, int NW>
 using W4Acc = gemm_f32x16[W4Layout<BM, NW>::TM][W4Layout<BM, NW>::TN];
 
-// The stage row (of 256) of weight column block j of wave column wn: WC
-// consecutive rows per wave; paired tiles: gate rows wn 32 .. (j = 0) and
-// the same up rows, 128 further (j = 1).
+// The stage row (of 256) of a lane's column in block j of its wave: WC
+// consecutive rows per wave; paired tiles (WC 32): lanes 0..15 gate rows 16
+// wave .., lanes 16..31 the same up rows, 128 further.
 template <bool PAIR, int WC>
-__device__ __forceinline__ int w4_brow(int wn, int j, int lane) {
-    return PAIR ? j * 128 + wn * 32 + (lane & 31) : wn * WC + j * 32 + (lane & 31);
+__device__ __forceinline__ int w4_brow(int wave, int j, int lane) {
+    static_assert(!PAIR || WC == 32, "paired tiles: 16 gate and 16 up rows a wave");
+    return PAIR ? (lane & 16) * 8 + wave * 16 + (lane & 15) : wave * WC + j * 32 + (lane & 31);
 }
 
 // K steps [k0, k0 + nk) of one tile into acc (which it adds to): the copy
@@ -236,18 +230,17 @@ template <int BM, int NW, int SG, bool PAIR = false>
 __device__ __forceinline__ void w4_segment(W4Acc<BM, NW>& acc, char* lds, const W4Tile& t, const W4Src<BM, NW>& src,
                                            int k0, int nk, int wave, int lane) {
     using L = W4Layout<BM, NW>;
-    constexpr int WN = L::WN, WC = L::WC, RW = L::RW, TM = L::TM, TN = L::TN;
+    constexpr int WC = L::WC, TM = L::TM, TN = L::TN;
     constexpr int COPIES = w4_copies<BM, NW>(), A_DMA = BM / (8 * NW);
     constexpr int NM = TM * TN, NPC = TN * 4;                      // MFMAs, dequant pieces per slice
     const int hb = lane >> 5;
-    const int wm = wave / WN, wn = wave % WN;
     auto issue = [&](int i, int it) {
         w4_issue<BM, NW, SG, PAIR>(i, lds, t, src.a, src.b, src.g, k0 + it, it % 3, it == 0, wave);
     };
     // the operands of slice ks of step it: lane half hb takes 16-byte chunk
     // (8 values of x) and packed word 4 hb + ks of the 64
     auto a_frag = [&](int it, int ks, int i) {
-        const int row = wm * RW + i * 32 + (lane & 31);
+        const int row = i * 32 + (lane & 31);
         const int c = (4 * hb + ks) ^ (row >> 1 & 7);
         return *reinterpret_cast<const gemm_bf16x8*>(lds + it % 3 * (BM * 128) + row * 128 + c * 16);
     };
@@ -260,7 +253,7 @@ __device__ __forceinline__ void w4_segment(W4Acc<BM, NW>& acc, char* lds, const 
         const char* ss = lds + w4_s0(BM) + (k / SG & 1) * (512 * RB) + k % SG * 2;
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-            const int row = w4_brow<PAIR, WC>(wn, j, lane);
+            const int row = w4_brow<PAIR, WC>(wave, j, lane);
             const uint4 w = *reinterpret_cast<const uint4*>(bs + row * 64 + (((k & 1) * 2 + hb) ^ (row >> 2 & 3)) * 16);
             bw[j][0] = w.x; bw[j][1] = w.y; bw[j][2] = w.z; bw[j][3] = w.w;
             sf[j] = h2f(*reinterpret_cast<const uint16_t*>(ss + row * RB));
@@ -344,16 +337,16 @@ template <int BM, int NW>
 __device__ __forceinline__ void w4_store(const W4Acc<BM, NW>& acc, float* o, const W4Tile& t, int M, int N, int ldo,
                                          int c0, int wave, int lane) {
     using L = W4Layout<BM, NW>;
-    constexpr int WN = L::WN, WC = L::WC, RW = L::RW, TM = L::TM, TN = L::TN;
-    const int hb = lane >> 5, wm = wave / WN, wn = wave % WN;
+    constexpr int WC = L::WC, TM = L::TM, TN = L::TN;
+    const int hb = lane >> 5;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
         for (int j = 0; j < TN; j++)
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                const int row = t.m0 + wm * RW + i * 32 + 8 * (v >> 2) + 4 * hb + (v & 3);
-                const int col = t.n0 + wn * WC + j * 32 + (lane & 31);
+                const int row = t.m0 + i * 32 + 8 * (v >> 2) + 4 * hb + (v & 3);
+                const int col = t.n0 + wave * WC + j * 32 + (lane & 31);
                 if (row < M && col < N) o[static_cast<size_t>(row) * ldo + (col - c0)] = acc[i][j][v];
             }
 }
@@ -364,8 +357,8 @@ template <int BM, int NW, int NP>
 __device__ __forceinline__ void w4_store_rows(const W4Acc<BM, NW>& acc, float* o, const W4Tile& t, int M, int N, int h,
                                               bool poison, int wave, int lane) {
     using L = W4Layout<BM, NW>;
-    constexpr int WN = L::WN, WC = L::WC, RW = L::RW, TM = L::TM, TN = L::TN;
-    const int hb = lane >> 5, wm = wave / WN, wn = wave % WN;
+    constexpr int WC = L::WC, TM = L::TM, TN = L::TN;
+    const int hb = lane >> 5;
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
@@ -373,8 +366,8 @@ __device__ __forceinline__ void w4_store_rows(const W4Acc<BM, NW>& acc, float* o
             if ((i * TN + j) / (TM * TN / NP) != h) continue;
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                const int row = t.m0 + wm * RW + i * 32 + 8 * (v >> 2) + 4 * hb + (v & 3);
-                const int col = t.n0 + wn * WC + j * 32 + (lane & 31);
+                const int row = t.m0 + i * 32 + 8 * (v >> 2) + 4 * hb + (v & 3);
+                const int col = t.n0 + wave * WC + j * 32 + (lane & 31);
                 if (row < M && col < N)
                     o[static_cast<size_t>(row) * N + col] = poison ? __builtin_nanf("") : acc[i][j][v];
             }
@@ -416,7 +409,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4_kernel(const uint16_t* __rest
     const int nk = G - kt0 < kt_split ? G - kt0 : kt_split;
     const int k = gm_mat(gm, blockIdx.y);
     const int N = gm.n_out[k];
-    const W4Tile t = w4_tile<BM>(xb, gm.w[k], gm.s[k], gm.b[k], M, N, K, blockIdx.x, blockIdx.y - gm.nb0[k]);
+    const W4Tile t = w4_tile<BM>(xb, gm.w[k], gm.s[k], gm.b[k], M, N, K, blockIdx.x, blockIdx.y - gm.nb0[k],
+                                  wave);
     W4Src<BM, NW> src;
     w4_src<BM, NW, false>(src, K, wave, lane);
     W4Acc<BM, NW> acc;
@@ -429,6 +423,25 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4_kernel(const uint16_t* __rest
         w4_store<BM, NW>(acc, gm.out[k], t, M, N, N, 0, wave, lane);
 }
 
+// Row block i of a paired tile's outputs, h = bf16(SiLU(gate) * up), NaN if
+// `poison`.  Lanes 0..15 of a half hold gate and lanes 16..31 up of the same
+// 16 columns, row r in register v and r + 1 in v + 1; the swap of odd and even
+// 16-lane rows leaves gate in one register and up in the other, of row r in
+// lanes 0..15 and r + 1 in lanes 16..31.
+__device__ __forceinline__ void w4_store_pair(const gemm_f32x16 a, uint16_t* h, const W4Tile& t, int M, int N, int i,
+                                              bool poison, int wave, int lane) {
+    const int col = t.n0 + wave * 16 + (lane & 15);
+#pragma unroll
+    for (int v = 0; v < 16; v += 2) {
+        const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(a[v]), __float_as_uint(a[v + 1]), false, false);
+        const float o = silu_mul(__uint_as_float(s[0]), __uint_as_float(s[1]));
+        const int row = t.m0 + i * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3) + (lane >> 4 & 1);
+        if (row < M && col < N)
+            h[static_cast<size_t>(row) * N + col] =
+                poison ? static_cast<uint16_t>(0x7FC0u) : static_cast<uint16_t>(w4_pack_bf16(o, o) & 0xFFFFu);
+    }
+}
+
 // Paired gate/up tiles (blockIdx.y = block of 128 output columns), every K
 // step: h[r][c] = bf16(SiLU(x W_gate^T) * (x W_up^T)), rounded to nearest
 // even -- the fp32 products of two gemm_w4_kernel calls through silu_mul,
@@ -436,32 +449,21 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4_kernel(const uint16_t* __rest
 template <int BM, int NW, int SG>
 __global__ __launch_bounds__(64 * NW) void gemm_w4_pair_kernel(const uint16_t* __restrict__ xb, GemmMats gm,
                                                                uint16_t* __restrict__ h, int M, int K) {
-    static_assert(BM == 256 && NW == 4, "paired tiles: 4 waves of 256 x (32 gate + 32 up) columns");
     using L = W4Layout<BM, NW>;
     constexpr int TM = L::TM;
     extern __shared__ uint4 w4_lds[];
     char* lds = reinterpret_cast<char*>(w4_lds);
-    const int lane = threadIdx.x & 63, hb = lane >> 5;
+    const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int N = gm.n_out[0];
-    const W4Tile t = w4_tile_pair<BM>(xb, gm, M, N, K, blockIdx.x, blockIdx.y);
+    const W4Tile t = w4_tile_pair<BM>(xb, gm, M, N, K, blockIdx.x, blockIdx.y, wave);
     W4Src<BM, NW> src;
     w4_src<BM, NW, true>(src, K, wave, lane);
     W4Acc<BM, NW> acc;
     w4_zero<BM, NW>(acc);
     w4_segment<BM, NW, SG, true>(acc, lds, t, src, 0, K >> 6, wave, lane);
-    const int col = t.n0 + wave * 32 + (lane & 31);
-    if (col >= N) return;
 #pragma unroll
-    for (int i = 0; i < TM; i++)
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int row = t.m0 + i * 32 + 8 * (v >> 2) + 4 * hb + (v & 3);
-            if (row < M) {
-                const float a = silu_mul(acc[i][0][v], acc[i][1][v]);
-                h[static_cast<size_t>(row) * N + col] = static_cast<uint16_t>(w4_pack_bf16(a, a) & 0xFFFFu);
-            }
-        }
+    for (int i = 0; i < TM; i++) w4_store_pair(acc[i][0], h, t, M, N, i, false, wave, lane);
 }
 
 // Stream-K: the tiles (m block major) are split into nx contiguous groups,
@@ -514,31 +516,6 @@ struct SkGroup {
     __device__ int phys(int s) const { return xcd + nx * s; }
 };
 
-// Part hp of NP of a paired tile's outputs: h = bf16(SiLU(gate) * up) of
-// the accumulator rows i with i TN / (TM TN / NP) = hp; NaN if `poison`.
-template <int BM, int NW, int NP>
-__device__ __forceinline__ void w4_store_pair_rows(const W4Acc<BM, NW>& acc, uint16_t* h, const W4Tile& t, int M,
-                                                   int N, int hp, bool poison, int wave, int lane) {
-    constexpr int TM = W4Layout<BM, NW>::TM, TN = W4Layout<BM, NW>::TN;
-    static_assert(TN == 2, "paired tiles hold a gate and an up block per wave");
-    const int hb = lane >> 5;
-    const int col = t.n0 + wave * 32 + (lane & 31);
-    if (col >= N) return;
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-        if ((i * TN) / (TM * TN / NP) != hp) continue;
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const int row = t.m0 + i * 32 + 8 * (v >> 2) + 4 * hb + (v & 3);
-            if (row < M) {
-                const float a = silu_mul(acc[i][0][v], acc[i][1][v]);
-                h[static_cast<size_t>(row) * N + col] =
-                    poison ? static_cast<uint16_t>(0x7FC0u) : static_cast<uint16_t>(w4_pack_bf16(a, a) & 0xFFFFu);
-            }
-        }
-    }
-}
-
 // Segment [it, stop) of a stream-K range (stop at most its tile's end).
 // NTL: tiles per block row (the N blocks of gm, or of the paired columns).
 template <int BM, int NW, int SG, bool PAIR>
@@ -563,8 +540,9 @@ __device__ __forceinline__ void w4_sk_segment(char* lds, const uint16_t* xb, con
     const int nt = tile % NTL, mk = PAIR ? 0 : gm_mat(gm, nt);
     const int N = gm.n_out[mk];
     float* const out = gm.out[mk];
-    const W4Tile t = PAIR ? w4_tile_pair<BM>(xb, gm, M, N, K, tile / NTL, nt)
-                          : w4_tile<BM>(xb, gm.w[mk], gm.s[mk], gm.b[mk], M, N, K, tile / NTL, nt - gm.nb0[mk]);
+    const W4Tile t = PAIR ? w4_tile_pair<BM>(xb, gm, M, N, K, tile / NTL, nt, wave)
+                          : w4_tile<BM>(xb, gm.w[mk], gm.s[mk], gm.b[mk], M, N, K, tile / NTL, nt - gm.nb0[mk],
+                                        wave);
     w4_zero<BM, NW>(acc);
     w4_segment<BM, NW, SG, PAIR>(acc, lds, t, src, k0, nk, wave, lane);
     if (stop < tile_start + G) {
@@ -618,7 +596,7 @@ __device__ __forceinline__ void w4_sk_segment(char* lds, const uint16_t* xb, con
         // in turn through LDS, then the part is stored, so only a quarter of
         // the accumulators is ever live in VGPRs
         constexpr int PB = NB / kSkParts;                          // blocks per part
-        constexpr int PCH = PB * 16;                               // 1 KiB chunks per part
+        constexpr int PCH = PB * 4 * NW;                           // 1 KiB chunks per part
 #pragma unroll
         for (int h = 0; h < kSkParts; h++) {
             for (int j = wg - 1; j >= j1; j--) {
@@ -648,7 +626,10 @@ __device__ __forceinline__ void w4_sk_segment(char* lds, const uint16_t* xb, con
                     }
                 __syncthreads();                               // before the next copies overwrite LDS
             }
-            if constexpr (PAIR) w4_store_pair_rows<BM, NW, kSkParts>(acc, hout, t, M, N, h, poison, wave, lane);
+            if constexpr (PAIR) {
+#pragma unroll
+                for (int b = 0; b < PB; b++) w4_store_pair(acc[h * PB + b][0], hout, t, M, N, h * PB + b, poison, wave, lane);
+            }
             else w4_store_rows<BM, NW, kSkParts>(acc, out, t, M, N, h, poison, wave, lane);
         }
     }
@@ -659,7 +640,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_w4_sk_kernel(const uint16_t* __r
                                                              float* __restrict__ part, unsigned* __restrict__ flags,
                                                              unsigned* __restrict__ ctl, int M, int K, int nx,
                                                              uint16_t* __restrict__ hout) {
-    static_assert(BM == 256 && NW == 4, "stream-K slots assume 256 x 256 tiles of 4 waves");
+    static_assert(BM == 256 && (!PAIR || NW == 8), "stream-K slots hold 256 x 256 tiles");
     extern __shared__ uint4 w4_lds[];
     char* lds = reinterpret_cast<char*>(w4_lds);
     const int tid = threadIdx.x, lane = tid & 63;
@@ -744,45 +725,60 @@ int launch_w4_sk(const uint16_t* xb, const GemmMats& gm, float* part, unsigned* 
     return 0;
 }
 
-template <int SG>
+template <int BM, int SG>
 int launch_w4_pair(const uint16_t* xb, const GemmMats& gm, uint16_t* h, int M, int K, hipStream_t st) {
-    auto kern = gemm_w4_pair_kernel<256, 4, SG>;
-    constexpr size_t lds = w4_lds_bytes(256, SG);
+    auto kern = gemm_w4_pair_kernel<BM, 8, SG>;
+    constexpr size_t lds = w4_lds_bytes(BM, SG);
     static std::atomic<uint64_t> lds_raised{0};
     if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kern), lds, lds_raised)) return rc;
-    hipLaunchKernelGGL(kern, dim3((M + 255) / 256, (gm.n_out[0] + 127) / 128), dim3(256), lds, st, xb, gm, h, M, K);
+    hipLaunchKernelGGL(kern, dim3((M + BM - 1) / BM, (gm.n_out[0] + 127) / 128), dim3(64 * 8), lds, st, xb, gm, h, M, K);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(Q4_EHIP, "prefill gate/up gemm launch: %s", hipGetErrorString(e));
     return 0;
 }
 
-int gemm_w4_pair(const uint16_t* xb, const GemmMats& gm, uint16_t* h, int M, int K, hipStream_t st) {
+template <int BM>
+int pair_by_groups(const uint16_t* xb, const GemmMats& gm, uint16_t* h, int M, int K, hipStream_t st) {
     const int sg = w4_groups(gm, K);
-    return sg == 8 ? launch_w4_pair<8>(xb, gm, h, M, K, st)
-                   : sg == 2 ? launch_w4_pair<2>(xb, gm, h, M, K, st) : launch_w4_pair<1>(xb, gm, h, M, K, st);
+    return sg == 8 ? launch_w4_pair<BM, 8>(xb, gm, h, M, K, st)
+                   : sg == 2 ? launch_w4_pair<BM, 2>(xb, gm, h, M, K, st) : launch_w4_pair<BM, 1>(xb, gm, h, M, K, st);
+}
+
+int gemm_w4_pair(const uint16_t* xb, const GemmMats& gm, uint16_t* h, int M, int K, int bm, hipStream_t st) {
+    switch (bm) {
+        case 64: return pair_by_groups<64>(xb, gm, h, M, K, st);
+        case 128: return pair_by_groups<128>(xb, gm, h, M, K, st);
+        case 192: return pair_by_groups<192>(xb, gm, h, M, K, st);
+        default: return pair_by_groups<256>(xb, gm, h, M, K, st);
+    }
+}
+
+template <int BM, int NW>
+int w4_by_groups(const uint16_t* xb, const GemmMats& gm, float* part, int M, int K, int S, int kt_split, int ldp,
+                 hipStream_t st) {
+    const int sg = w4_groups(gm, K);
+    return sg == 8 ? launch_w4<BM, NW, 8>(xb, gm, part, M, K, S, kt_split, ldp, st)
+                   : sg == 2 ? launch_w4<BM, NW, 2>(xb, gm, part, M, K, S, kt_split, ldp, st)
+                             : launch_w4<BM, NW, 1>(xb, gm, part, M, K, S, kt_split, ldp, st);
 }
 
 int gemm_w4(const uint16_t* xb, const GemmMats& gm, float* part, int M, int K, int bm, int S, int kt_split, int ldp,
             hipStream_t st) {
-    // 256-row tiles: 4 waves of 256 x 64 (a dequantised weight word feeds 8
-    // MFMAs); 128-row tiles: 8 waves of 64 x 64
-    const int sg = w4_groups(gm, K);
-    if (bm == 256)
-        return sg == 8 ? launch_w4<256, 4, 8>(xb, gm, part, M, K, S, kt_split, ldp, st)
-                       : sg == 2 ? launch_w4<256, 4, 2>(xb, gm, part, M, K, S, kt_split, ldp, st)
-                                 : launch_w4<256, 4, 1>(xb, gm, part, M, K, S, kt_split, ldp, st);
-    return sg == 8 ? launch_w4<128, 8, 8>(xb, gm, part, M, K, S, kt_split, ldp, st)
-                   : sg == 2 ? launch_w4<128, 8, 2>(xb, gm, part, M, K, S, kt_split, ldp, st)
-                             : launch_w4<128, 8, 1>(xb, gm, part, M, K, S, kt_split, ldp, st);
+    switch (bm) {
+        case 64: return w4_by_groups<64, 8>(xb, gm, part, M, K, S, kt_split, ldp, st);
+        case 128: return w4_by_groups<128, 8>(xb, gm, part, M, K, S, kt_split, ldp, st);
+        case 192: return w4_by_groups<192, 8>(xb, gm, part, M, K, S, kt_split, ldp, st);
+        default: return w4_by_groups<256, 8>(xb, gm, part, M, K, S, kt_split, ldp, st);
+    }
 }
 
 template <bool PAIR>
 int sk_by_groups(const uint16_t* xb, const GemmMats& gm, float* part, unsigned* flags, unsigned* ctl, uint16_t* h, int M,
                  int K, int P, int nx, hipStream_t st) {
     const int sg = w4_groups(gm, K);
-    return sg == 8 ? launch_w4_sk<256, 4, 8, PAIR>(xb, gm, part, flags, ctl, M, K, P, nx, h, st)
-                   : sg == 2 ? launch_w4_sk<256, 4, 2, PAIR>(xb, gm, part, flags, ctl, M, K, P, nx, h, st)
-                             : launch_w4_sk<256, 4, 1, PAIR>(xb, gm, part, flags, ctl, M, K, P, nx, h, st);
+    return sg == 8 ? launch_w4_sk<256, 8, 8, PAIR>(xb, gm, part, flags, ctl, M, K, P, nx, h, st)
+                   : sg == 2 ? launch_w4_sk<256, 8, 2, PAIR>(xb, gm, part, flags, ctl, M, K, P, nx, h, st)
+                             : launch_w4_sk<256, 8, 1, PAIR>(xb, gm, part, flags, ctl, M, K, P, nx, h, st);
 }
 
 int gemm_w4_sk(const uint16_t* xb, const GemmMats& gm, float* part, unsigned* flags, unsigned* ctl, int M, int K,

@@ -1211,12 +1211,26 @@ int scratch_workspace(Workspace* ws) {
     return 0;
 }
 
-// The prefill GEMM's plan: data-parallel tiles of height bm (256 or 128)
-// with K split S ways (S > 1: partial planes and a sum launch), or, when
+// The prefill GEMM's plan: data-parallel tiles of height bm (256, 192, 128 or
+// 64) with K split S ways (S > 1: partial planes and a sum launch), or, when
 // sk_p > 0, stream-K over sk_p workgroups of 256 x 256 tiles.
 struct PrefillPlan {
     int bm = 256, S = 1, sk_p = 0, sk_nx = 1;
 };
+
+// Estimated us of wgs data-parallel workgroups of kts K steps each, from
+// timings over 17 to 1000 rows (K 3584 and 18944, N 3584 to 18944): a step of
+// a lone tile takes 0.77 / 0.89 / 1.09 / 1.31 us at 64 / 128 / 192 / 256
+// rows (dequantising the tile's 256 columns and the copies are most of the
+// low ones), up to 35 % more as the CUs fill (the clock drops), and a round
+// 3 us of pipeline fill and stores.  One workgroup per CU, two of 64 rows
+// (72 KiB of LDS), which then take up to 75 % longer.
+double prefill_dp_us(int bm, long wgs, int kts, int cus) {
+    const double t0 = bm == 64 ? 0.77 : bm == 128 ? 0.89 : bm == 192 ? 1.09 : 1.31, grow = bm == 64 ? 0.75 : 0.35;
+    const long cap = static_cast<long>(cus) * (bm == 64 ? 2 : 1), full = wgs / cap, rest = wgs % cap;
+    const double us = full * (kts * t0 * (1.0 + grow) + 3.0);
+    return rest ? us + kts * t0 * (1.0 + grow * static_cast<double>(rest) / cap) + 3.0 : us;
+}
 
 // XCD groups of a stream-K launch of P workgroups over `tiles` tiles: one per
 // XCD when P spreads evenly over 8 of them and there are tiles for each.
@@ -1227,17 +1241,17 @@ bool sk_ok(int P, long tiles, long T, int cus) {
     return P >= 1 && P <= cus && P <= T && P / nx >= (tiles + nx - 1) / nx;
 }
 
-// From a cost model of the kernels measured at M = 512: a K step of a
-// 256 x 256 tile takes about 2.3 us, of a 128 x 256 tile 2.0 us, plus about
-// two steps of pipeline fill per workgroup; data-parallel workgroups run in
-// rounds of one per CU, and split partials cost a write and a read of
-// M x N floats each (about 4.5 TB/s) plus the sum launch.  Stream-K keeps
-// every CU busy, where a step takes about 2.7 us (the clock drops), and a
-// tile's owner adds one 256 KiB partial per range before it in the tile
-// (about 5 us each, serially), plus about 20 us of partial stores, restarts
-// and imbalance: it wins only where each tile has one or two ranges
-// (gate/up of a 512-token prompt: 124 us against 132 us).
-// Q4_GEMM_PLAN="dp:<bm>:<S>" or "sk:<P>" sets the plan instead (for tests
+// The plan of least estimated time: prefill_dp_us over tile heights and
+// splits, whose partials cost a write and a read of M x N floats each (about
+// 4.5 TB/s) plus the sum launch; or stream-K, which keeps every CU busy
+// (about 1.7 us a step) but whose tiles' owners add one 256 KiB partial per
+// range before theirs (about 5 us each, serially), plus about 28 us of
+// partial stores, restarts and imbalance.  At 512 rows it picks, against the
+// plans before the 64- to 192-row tiles: q/k/v three splits of 128 rows, 38
+// us (48), o four of 128 rows, 34 us (38), gate or up alone 192 rows, 86 us
+// (101); at 37 rows q/k/v 64 rows, 16.6 us (20).
+// Q4_GEMM_PLAN="rows:<bm>:<S>" (or "dp:", 128 and 256 rows only) or "sk:<P>"
+// sets the plan instead (for tests
 // and measurement).
 // nblocks: 256-column blocks of the launch; ncols: its columns.
 int plan_prefill(int m, int nblocks, int ncols, int n_in, PrefillPlan* out) {
@@ -1258,35 +1272,38 @@ int plan_prefill(int m, int nblocks, int ncols, int n_in, PrefillPlan* out) {
             if ((p.bm != 256 && p.bm != 128) || !splits_ok(p.S))
                 return fail(Q4_EARG, "Q4_GEMM_PLAN=%s: bm is 128 or 256, and S splits of %d K steps must all be "
                                      "non-empty", env, G);
+        } else if (sscanf(env, "rows:%d:%d%c", &p.bm, &p.S, &tail) == 2) {
+            if ((p.bm != 256 && p.bm != 192 && p.bm != 128 && p.bm != 64) || !splits_ok(p.S))
+                return fail(Q4_EARG, "Q4_GEMM_PLAN=%s: bm is 64, 128, 192 or 256, and S splits of %d K steps must "
+                                     "all be non-empty", env, G);
         } else {
-            return fail(Q4_EARG, "Q4_GEMM_PLAN=%s: expected dp:<bm>:<S> or sk:<P>", env);
+            return fail(Q4_EARG, "Q4_GEMM_PLAN=%s: expected dp:<bm>:<S>, rows:<bm>:<S> or sk:<P>", env);
         }
         *out = p;
         return 0;
     }
     PrefillPlan best_plan;
     double best = 1e30;
-    for (int bm : {256, 128}) {
+    for (int bm : {256, 192, 128, 64}) {
         const long tiles = static_cast<long>((m + bm - 1) / bm) * nblocks;
-        const double t_step = bm == 256 ? 2.3 : 2.0;
-        for (int S = 1; S <= 16 && G / S >= 2; S++) {
+        // (splits past two rounds only add partials)
+        for (int S = 1; S <= 32 && G / S >= 2 && (S == 1 || tiles * S <= 2L * cus); S++) {
             if (!splits_ok(S)) continue;
-            const int kts = (G + S - 1) / S;
-            const long rounds = (tiles * S + cus - 1) / cus;
-            const double est = static_cast<double>(rounds) * (kts + 2) * t_step +
-                               (S > 1 ? static_cast<double>(S) * m * ncols * 8.0 / 4.5e6 + 3.0 : 0.0);
+            const double est = prefill_dp_us(bm, tiles * S, (G + S - 1) / S, cus) +
+                               (S > 1 ? static_cast<double>(S) * m * ncols * 8.0 / 4.5e6 + 3.0 + 0.2 * S : 0.0);
             if (est < best) {
                 best = est;
                 best_plan = PrefillPlan{bm, S, 0};
             }
         }
     }
-    for (int P = 8; P <= cus; P += 8) {
+    // (few tiles: every owner would add many partials)
+    for (int P = 8; P <= cus && tiles256 * 5 >= cus; P += 8) {
         if (!sk_ok(P, tiles256, T, cus) || sk_groups(P, tiles256) != 8) continue;
         const long Tg = (tiles256 + 7) / 8 * G, Pg = P / 8;
         const long L = (Tg + Pg - 1) / Pg, Lmin = Tg / Pg;
         const long partials = (G + Lmin - 1) / Lmin - 1;            // per owner, at most
-        const double est = static_cast<double>(L + 4) * 2.7 + static_cast<double>(partials) * 5.0 + 20.0;
+        const double est = static_cast<double>(L + 4) * 1.7 + static_cast<double>(partials) * 5.0 + 28.0;
         if (est < best) {
             best = est;
             best_plan = PrefillPlan{256, 1, P, 8};
@@ -1845,23 +1862,40 @@ int q4_gemm_bf16in_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate
     gm.b[1] = up_b;
     gm.n_out[0] = gm.n_out[1] = n_inter;
     gm.count = 2;
-    // one 256 x (128 + 128) tile per workgroup while the tiles fit the CUs
-    // in one round; past that, stream-K over one workgroup per CU, so that
-    // a last partial round does not double the time (Q4_PAIR_PLAN=dp or
-    // sk:<P> chooses)
-    const int cus = num_cus();
-    const long tiles = static_cast<long>((m + 255) / 256) * ((n_inter + 127) / 128);
-    const long T = tiles * (n_in / 64);
-    int P = tiles > cus ? static_cast<int>(std::min<long>(cus >= 8 ? cus / 8 * 8 : cus, T)) : 0;
+    // one BM x (128 + 128) tile per workgroup, of the height with the least
+    // estimated time, or past one round of 256-row tiles stream-K over one
+    // workgroup per CU, so that a last partial round does not double the time
+    // (about 1.9 us a step and 53 us of partials, restarts and imbalance).
+    // n_inter 18944, n_in 3584: 64 rows up to 64 (50 us; 256 rows take 84),
+    // 128 up to 128 (57), 256 up to 256 (90), 128 up to 384 (138; stream-K
+    // 172), 192 at 512 (169; 176), stream-K at 1000 (299).
+    // Q4_PAIR_PLAN=dp (256 rows), rows:<bm> or sk:<P> chooses.
+    const int cus = num_cus(), G = n_in / 64;
+    const long nblocks = (n_inter + 127) / 128, tiles = static_cast<long>((m + 255) / 256) * nblocks;
+    const long T = tiles * G;
+    int bm = 256, P = 0;
+    double best = 1e30;
+    for (int h : {256, 192, 128, 64}) {
+        const double est = prefill_dp_us(h, (m + h - 1) / h * nblocks, G, cus);
+        if (est < best) {
+            best = est;
+            bm = h;
+        }
+    }
+    if (tiles > cus) {
+        const int p = static_cast<int>(std::min<long>(cus >= 8 ? cus / 8 * 8 : cus, T));
+        if (1.9 * static_cast<double>(T) / p + 53.0 < best) P = p;
+    }
     if (const char* env = getenv("Q4_PAIR_PLAN")) {
         char tail = 0;
         int p = 0;
-        if (std::strcmp(env, "dp") == 0) P = 0;
+        if (std::strcmp(env, "dp") == 0) P = 0, bm = 256;
+        else if (sscanf(env, "rows:%d%c", &p, &tail) == 1 && (p == 64 || p == 128 || p == 192 || p == 256)) P = 0, bm = p;
         else if (sscanf(env, "sk:%d%c", &p, &tail) == 1 && p >= 1 && p <= cus && p <= T) P = p;
-        else return fail(Q4_EARG, "Q4_PAIR_PLAN=%s: expected dp or sk:<P> with P in [1, %ld]", env,
+        else return fail(Q4_EARG, "Q4_PAIR_PLAN=%s: expected dp, rows:<bm> or sk:<P> with P in [1, %ld]", env,
                          std::min<long>(cus, T));
     }
-    if (P == 0) return gemm_w4_pair(xb, gm, h, m, n_in, st);
+    if (P == 0) return gemm_w4_pair(xb, gm, h, m, n_in, bm, st);
     Workspace* ws;
     if ((rc = stream_workspace(st, &ws))) return rc;
     if ((rc = sk_workspace(*ws, P, st))) return rc;

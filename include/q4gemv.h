@@ -186,13 +186,13 @@ int q4_gemm_bf16in_multi_dev(int count, const uint32_t *const *w, const uint16_t
  * h[m][n_inter] = bf16(SiLU(x . Wg^T) * (x . Wu^T)) as bf16 bit patterns,
  * rounded to nearest even -- the down projection's operand.  One launch:
  * each tile holds the same 128 rows of both matrices, so the SiLU * mul is
- * the GEMM's epilogue.  While the 256 x 128 output tiles fit the CUs in
- * one round, each tile is one workgroup and the fp32 sums are those of
- * q4_gemm_bf16in_multi_dev on {gate, up} without split-K (bit for bit);
- * past that (a 512-token prompt at n_inter 18944 has 296 tiles) the tiles'
+ * the GEMM's epilogue.  With a tile per workgroup the fp32 sums are those of
+ * q4_gemm_bf16in_multi_dev on {gate, up} without split-K (bit for bit,
+ * whatever the tile's height); where many rows would leave a last partial
+ * round of tiles (past about 600 rows at n_inter 18944) the tiles'
  * K steps are shared out stream-K over one workgroup per CU and a tile's
  * partial sums are added in a fixed order, which may move a value by one
- * bf16 unit.  Q4_PAIR_PLAN=dp or sk:<P> forces either form.  gs must be
+ * bf16 unit.  Q4_PAIR_PLAN=dp, rows:<bm> or sk:<P> forces a form.  gs must be
  * 64; w and x 16-byte aligned.  The stream-K form uses the calling
  * stream's workspace, which grows on first use (run the largest call once
  * before capturing it in a graph). */

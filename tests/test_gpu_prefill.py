@@ -233,3 +233,38 @@ def test_gemm_bf16_group_copies(monkeypatch, groups, plans):
             assert torch.equal(got, one), "the copies' width changed the result"
     _plan(monkeypatch, None)
     assert q4.prefill_errors() == 0
+
+
+@pytest.mark.parametrize("m", [1, 33, 64, 65, 129, 200, 257])
+def test_gemm_bf16_tile_heights(monkeypatch, m):
+    """Every tile height and split of it, rows at and past its edges: within
+    the bar of the exact-operand product, unsplit sums the same bits whatever
+    the height; the paired gate/up tiles the same bits at every height too."""
+    import torch
+    n_out, n_in = 520, 64 * 9
+    (tw, ts, tb, tx), exact = _operands(940 + m, m, n_out, n_in)
+    (uw, us, ub, _), _ = _operands(960 + m, m, n_out, n_in)
+    first = pair = None
+    for bm in (64, 128, 192, 256):
+        for split in (1, 2, 9):                                # 9: one K step each
+            print(f"tile heights m={m} rows:{bm}:{split}", flush=True)
+            _plan(monkeypatch, f"rows:{bm}:{split}")
+            got = q4.gemm_bf16_dev(tw, ts, tb, tx)
+            torch.cuda.synchronize()
+            assert oracle.normwise_rel(got.cpu().numpy(), exact) < EXACT_OPERAND_TOL
+            if split == 1:
+                first = got if first is None else first
+                assert torch.equal(got, first), bm
+        monkeypatch.setenv("Q4_PAIR_PLAN", f"rows:{bm}")
+        h = q4.gemm_bf16_gate_up_silu_dev((tw, ts, tb), (uw, us, ub), tx.bfloat16())
+        torch.cuda.synchronize()
+        pair = h if pair is None else pair
+        assert torch.equal(h, pair), bm
+    _plan(monkeypatch, "rows:256:1")
+    monkeypatch.delenv("Q4_PAIR_PLAN")
+    g, u = q4.gemm_bf16_multi_dev([(tw, ts, tb), (uw, us, ub)], tx.bfloat16())
+    want = torch.nn.functional.silu(g.double()) * u.double()
+    torch.cuda.synchronize()
+    err = (pair.double() - want).abs() / want.abs().clamp_min(1e-30)
+    assert float(err.max()) < 2.0 ** -8                          # one rounding to bf16 of an fp32 expression
+    _plan(monkeypatch, None)
