@@ -1,12 +1,11 @@
 """GPU checks of the prompt chunk's causal attention, q4_prompt_attention_dev
-(head_dim 128 on the matrix cores with two-term fp16 operands, 64 and 32 on
-the vector ALUs), against the reference's sdpa with causal=True
+(on the matrix cores with two-term fp16 operands), against the reference's sdpa with causal=True
 (hetero/cpu_model.py:233-252) evaluated in float64 here: query row i of a
 chunk at positions [pos0, pos0 + rows) sees the cache positions
 [0, pos0 + i], query head h reads kv head h / (nh / nkv),
 o = softmax((q . k) * scale) v.
 
-Both kernels evaluate the softmax online (tile by tile) and sum in fp32, so
+The kernel evaluates the softmax online (tile by tile) and sum in fp32, so
 the bar is fp32 rounding, not bit equality: normwise relative error (max
 |diff| / max |ref|) below ATTN_TOL = 2e-6, stated here.  A planted
 mistake -- one position too many or too few, the wrong kv head, a missing
@@ -44,7 +43,7 @@ def sdpa_causal(q, kc, vc, pos0, nh, nkv, scale, extra=0, head_shift=0):
 
 # (heads, kv heads, head_dim, rows, pos0, cap): a 512-token Qwen2.5-7B chunk
 # (7 heads per kv head, 8 tiles); a chunk after a context; a single row;
-# 1 and 8 heads per kv head; head_dim 64 and 32 (vector path); ragged row
+# 1 and 8 heads per kv head; head_dim 64 and 32; ragged row
 # blocks and tiles throughout
 CASES = [(28, 4, 128, 512, 0, 512), (28, 4, 128, 70, 64, 200), (28, 4, 128, 1, 300, 301),
          (8, 8, 128, 33, 100, 140), (16, 2, 128, 40, 5, 45), (4, 2, 128, 24, 0, 24),
@@ -94,3 +93,84 @@ def test_planted_mistakes_exceed_the_bar():
                 sdpa_causal(q, kc, vc, pos0, nh, nkv, scale, head_shift=1),
                 sdpa_causal(q, kc, vc, pos0, nh, nkv, 1.0)):
         assert oracle.normwise_rel(bad, ref) > 1e3 * ATTN_TOL
+
+
+# The tiles of a row block go to 2 or 4 groups of waves and its heads to
+# workgroups of 1 to 4: fewer tiles than groups, a last round of some groups
+# only, rows that see none of a group's positions, heads that leave a
+# workgroup's last waves idle, few and many workgroups (pairs of heads while
+# they fit the 256 CUs).  The bar is the one above: the groups' sums are
+# merged by one more rescaling, 2 fp32 roundings against the up to 40 of the
+# tiles' running ones.
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv,d,rows,pos0", [
+    (7, 1, 128, 5, 62), (7, 1, 64, 16, 112), (5, 1, 128, 20, 250), (10, 2, 64, 700, 0), (12, 2, 32, 700, 60),
+    (28, 4, 128, 330, 15), (16, 8, 64, 17, 600), (3, 3, 128, 40, 127), (24, 3, 64, 48, 300), (15, 5, 128, 2, 2500)],
+    ids=lambda v: str(v))
+def test_prompt_attention_groups_and_heads(nh, nkv, d, rows, pos0):
+    import torch
+    rng = np.random.default_rng(nh * 100 + rows + pos0)
+    cap = pos0 + rows + 3
+    q = rng.normal(0, 2, (rows, nh * d)).astype(np.float32)
+    kc = rng.normal(0, 1, (nkv, cap, d)).astype(np.float16)
+    vc = rng.normal(0, 1, (nkv, cap, d)).astype(np.float16)
+    kc[:, pos0 + rows:] = np.nan                              # no row sees these
+    vc[:, pos0 + rows:] = np.nan
+    scale = ctypes.c_float(d ** -0.5).value
+    lib = q4.load()
+    tq, tk, tv = (torch.from_numpy(a).cuda() for a in (q, kc, vc))
+    out = torch.full((rows + 1, nh * d), -7.0, device="cuda")
+    rc = lib.q4_prompt_attention_dev(tq.data_ptr(), tk.data_ptr(), tv.data_ptr(), out.data_ptr(), rows, pos0, nh,
+                                     nkv, d, cap, scale, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, q4.last_error(lib)
+    got = out.cpu().numpy()
+    assert (got[rows] == -7.0).all()
+    err = oracle.normwise_rel(got[:rows], sdpa_causal(q, kc, vc, pos0, nh, nkv, scale))
+    assert err < ATTN_TOL, err
+
+
+def _one_head(q, k, v, scale):
+    """One query row over every position of one head."""
+    import torch
+    lib, (n, d) = q4.load(), k.shape
+    tq, tk, tv = (torch.from_numpy(a).cuda() for a in (q, k, v))
+    out = torch.zeros((1, d), device="cuda")
+    rc = lib.q4_prompt_attention_dev(tq.data_ptr(), tk.data_ptr(), tv.data_ptr(), out.data_ptr(), 1, n - 1, 1, 1, d,
+                                     n, scale, torch.cuda.current_stream().cuda_stream)
+    assert rc == 0, q4.last_error(lib)
+    return out.cpu().numpy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_prompt_attention_scores_of_minus_infinity(d):
+    """Scores of -inf over a whole tile leave the others' softmax alone; a row
+    whose every score is -inf is 0 / 0."""
+    n = 400
+    q = np.full((1, d), 1e38, np.float32)
+    k = np.full((n, d), -1.0, np.float16)                     # q . k = -1e38 d: -inf in fp32
+    v = np.random.default_rng(d).normal(0, 1, (n, d)).astype(np.float16)
+    assert np.isnan(_one_head(q, k, v, 1.0)).all()
+    for seen in (3, 70, 399):
+        k1 = k.copy()
+        k1[seen] = 0.0
+        np.testing.assert_array_equal(_one_head(q, k1, v, 1.0)[0], v[seen].astype(np.float32))
+    q[0, 5] = np.inf
+    assert np.isnan(_one_head(q, k, v, 1.0)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_prompt_attention_queries_past_fp16(d):
+    """Queries beyond fp16's range: scores of q = 2^17 and k of about 2^-14,
+    |s| up to 16, each to 2^-21 of its value (the two-term operands), so
+    probabilities to 16 x 2^-21 besides the fp32 rounding of ATTN_TOL."""
+    rng = np.random.default_rng(d)
+    n = 300
+    q = np.zeros((1, d), np.float32)
+    q[0, 3] = 2.0 ** 17
+    k = np.zeros((n, d), np.float16)
+    k[:, 3] = rng.choice([-1, 1], n) * (1 + rng.random(n)) * 2.0 ** -14
+    v = rng.normal(0, 1, (n, d)).astype(np.float16)
+    ref = sdpa_causal(q, k[None], v[None], n - 1, 1, 1, 1.0)
+    assert oracle.normwise_rel(_one_head(q, k, v, 1.0), ref) < ATTN_TOL + 2 * 16 * 2.0 ** -21
