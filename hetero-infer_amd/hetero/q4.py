@@ -190,9 +190,13 @@ def _ptr(t) -> int:
 # every tensor they pass (a too-small buffer would be read or written past
 # its end by a kernel) and raise before any library call.
 
+def _is_tensor(t, cls):
+    return type(t) is cls or isinstance(t, cls)               # the exact type first: torch's isinstance hook is slow
+
+
 def _need(t, name, dtypes, numel=None, shape=None):
     import torch
-    if not isinstance(t, torch.Tensor):
+    if not _is_tensor(t, torch.Tensor):
         raise TypeError(f"{name}: a torch tensor, got {type(t).__name__}")
     if t.dtype not in dtypes:
         raise TypeError(f"{name}: dtype {t.dtype}, expected {' or '.join(str(d) for d in dtypes)}")
@@ -209,10 +213,12 @@ def _gpu(*ts):
     """Every tensor given (None skipped) on one GPU; after the type and size
     checks, so that those report first."""
     ts = [t for t in ts if t is not None]
-    for t in ts:
-        if t.device.type != "cuda":
-            raise ValueError(f"a tensor on {t.device}: the library takes GPU tensors")
-    if len({t.device for t in ts}) > 1:
+    # device objects cost twice as much to read and compare (13 tensors: 8 us)
+    at = {t.get_device() if t.is_cuda else -1 for t in ts}
+    if -1 in at:
+        bad = next(t for t in ts if not t.is_cuda)
+        raise ValueError(f"a tensor on {bad.device}: the library takes GPU tensors")
+    if len(at) > 1:
         raise ValueError("tensors on more than one GPU")
 
 
@@ -223,26 +229,46 @@ def _f32():
 
 def _mat(mat, name="w"):
     """(n_out, n_in, gs) of a (w, scales, biases) triple: int32 words
-    [n_out, n_in / 8], 16-bit scales and biases [n_out, n_in / gs]."""
+    [n_out, n_in / 8], 16-bit scales and biases [n_out, n_in / gs].  Each
+    shape is read once and names are put together only for an error (three
+    matrices: 13 us before, as long as their kernel, 8 so)."""
     import torch
     w, sc, b = mat
-    if w.dim() != 2 or sc.dim() != 2:
+    ws, ss = w.shape, sc.shape
+    if len(ws) != 2 or len(ss) != 2:
         raise ValueError(f"{name}: w and scales are 2-D")
-    n_out, n_in = w.shape[0], w.shape[1] * 8
-    if sc.shape[1] == 0 or n_in % sc.shape[1]:
-        raise ValueError(f"{name}: {sc.shape[1]} scale groups do not divide n_in {n_in}")
-    gs = n_in // sc.shape[1]
-    _need(w, name, (torch.int32, torch.uint32))
-    for t, k in ((sc, "scales"), (b, "biases")):
-        _need(t, f"{name} {k}", (torch.int16, torch.float16), shape=(n_out, n_in // gs))
+    n_out, n_in, groups = ws[0], ws[1] * 8, ss[1]
+    if groups == 0 or n_in % groups:
+        raise ValueError(f"{name}: {groups} scale groups do not divide n_in {n_in}")
+    gs = n_in // groups
+    words, halves = (torch.int32, torch.uint32), (torch.int16, torch.float16)
+    if not (_is_tensor(w, torch.Tensor) and w.dtype in words and w.is_contiguous()):
+        _need(w, name, words)
+    shape = (n_out, n_in // gs)
+    if not (_is_tensor(sc, torch.Tensor) and sc.dtype in halves and ss == shape and sc.is_contiguous()):
+        _need(sc, f"{name} scales", halves, shape=shape)
+    if not (_is_tensor(b, torch.Tensor) and b.dtype in halves and b.shape == shape and b.is_contiguous()):
+        _need(b, f"{name} biases", halves, shape=shape)
     return n_out, n_in, gs
+
+
+def _rows(x, n_in):
+    """x as rows of n_in."""
+    return x if x.dim() == 2 and x.shape[1] == n_in else x.reshape(-1, n_in)
+
+
+def _ptrs(*columns):
+    """One pointer array per column of tensors."""
+    arr = _VP * len(columns[0])
+    return [arr(*[t.data_ptr() for t in c]) for c in columns]
 
 
 def _same_in(mats, name="mats"):
     dims = [_mat(m, f"{name}[{i}]") for i, m in enumerate(mats)]
     if not dims:
         raise ValueError(f"{name}: no matrices")
-    if any(d[1:] != dims[0][1:] for d in dims):
+    _, n_in, gs = dims[0]
+    if any(d[1] != n_in or d[2] != gs for d in dims):
         raise ValueError(f"{name}: the matrices differ in n_in or group size")
     return dims
 
@@ -261,7 +287,7 @@ def gemv_dev(w, scales, biases, x, out=None, stream=None, lib=None):
     """out[m, n_out] = x[m, n_in] @ W^T on the GPU (torch tensors on one device)."""
     import torch
     n_out, n_in, gs = _mat((w, scales, biases))
-    x2 = _need(x, "x", _f32()).reshape(-1, n_in)
+    x2 = _rows(_need(x, "x", _f32()), n_in)
     if out is None:
         out = torch.empty((x2.shape[0], n_out), dtype=torch.float32, device=x.device)
     _need(out, "out", _f32(), numel=x2.shape[0] * n_out)
@@ -278,7 +304,7 @@ def gemv_multi_dev(mats, x, outs=None, stream=None, lib=None):
     import torch
     dims = _same_in(mats)
     n_in, gs = dims[0][1], dims[0][2]
-    x2 = _need(x, "x", _f32()).reshape(-1, n_in)
+    x2 = _rows(_need(x, "x", _f32()), n_in)
     m = x2.shape[0]
     if outs is None:
         outs = [torch.empty((m, d[0]), dtype=torch.float32, device=x.device) for d in dims]
@@ -287,11 +313,8 @@ def gemv_multi_dev(mats, x, outs=None, stream=None, lib=None):
     k = len(mats)
     _gpu(x2, *outs, *(t for m in mats for t in m))
     lib = lib or load()
-    arr = lambda vals: (ctypes.c_void_p * k)(*vals)
-    rc = lib.q4_gemv_multi_dev(k, arr([_ptr(a[0]) for a in mats]), arr([_ptr(a[1]) for a in mats]),
-                               arr([_ptr(a[2]) for a in mats]), arr([_ptr(o) for o in outs]),
-                               (ctypes.c_int * k)(*[a[0].shape[0] for a in mats]),
-                               _ptr(x2), m, n_in, gs, _stream(stream))
+    rc = lib.q4_gemv_multi_dev(k, *_ptrs(*zip(*mats), outs), (_I * k)(*[d[0] for d in dims]), _ptr(x2), m, n_in, gs,
+                               _stream(stream))
     check(lib, rc, "q4_gemv_multi_dev")
     return outs
 
@@ -320,10 +343,7 @@ def norm_gemv_multi_dev(mats, x, delta, norm_w, eps, x_out=None, outs=None, stre
     k = len(mats)
     _gpu(x, delta, norm_w, x_out, *outs, *(t for m in mats for t in m))
     lib = lib or load()
-    arr = lambda vals: (ctypes.c_void_p * k)(*vals)
-    rc = lib.q4_norm_gemv_multi_dev(k, arr([_ptr(a[0]) for a in mats]), arr([_ptr(a[1]) for a in mats]),
-                                    arr([_ptr(a[2]) for a in mats]), arr([_ptr(o) for o in outs]),
-                                    (ctypes.c_int * k)(*[a[0].shape[0] for a in mats]), _ptr(x),
+    rc = lib.q4_norm_gemv_multi_dev(k, *_ptrs(*zip(*mats), outs), (_I * k)(*[d[0] for d in dims]), _ptr(x),
                                     _ptr_or_null(delta), _ptr(norm_w), eps, _ptr_or_null(x_out), n_in, gs,
                                     _stream(stream))
     check(lib, rc, "q4_norm_gemv_multi_dev")
@@ -385,7 +405,7 @@ def gate_up_silu_dev(gate, up, x, h=None, stream=None, lib=None):
     """h[m, n_inter] = SiLU(x @ gate^T) * (x @ up^T); gate/up = (w, scales, biases)."""
     import torch
     n_inter, n_in, gs = _pair(gate, up)
-    x2 = _need(x, "x", _f32()).reshape(-1, n_in)
+    x2 = _rows(_need(x, "x", _f32()), n_in)
     if h is None:
         h = torch.empty((x2.shape[0], n_inter), dtype=torch.float32, device=x.device)
     _need(h, "h", _f32(), numel=x2.shape[0] * n_inter)
@@ -403,7 +423,7 @@ def mlp_dev(gate, up, down, x, h=None, out=None, stream=None, lib=None):
     n_inter, n_hidden, gs = _pair(gate, up)
     if _mat(down, "down") != (n_hidden, n_inter, gs):
         raise ValueError("down must map n_inter back to n_hidden with the same group size")
-    x2 = _need(x, "x", _f32()).reshape(-1, n_hidden)
+    x2 = _rows(_need(x, "x", _f32()), n_hidden)
     m = x2.shape[0]
     if h is None:
         h = torch.empty((m, n_inter), dtype=torch.float32, device=x.device)
@@ -423,7 +443,7 @@ def gemm_bf16_dev(w, scales, biases, x, out=None, stream=None, lib=None):
     """Prefill: out[m, n_out] = bf16(x) @ bf16(dequant(W))^T with fp32 accumulation."""
     import torch
     n_out, n_in, gs = _mat((w, scales, biases))
-    x2 = _need(x, "x", _f32()).reshape(-1, n_in)             # rounded to bf16 by the call
+    x2 = _rows(_need(x, "x", _f32()), n_in)             # rounded to bf16 by the call
     if out is None:
         out = torch.empty((x2.shape[0], n_out), dtype=torch.float32, device=x.device)
     _need(out, "out", _f32(), numel=x2.shape[0] * n_out)
@@ -441,7 +461,7 @@ def gemm_bf16_multi_dev(mats, x, outs=None, stream=None, lib=None):
     import torch
     dims = _same_in(mats)
     n_in, gs = dims[0][1], dims[0][2]
-    x2 = _need(x, "x", (torch.float32, torch.bfloat16)).reshape(-1, n_in)
+    x2 = _rows(_need(x, "x", (torch.float32, torch.bfloat16)), n_in)
     m = x2.shape[0]
     if outs is None:
         outs = [torch.empty((m, d[0]), dtype=torch.float32, device=x.device) for d in dims]
@@ -450,12 +470,8 @@ def gemm_bf16_multi_dev(mats, x, outs=None, stream=None, lib=None):
     k = len(mats)
     _gpu(x2, *outs, *(t for m in mats for t in m))
     lib = lib or load()
-    arr = lambda vals: (ctypes.c_void_p * k)(*vals)
     fn = lib.q4_gemm_bf16in_multi_dev if x2.dtype == torch.bfloat16 else lib.q4_gemm_bf16_multi_dev
-    rc = fn(k, arr([_ptr(a[0]) for a in mats]), arr([_ptr(a[1]) for a in mats]),
-            arr([_ptr(a[2]) for a in mats]), arr([_ptr(o) for o in outs]),
-            (ctypes.c_int * k)(*[a[0].shape[0] for a in mats]),
-            _ptr(x2), m, n_in, gs, _stream(stream))
+    rc = fn(k, *_ptrs(*zip(*mats), outs), (_I * k)(*[d[0] for d in dims]), _ptr(x2), m, n_in, gs, _stream(stream))
     check(lib, rc, fn.__name__)
     return outs
 
@@ -465,7 +481,7 @@ def gemm_bf16_gate_up_silu_dev(gate, up, xb, h=None, stream=None, lib=None):
     gate^T) * (x @ up^T)), the down projection's bf16 operand."""
     import torch
     n_inter, n_in, gs = _pair(gate, up)
-    x2 = _need(xb, "x", (torch.bfloat16,)).reshape(-1, n_in)
+    x2 = _rows(_need(xb, "x", (torch.bfloat16,)), n_in)
     if h is None:
         h = torch.empty((x2.shape[0], n_inter), dtype=torch.bfloat16, device=xb.device)
     _need(h, "h", (torch.bfloat16,), numel=x2.shape[0] * n_inter)

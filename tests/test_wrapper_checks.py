@@ -46,3 +46,46 @@ def test_wrong_types_and_sizes_raise_before_the_library():
                                 torch.zeros(1, dtype=torch.int64))
     with pytest.raises(ValueError, match="GPU tensors"):
         q4.gemv_dev(*m, x32)                                      # right types, but on the CPU
+
+
+class _At:
+    """What _gpu reads of a tensor."""
+
+    def __init__(self, index):
+        self.is_cuda, self.device = index is not None, "cpu" if index is None else f"cuda:{index}"
+        self.get_device = lambda: index
+
+
+@pytest.mark.parametrize("at,match", [((0, None, 0), "on cpu"), ((0, 1, 0), "more than one"), ((1, 1, 1), None)])
+def test_tensors_on_one_gpu(at, match):
+    ts = [_At(i) for i in at]
+    if match is None:
+        return q4._gpu(None, *ts)
+    with pytest.raises(ValueError, match=match):
+        q4._gpu(*ts, None)
+
+
+@pytest.mark.parametrize("bad,err,match", [
+    ({"w": lambda t: t.to(torch.int64)}, TypeError, "mats.1.: dtype"),
+    ({"w": lambda t: t.t().contiguous().t()}, ValueError, "mats.1.: not contiguous"),
+    ({"w": lambda t: t[0]}, ValueError, "2-D"),
+    ({"w": lambda t: t[:, :7]}, ValueError, "not contiguous"),
+    ({"sc": lambda t: t.repeat(1, 2)[:, :3]}, ValueError, "scale groups"),
+    ({"sc": lambda t: t[:, :0]}, ValueError, "scale groups"),
+    ({"sc": lambda t: t.float()}, TypeError, "mats.1. scales: dtype"),
+    ({"sc": lambda t: t[:3]}, ValueError, "mats.1. scales: shape"),
+    ({"b": lambda t: t[:, :1]}, ValueError, "mats.1. biases: shape"),
+    ({"b": lambda t: t.t().contiguous().t()}, ValueError, "mats.1. biases: not contiguous"),
+    ({"b": lambda t: t.flatten()}, ValueError, "mats.1. biases: shape"),
+    ({"sc": lambda t: t.repeat(1, 2), "b": lambda t: t.repeat(1, 2)}, ValueError, "differ in n_in or group size")],
+    ids=lambda v: str(v) if isinstance(v, str) else None)
+def test_every_matrix_of_a_call_is_checked(bad, err, match):
+    def mat(change=None):
+        t = {"w": torch.zeros(6, 16, dtype=torch.int32), "sc": torch.zeros(6, 2, dtype=torch.float16),
+             "b": torch.zeros(6, 2, dtype=torch.int16)}
+        for k, f in (change or {}).items():
+            t[k] = f(t[k])
+        return t["w"], t["sc"], t["b"]
+    assert q4._same_in([mat(), mat()]) == [(6, 128, 64)] * 2
+    with pytest.raises(err, match=match):
+        q4._same_in([mat(), mat(bad)])
