@@ -173,7 +173,7 @@ __device__ __forceinline__ float pa_rows4(float x, F f) {
 }
 
 template <int HPW, int KS, int D, bool BF>
-__global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(2, 2))) void prompt_attn_kernel(PromptAttnArgs a) {
+__global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(HPW == 1 ? 1 : 2, 2))) void prompt_attn_kernel(PromptAttnArgs a) {
     constexpr int NT = 64 * HPW, KT = D / 32, DT = D / 16;
     using S = PaShape<D, NT>;
     // a wave's maximum, sum and outputs, when the groups are merged

@@ -536,6 +536,7 @@ struct Workspace {
     size_t cap[7] = {0, 0, 0, 0, 0, 0, 0};      // bytes, in the order above
     bool in_graph[7] = {false, false, false, false, false, false, false};
     bool fixed = false;
+    bool prefill_reserved = false;              // part and sk once sized for every plan (prefill_workspace)
     std::vector<void*> retired;
 };
 enum WsBuf { kWsPlanes, kWsXsum, kWsXscale, kWsTmp, kWsXbf, kWsPart, kWsSk };
@@ -744,7 +745,7 @@ int try_fused_m(const MatList& ml, const float* x, int m, int n_in, int gs, hipS
     switch (m) {
         case 1: return try_fused<1>(mm, x, n_in, gs, st);
         case 2: return try_fused<2>(mm, x, n_in, gs, st);
-        // (3..8 rows take the matrix cores, or the split path where those
+        // (more take the matrix cores, or the split path where those
         // decline the shape)
         default: return 0;
     }
@@ -1719,16 +1720,13 @@ int stream_workspace(hipStream_t st, Workspace** ws) {
     return 0;
 }
 
-// Room for P stream-K partial slots (256 x 256 floats each) and the flags
-// of up to one workgroup per CU, then the control words; flags and control
-// words start at zero once, and every launch leaves them consistent (the
-// epoch scheme of q4_gemm.hip).
-int sk_workspace(Workspace& ws, int P, hipStream_t st) {
-    int rc;
+// The flags of up to one workgroup per CU, then the control words, which
+// start at zero once; every stream-K launch leaves them consistent (the epoch
+// scheme of q4_gemm.hip).
+int sk_flags(Workspace& ws, hipStream_t st) {
     const size_t flag_words = static_cast<size_t>(num_cus()) * 32 + kSkCtlWordsHost;
-    if ((rc = grow(ws, ws.part, kWsPart, static_cast<size_t>(P) * 256 * 256 * 4, st, "prefill"))) return rc;
     const size_t cap_before = ws.cap[kWsSk];
-    if ((rc = grow(ws, ws.sk, kWsSk, flag_words * 4, st, "prefill"))) return rc;
+    if (int rc = grow(ws, ws.sk, kWsSk, flag_words * 4, st, "prefill")) return rc;
     if (ws.cap[kWsSk] != cap_before) {
         const long n = static_cast<long>(ws.cap[kWsSk] / 4);
         hipLaunchKernelGGL(fill_zero_kernel, dim3((n + 255) / 256), dim3(256), 0, st, reinterpret_cast<float*>(ws.sk),
@@ -1737,6 +1735,31 @@ int sk_workspace(Workspace& ws, int P, hipStream_t st) {
     }
     return 0;
 }
+
+// Room for a prefill plan's partial sums (stream-K: 256 KiB per workgroup;
+// split-K: S M N floats) and, for stream-K, its flags.  A stream's first
+// prefill call outside a capture reserves what any plan takes -- two tiles of
+// 256 x 256 per CU, 128 MiB on 256 CUs, and the flags -- because which plan
+// and how much a call needs is not monotonic in its rows: a captured call may
+// split where the larger one run before it did not.  Where that much memory
+// is not to be had, a call takes what it needs.
+int prefill_workspace(Workspace& ws, size_t part_bytes, bool flags, hipStream_t st) {
+    if (!ws.prefill_reserved) {
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        HIP_TRY(hipStreamIsCapturing(st, &cs));
+        if (cs == hipStreamCaptureStatusNone) {
+            ws.prefill_reserved = true;
+            const size_t most = static_cast<size_t>(num_cus()) * 2 * 256 * 256 * 4;
+            if (grow(ws, ws.part, kWsPart, std::max(part_bytes, most), st, "prefill") || sk_flags(ws, st))
+                (void)hipGetLastError();
+        }
+    }
+    if (part_bytes)
+        if (int rc = grow(ws, ws.part, kWsPart, part_bytes, st, "prefill")) return rc;
+    return flags ? sk_flags(ws, st) : 0;
+}
+
+size_t sk_part_bytes(int P) { return static_cast<size_t>(P) * 256 * 256 * 4; }
 
 // q4_gemm_bf16_multi_dev on x given in fp32 (x, rounded to bf16 into the
 // workspace first) or already in bf16 (xb).
@@ -1788,11 +1811,8 @@ int gemm_bf16_multi(int count, const uint32_t* const* w, const uint16_t* const* 
     if ((rc = plan_prefill(m, nblocks, ncols, n_in, &plan))) return rc;
     const size_t mk = static_cast<size_t>(m) * n_in, mn = static_cast<size_t>(m) * ncols;
     if (!xb_in && (rc = grow(*ws, ws->xbf, kWsXbf, mk * 2, st, "prefill"))) return rc;
-    if (plan.sk_p > 0) {
-        if ((rc = sk_workspace(*ws, plan.sk_p, st))) return rc;
-    } else if (plan.S > 1 && (rc = grow(*ws, ws->part, kWsPart, plan.S * mn * 4, st, "prefill"))) {
-        return rc;
-    }
+    const size_t part_bytes = plan.sk_p > 0 ? sk_part_bytes(plan.sk_p) : plan.S > 1 ? plan.S * mn * 4 : 0;
+    if ((rc = prefill_workspace(*ws, part_bytes, plan.sk_p > 0, st))) return rc;
     const uint16_t* xb = xb_in;
     if (!xb) {
         const long n8 = static_cast<long>(mk / 8);
@@ -1895,10 +1915,12 @@ int q4_gemm_bf16in_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate
         else return fail(Q4_EARG, "Q4_PAIR_PLAN=%s: expected dp, rows:<bm> or sk:<P> with P in [1, %ld]", env,
                          std::min<long>(cus, T));
     }
+    Workspace* ws = nullptr;
+    if (P > 0 || tiles > cus) {                        // (tiles of less than 256 rows need none themselves)
+        if ((rc = stream_workspace(st, &ws))) return rc;
+        if ((rc = prefill_workspace(*ws, P > 0 ? sk_part_bytes(P) : 0, P > 0, st))) return rc;
+    }
     if (P == 0) return gemm_w4_pair(xb, gm, h, m, n_in, bm, st);
-    Workspace* ws;
-    if ((rc = stream_workspace(st, &ws))) return rc;
-    if ((rc = sk_workspace(*ws, P, st))) return rc;
     return gemm_w4_sk_pair(xb, gm, static_cast<float*>(ws->part), ws->sk, sk_ctl(*ws), h, m, n_in, P,
                            sk_groups(P, tiles), st);
 }

@@ -268,3 +268,29 @@ def test_gemm_bf16_tile_heights(monkeypatch, m):
     err = (pair.double() - want).abs() / want.abs().clamp_min(1e-30)
     assert float(err.max()) < 2.0 ** -8                          # one rounding to bf16 of an fp32 expression
     _plan(monkeypatch, None)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n_out,n_in,warm", [(512, 3584, 300), (3584, 3584, 520), (9000, 1024, 512)])
+def test_smaller_calls_under_capture_after_the_largest(n_out, n_in, warm):
+    """Plans and their scratch are not monotonic in the rows: after one call of
+    the most rows, every smaller one can be captured on the stream, and its
+    replays equal the eager result."""
+    import torch
+    s = torch.cuda.Stream()
+    (tw, ts, tb, tx), _ = _operands(911, warm, n_out, n_in)
+    eager = [q4.gemm_bf16_dev(tw, ts, tb, tx[:m]) for m in (17, 64, 130, 200, 257)]
+    torch.cuda.synchronize()
+    with torch.cuda.stream(s):
+        q4.gemm_bf16_dev(tw, ts, tb, tx, stream=s)
+    s.synchronize()
+    for e in eager:
+        m, out, g = e.shape[0], torch.full_like(e, float("nan")), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            q4.gemm_bf16_dev(tw, ts, tb, tx[:m], out=out, stream=s)
+        for _ in range(2):
+            out.fill_(float("nan"))
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(out, e), m
