@@ -67,10 +67,11 @@ struct PromptAttnArgs {
 // 512 rows after 1536 positions, 28 heads of 4 kv heads, head_dim 128: all
 // heads of a kv head in one workgroup, one group 89 us; two groups of four
 // heads 57; operands read a step ahead, unmasked tiles without the mask, sums
-// across lanes once at the end 46 (560 TFLOP/s of MFMA).  512 rows from an
-// empty cache 26 -> 16.5 us, 17 rows after 4000 positions 162 -> 57.  head_dim
-// 64 (on the vector ALUs before) 300 -> 28, 17 rows after 4000 (32 heads)
-// 497 -> 33; errors against float64 at these sizes are at most what they were.
+// across lanes once at the end 46-49; two tile buffers, one barrier a tile,
+// 45 (590 TFLOP/s of MFMA).  512 rows from an empty cache 26 -> 16 us, 17 rows
+// after 4000 positions 162 -> 57.  head_dim
+// 64 (on the vector ALUs before) 300 -> 27, 17 rows after 4000 (32 heads)
+// 497 -> 30; errors against float64 at these sizes are at most what they were.
 constexpr int kMRows = 16;                         // query rows per workgroup
 constexpr int kVRowH = kPTile + 8;                 // vt_s row: 64 fp16 + 8 pad (144 bytes: 16-byte reads spread)
 
@@ -179,15 +180,14 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
     // a wave's maximum, sum and outputs, when the groups are merged
     constexpr int PART = (2 + 4 * DT) * 64;
     static_assert((KS - 1) * HPW * PART * 4 <= KS * S::TILE * 2, "the parts reuse the tiles' LDS");
-    __shared__ __attribute__((aligned(16))) _Float16 lds[KS * S::TILE];
+    constexpr int NB = 2 * KS * S::TILE * 2 <= 160 * 1024 ? 2 : 1;     // tile buffers
+    __shared__ __attribute__((aligned(16))) _Float16 lds[NB * KS * S::TILE];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
     const int kg = wave / HPW;                                  // the wave's group
     const int tid = threadIdx.x - kg * NT;                      // thread of the group
     const int G = a.nh / a.nkv;
     const int h = blockIdx.z * HPW + wave % HPW;                // query head of the kv head
-    _Float16* k_s = lds + kg * S::TILE;
-    _Float16* vt_s = k_s + kPTile * S::KROW;
     const int c = lane & 15, qd = lane >> 4;
     const int kvh = blockIdx.y;
     const int r0 = (static_cast<int>(gridDim.x) - 1 - static_cast<int>(blockIdx.x)) * kMRows;
@@ -251,7 +251,11 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
 
     for (int t0 = 0; t0 < n_tiles; t0 += KS) {
         const int64_t c0 = static_cast<int64_t>(t0 + kg) * kPTile;
-        __syncthreads();                                       // every wave is done with the last tiles
+        // with two buffers, the barrier below has every wave past the tiles
+        // before the last, which this store replaces
+        _Float16* k_s = lds + ((NB == 2 ? t0 / KS & 1 : 0) * KS + kg) * S::TILE;
+        _Float16* vt_s = k_s + kPTile * S::KROW;
+        if (NB == 1) __syncthreads();                          // every wave is done with the last tiles
         pa_store<D, NT>(st, k_s, vt_s, tid);
         __syncthreads();
         if (t0 + KS < n_tiles) pa_load<D, NT>(st, a, head_row0, c0 + KS * kPTile, wg_last + 1 - c0 - KS * kPTile, tid);
@@ -411,8 +415,8 @@ void launch_prompt(const PromptAttnArgs& a, bool bf, hipStream_t st) {
 // workgroups of at most 4 heads, as even as they come (in two groups), which
 // read each K and V operand for more heads.  Pairs / fours, 28 heads of 4 kv
 // heads: 17 rows after 4000 positions 57 / 75 us, 100 after 2000 37 / 43, 256
-// after 1000 (256 workgroups of pairs) 25 / 29, 300 after 3000 (304) 94 / 64,
-// 512 after 1536 69 / 46.
+// after 1000 (256 workgroups of pairs) 25 / 29, 300 after 3000 (304) 94 / 60,
+// 512 after 1536 69 / 45.
 template <int D>
 void launch_prompt_heads(const PromptAttnArgs& a, bool bf, hipStream_t st) {
     const int G = a.nh / a.nkv, parts = (G + 3) / 4;
