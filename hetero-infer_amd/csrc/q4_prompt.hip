@@ -53,12 +53,22 @@ struct PromptAttnArgs {
 //   O^T += V^T P^T: D / 16 x 2 MFMAs; lane l holds query row c's outputs at
 //     dims 16 dt + 4 qd + v, rescaled by the row's correction in place.
 // The MFMA operands are fp16, the sums fp32.  Exact fp16 operands: the
-// cache is fp16, and q and p enter as two fp16 terms each (pa_split), two
-// MFMAs per product -- x to about 2^-21 of its value (or 2^-25 absolutely),
-// so the scores and weighted sums keep fp32 accuracy.  q is multiplied by
-// scale * log2(e) first and the softmax taken with exp2, which is exp of the
-// scaled score.  Workgroups of the last rows, which see the most positions,
-// are launched first.
+// cache is fp16, and q and p enter as two fp16 terms each, two MFMAs per
+// product, placed in fp16's range so that nothing that counts is rounded away:
+//   q: a row is scaled by a power of two to a maximum in [2^14, 2^15)
+//     (pa_split), each value to 2^-22 of itself or 2^-38 of the maximum;
+//   p: relative to a power of two just above its tile's own maximum (the
+//     online softmax's running maximum replaced by the tile's, so that
+//     rescaling l and O^T is exact) and times 2^15, as hi + lo (pa_split_p), to
+//     2^-23 of itself or 2^-40 of the tile's largest.
+// One dominant key (an attention sink, whose value is near zero) leaves
+// thousands of small p to make the output: from p below the running maximum,
+// unscaled and so to 2^-25, 6e-5 of them was lost 10 nats below that key and
+// 0.19 at 18; now 2e-6, as with fp32 probabilities, in the same time (45 us
+// against 46 for the case below).
+// q is multiplied by scale * log2(e) first and the softmax taken with exp2,
+// which is exp of the scaled score.  Workgroups of the last rows, which see
+// the most positions, are launched first.
 //
 // Bound by the matrix and vector ALUs of the few waves there are: 16 rows of
 // 28 heads are 28 waves, 512 rows 896, so the groups put two waves on every
@@ -153,15 +163,30 @@ __device__ __forceinline__ void pa_store(const PaStage<D, NT>& st, _Float16* k_s
     }
 }
 
-// x = hi + lo in fp16: hi is x with its low 13 significand bits cleared,
-// which fp16 holds exactly whenever |x| >= 2^-14, so no conversion of it can
-// round (the compiler may convert it again, packed, for the MFMA operand:
-// any rounding mode gives the same value); lo = fp16(x - hi), x - hi exact
-// in fp32.  Below 2^-14 the pair is within 2^-25 of x.
+// x = hi + lo in fp16: hi is the next value below |x| with its low 13
+// significand bits cleared, which fp16 holds exactly whenever it is at least
+// 2^-14, so no conversion of it can round (the compiler may convert it again,
+// packed, for the MFMA operand: any rounding mode gives the same value); lo =
+// fp16(x - hi), x - hi exact in fp32.  Below 2^-14 the pair is within 2^-24 of
+// x.  From 2^-2 on lo is never 0 and both have x's sign, so that an infinite
+// key gives an infinite score and not a NaN.
 __device__ __forceinline__ void pa_split(float x, _Float16& hi, _Float16& lo) {
-    const float h = __uint_as_float(__float_as_uint(x) & 0xFFFFE000u);
+    const float h = __uint_as_float(__float_as_uint(__fmul_rn(x, 0x1.fffffcp-1f)) & 0xFFFFE000u);
     hi = static_cast<_Float16>(h);
     lo = static_cast<_Float16>(__fsub_rn(x, h));
+}
+
+// Two values of p, times 2^15, as hi + lo: hi the nearest fp16 value, lo the
+// rest.  (Vector conversions: the packed one, where a product converted alone
+// becomes a half-register write of its own.)
+constexpr float kPScale = 32768.0f;
+constexpr float kPDrop = 32.0f;                    // see the softmax of a tile
+typedef float pa_f2 __attribute__((ext_vector_type(2)));
+typedef _Float16 pa_h2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void pa_split_p(const float (&x)[2], pa_h2& hi, pa_h2& lo) {
+    hi = __builtin_convertvector((pa_f2{x[0], x[1]}), pa_h2);
+    lo = __builtin_convertvector(
+        (pa_f2{__fsub_rn(x[0], static_cast<float>(hi[0])), __fsub_rn(x[1], static_cast<float>(hi[1]))}), pa_h2);
 }
 
 // f over the four lanes of a query row (c, c + 16, c + 32, c + 48), in all of them.
@@ -206,7 +231,7 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
     // q of row r, head kvh G + h, as the B operand of S^T: dims 32 ks + 8 qd ..
     const float qs = __fmul_rn(a.scale, 1.44269504088896341f);
     pa_h8 qh[KT], ql[KT];
-    float up = 1.0f;                                           // what the row's operands were scaled down by
+    float up;                                                  // what the row's operands were scaled down by
     {
         const float* src = a.q + static_cast<size_t>(r) * hd + static_cast<size_t>(kvh * G + h) * D + 8 * qd;
         float xv[KT][8], am = 0.0f;
@@ -224,15 +249,13 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
                 am = fmaxf(am, fabsf(xv[ks][i]));
             }
         }
-        // a row that reaches 2^15 is scaled into fp16's range by a power of two,
-        // its scores back
+        // the row's maximum to [2^14, 2^15) by a power of two, its scores back
+        // by the inverse (exact; a maximum below 2^-86 is no matter to exp2)
         am = pa_rows4(am, [](float x, float y) { return fmaxf(x, y); });
-        const int e = static_cast<int>(__float_as_uint(am) >> 23) - 127 - 14;
-        float down = 1.0f;
-        if (e > 0) {
-            down = __uint_as_float(static_cast<uint32_t>(127 - e) << 23);
-            up = __uint_as_float(static_cast<uint32_t>(127 + e) << 23);
-        }
+        int e = static_cast<int>(__float_as_uint(am) >> 23) - 127 - 14;
+        e = e < -100 ? -100 : e;
+        const float down = __uint_as_float(static_cast<uint32_t>(127 - e) << 23);
+        up = __uint_as_float(static_cast<uint32_t>(127 + e) << 23);
 #pragma unroll
         for (int ks = 0; ks < KT; ks++)
 #pragma unroll
@@ -243,11 +266,10 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
                 ql[ks][i] = lo;
             }
     }
-    const bool any_up = __any(up != 1.0f);
     pa_f4 o[DT];
 #pragma unroll
     for (int dt = 0; dt < DT; dt++) o[dt] = pa_f4{0.f, 0.f, 0.f, 0.f};
-    float m = -__builtin_inff(), l = 0.0f;
+    float m = -__builtin_inff(), l = 0.0f, top = m;             // top: the largest m
 
     for (int t0 = 0; t0 < n_tiles; t0 += KS) {
         const int64_t c0 = static_cast<int64_t>(t0 + kg) * kPTile;
@@ -286,12 +308,10 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
 #pragma unroll
             for (int mt = 0; mt < 4; mt++) s[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[ks & 1][mt], ql[ks], s[mt], 0, 0, 0);
         }
-        if (any_up)
-#pragma unroll
-            for (int mt = 0; mt < 4; mt++)
-#pragma unroll
-                for (int v = 0; v < 4; v++) s[mt][v] = __fmul_rn(s[mt][v], up);
-        // the running softmax of row r
+        // the softmax of row r (s times up are the scores), l and o relative to
+        // 2^m: m the tile's maximum rounded up, but at most kPDrop (64 where m's
+        // spacing is that wide) below the row's largest so far, so that o stays
+        // below 2^(64 + 15 + 16 + 16)
         if (c0 + kPTile - 1 > a.pos0 + r0) {                   // uniform: some row does not see all of the tile
             const int vis = static_cast<int>(my_last - c0 < kPTile ? my_last - c0 : kPTile) - 4 * qd;
 #pragma unroll
@@ -304,7 +324,10 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
         for (int mt = 0; mt < 4; mt++)
 #pragma unroll
             for (int v = 0; v < 4; v++) mx = fmaxf(mx, s[mt][v]);
-        const float mn = fmaxf(m, pa_rows4(mx, [](float x, float y) { return fmaxf(x, y); }));
+        mx = pa_rows4(mx, [](float x, float y) { return fmaxf(x, y); });
+        const float mc = __builtin_ceilf(__fmul_rn(mx, up));
+        top = fmaxf(top, mc);
+        const float mn = fmaxf(mc, __fsub_rn(top, kPDrop));
         const float ms = mn == -__builtin_inff() ? 0.0f : mn;  // the row sees none of the group's positions so far
         const float corr = __builtin_amdgcn_exp2f(__fsub_rn(m, ms));
         m = mn;
@@ -313,13 +336,21 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
 #pragma unroll
         for (int mt = 0; mt < 4; mt++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const float p = __builtin_amdgcn_exp2f(__fsub_rn(s[mt][v], ms));   // 0 where masked
-                ps = __fadd_rn(ps, p);
-                _Float16 hi, lo;
-                pa_split(p, hi, lo);
-                ph[mt >> 1][(mt & 1) * 4 + v] = hi;
-                pl[mt >> 1][(mt & 1) * 4 + v] = lo;
+            for (int v = 0; v < 4; v += 2) {
+                float p[2];
+#pragma unroll
+                for (int k = 0; k < 2; k++) {                  // 0 where masked
+                    p[k] = __fmul_rn(kPScale, __builtin_amdgcn_exp2f(__fmaf_rn(s[mt][v + k], up, -ms)));
+                    asm("" : "+v"(p[k]));                      // one product for l and hi
+                    ps = __fadd_rn(ps, p[k]);
+                }
+                pa_h2 hi, lo;
+                pa_split_p(p, hi, lo);
+#pragma unroll
+                for (int k = 0; k < 2; k++) {
+                    ph[mt >> 1][(mt & 1) * 4 + v + k] = hi[k];
+                    pl[mt >> 1][(mt & 1) * 4 + v + k] = lo[k];
+                }
             }
         l = __fadd_rn(__fmul_rn(l, corr), ps);
 #pragma unroll

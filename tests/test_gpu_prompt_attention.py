@@ -174,3 +174,82 @@ def test_prompt_attention_queries_past_fp16(d):
     v = rng.normal(0, 1, (n, d)).astype(np.float16)
     ref = sdpa_causal(q, k[None], v[None], n - 1, 1, 1, 1.0)
     assert oracle.normwise_rel(_one_head(q, k, v, 1.0), ref) < ATTN_TOL + 2 * 16 * 2.0 ** -21
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv,d,rows", [(1, 1, 32, 1), (1, 1, 64, 1), (1, 1, 128, 1), (7, 1, 64, 20),
+                                           (32, 8, 32, 280), (32, 8, 64, 280), (32, 8, 128, 280)],
+                         ids=lambda v: str(v))
+def test_prompt_attention_one_dominant_key(nh, nkv, d, rows):
+    """One key far above the others whose value is 0, so that the output is
+    made of the others' small probabilities, 10 to 19 nats below (positive
+    values: nothing averages out).  Scores of one product each, to 2^-22 (q's
+    two terms) + 2^-23 (fp32) of their value, one sign in a row, so
+    probabilities to that times the largest score, besides ATTN_TOL."""
+    rng = np.random.default_rng(d + rows)
+    pos0, worst = 4000, 0.0
+    for nats in (10.0, 14.0, 18.0):
+        q = np.zeros((rows, nh * d), np.float32)
+        q.reshape(rows, nh, d)[:, :, 3] = 1.0
+        kc = np.zeros((nkv, pos0 + rows, d), np.float16)
+        kc[:, :, 3] = -nats * (1 + rng.random(kc.shape[:2]) / 16)
+        vc = rng.uniform(0.5, 1.5, kc.shape).astype(np.float16)
+        kc[:, 1000] = vc[:, 1000] = 0.0
+        import torch
+        lib = q4.load()
+        tq, tk, tv = (torch.from_numpy(a).cuda() for a in (q, kc, vc))
+        out = torch.zeros((rows, nh * d), device="cuda")
+        rc = lib.q4_prompt_attention_dev(tq.data_ptr(), tk.data_ptr(), tv.data_ptr(), out.data_ptr(), rows, pos0, nh,
+                                         nkv, d, pos0 + rows, 1.0, torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, q4.last_error(lib)
+        err = oracle.normwise_rel(out.cpu().numpy(), sdpa_causal(q, kc, vc, pos0, nh, nkv, 1.0))
+        print(f"{nats} nats: {err:.2e}", flush=True)
+        worst = max(worst, err)
+    assert worst < ATTN_TOL + 18 * 17 / 16 * (2.0 ** -22 + 2.0 ** -23)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_prompt_attention_small_queries_large_keys(d):
+    """Queries below fp16's range against keys near its end."""
+    rng = np.random.default_rng(d)
+    q = (rng.normal(0, 1, (1, d)) * 2.0 ** -17).astype(np.float32)
+    k = (rng.uniform(-1, 1, (300, d)) * 2.0 ** 15).astype(np.float16)
+    v = rng.normal(0, 1, (300, d)).astype(np.float16)
+    assert oracle.normwise_rel(_one_head(q, k, v, 1.0), sdpa_causal(q, k[None], v[None], 299, 1, 1, 1.0)) < ATTN_TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_prompt_attention_infinite_keys(d):
+    """A key of -inf times the query's sign (an overflow of the cache) has a
+    score of -inf and is left out, whatever bits the query has there (1.5 is
+    exact in one fp16 value)."""
+    rng = np.random.default_rng(d)
+    n, scale = 200, ctypes.c_float(np.log(2)).value          # times log2(e): the kernel's q is this one
+    for value in (1.5, -1.25, 2.0 ** -13):
+        q = rng.normal(0, 1, (1, d)).astype(np.float32)
+        q[0, 5] = value
+        k = rng.normal(0, 1, (n, d)).astype(np.float16)
+        k[77, 5] = -np.inf * value
+        v = rng.normal(0, 1, (n, d)).astype(np.float16)
+        got = _one_head(q, k, v, scale)
+        assert oracle.normwise_rel(got, sdpa_causal(q, k[None], v[None], n - 1, 1, 1, scale)) < ATTN_TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_prompt_attention_scores_far_apart(d):
+    """Scores of up to 2^30, every two at least 2^18 apart: the output is the
+    value of the largest, whichever tile and group it is in, exactly."""
+    rng = np.random.default_rng(d)
+    n = 400
+    q = np.zeros((1, d), np.float32)
+    q[0, 3] = 2.0 ** 14
+    v = rng.normal(0, 1, (n, d)).astype(np.float16)
+    for sign in (1, -1):
+        for best in (3, 70, 399):
+            k = np.zeros((n, d), np.float16)
+            k[:, 3] = sign * 32768.0 - 16.0 * (2 + rng.permutation(n))
+            k[best, 3] = sign * 32768.0 - 16.0
+            np.testing.assert_array_equal(_one_head(q, k, v, 1.0)[0], v[best].astype(np.float32))
