@@ -92,11 +92,14 @@ inline int attn_max_parts(int nkv) {
 // part of max_parts (the grid's x; at most kMaxParts and a.n_chunks).
 // RUNS: the cache holds more than max_parts chunks, so a part may be a run
 // of them; without it a part is one chunk, and the loop and its rescaling
-// are not compiled in (they cost the one-chunk kernel 0.3 of 8.3 us).  G: query heads per kv
-// head, D: head_dim (32, 64 or 128; a.d), template parameters so that the
-// loops over them unroll and their LDS reads are issued together.  Called
-// by the kAttnThreads threads of the workgroup.
-template <bool ROPE, bool RUNS, int G, int D>
+// are not compiled in (they cost the one-chunk kernel 0.3 of 8.3 us).  MANY:
+// max_parts may be more than 64; without it the merge has no second (m, l) per
+// lane (0.07 of 7.4 us, a decode layer 56.6 instead of 56.75; behind a branch
+// it took 0.3 us more).  G: query heads per kv head, D: head_dim (32, 64 or
+// 128; a.d), template parameters so that the loops over them unroll and their
+// LDS reads are issued together.  Called by the kAttnThreads threads of the
+// workgroup.
+template <bool ROPE, bool RUNS, bool MANY, int G, int D>
 __device__ __forceinline__ void attn_decode(const AttnArgs& a, int part, int max_parts, int kvh, char* lds) {
     static_assert(D == 32 || D == 64 || D == 128, "head_dim 32, 64 or 128");
     constexpr int NT = kAttnThreads;
@@ -341,7 +344,7 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, int part, int max
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
     {
     // the merge of query head h: lane c takes the (m, l) of parts c and
-    // c + 64: the maximum M over all parts, the weights e^(m_c - M)
+    // (MANY) c + 64: the maximum M over all parts, the weights e^(m_c - M)
     // and the lane tree of the w_c l_c; lane i then adds w_c o_c for its
     // dimensions 2i, 2i + 1 in part order, w_c read from lane c.  The first
     // kMergeBatch parts' o and the (m, l) are loaded in one round, the
@@ -362,14 +365,14 @@ __device__ __forceinline__ void attn_decode(const AttnArgs& a, int part, int max
     float2 ob[kMergeBatch];
 #pragma unroll
     for (int c = 0; c < kMergeBatch; c++) ob[c] = ld_o(c);
-    const float2 ml0 = ld_ml(lane), ml1 = ld_ml(lane + 64);
-    const float m0 = lane < n_act ? ml0.x : -__builtin_inff(), m1 = lane + 64 < n_act ? ml1.x : -__builtin_inff();
+    const float2 ml0 = ld_ml(lane), ml1 = MANY ? ld_ml(lane + 64) : make_float2(0.0f, 0.0f);
+    const float m0 = lane < n_act ? ml0.x : kNegInf, m1 = MANY && lane + 64 < n_act ? ml1.x : kNegInf;
     const float M = wave_max(fmaxf(m0, m1));
-    auto weight = [&](float mc) { return mc != -__builtin_inff() ? expf(__fsub_rn(mc, M)) : 0.0f; };
-    const float w0 = weight(m0), w1 = weight(m1);    // lane c: the weights of parts c and c + 64
-    const float lloc = n_act > 64 ? __builtin_fmaf(ml1.y, w1, __fmul_rn(ml0.y, w0)) : __fmul_rn(ml0.y, w0);
+    auto weight = [&](float mc) { return mc != kNegInf ? expf(__fsub_rn(mc, M)) : 0.0f; };
+    const float w0 = weight(m0), w1 = MANY ? weight(m1) : 0.0f;      // lane c: the weights of parts c and c + 64
+    const float lloc = MANY && n_act > 64 ? __builtin_fmaf(ml1.y, w1, __fmul_rn(ml0.y, w0)) : __fmul_rn(ml0.y, w0);
     auto wt = [&](int c) {                           // c uniform
-        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(c < 64 ? w0 : w1), c & 63));
+        return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(!MANY || c < 64 ? w0 : w1), c & 63));
     };
     float s0 = 0.0f, s1 = 0.0f;
 #pragma unroll

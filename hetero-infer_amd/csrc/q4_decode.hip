@@ -208,18 +208,18 @@ __global__ __launch_bounds__(256) void silu_mul_kernel(const float* __restrict__
 
 // ---------------------------------------------------------- attention ---
 // attn_decode of q4_attn.h as one launch over grid (part, kv head).
-template <bool ROPE, bool RUNS, int G, int D>
+template <bool ROPE, bool RUNS, bool MANY, int G, int D>
 __global__ __launch_bounds__(kAttnThreads) void attn_decode_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(16))) char lds[kAttnLdsBytes];
-    attn_decode<ROPE, RUNS, G, D>(a, blockIdx.x, gridDim.x, blockIdx.y, lds);
+    attn_decode<ROPE, RUNS, MANY, G, D>(a, blockIdx.x, gridDim.x, blockIdx.y, lds);
 }
 
-template <bool ROPE, bool RUNS, int D>
+template <bool ROPE, bool RUNS, bool MANY, int D>
 void launch_attention_d(int G, dim3 grid, hipStream_t st, const AttnArgs& a) {
     switch (G) {
 #define Q4_ATTN_CASE(g)                                                                                      \
     case g:                                                                                                  \
-        hipLaunchKernelGGL((attn_decode_kernel<ROPE, RUNS, g, D>), grid, dim3(kAttnThreads), 0, st, a);      \
+        hipLaunchKernelGGL((attn_decode_kernel<ROPE, RUNS, MANY, g, D>), grid, dim3(kAttnThreads), 0, st, a); \
         break;
         Q4_ATTN_CASE(1) Q4_ATTN_CASE(2) Q4_ATTN_CASE(3) Q4_ATTN_CASE(4)
         Q4_ATTN_CASE(5) Q4_ATTN_CASE(6) Q4_ATTN_CASE(7) Q4_ATTN_CASE(8)
@@ -228,17 +228,24 @@ void launch_attention_d(int G, dim3 grid, hipStream_t st, const AttnArgs& a) {
     }
 }
 
+template <bool ROPE, bool RUNS, bool MANY>
+void launch_attention_parts(dim3 grid, hipStream_t st, const AttnArgs& a) {
+    const int G = a.nh / a.nkv;
+    if (a.d == 128) launch_attention_d<ROPE, RUNS, MANY, 128>(G, grid, st, a);
+    else if (a.d == 64) launch_attention_d<ROPE, RUNS, MANY, 64>(G, grid, st, a);
+    else launch_attention_d<ROPE, RUNS, MANY, 32>(G, grid, st, a);
+}
+
 // head_dim 32, 64 or 128 (the callers check); a workgroup per part and kv
 // head: a part is one chunk while the cache has no more chunks than
 // attn_max_parts, else a run of chunks (q4_attn.h)
 template <bool ROPE>
 void launch_attention(hipStream_t st, const AttnArgs& a) {
-    const int G = a.nh / a.nkv, most = attn_max_parts(a.nkv);
+    const int most = attn_max_parts(a.nkv);
     const bool runs = a.n_chunks > most;
     const dim3 grid(runs ? most : a.n_chunks, a.nkv);
-    if (a.d == 128) runs ? launch_attention_d<ROPE, true, 128>(G, grid, st, a) : launch_attention_d<ROPE, false, 128>(G, grid, st, a);
-    else if (a.d == 64) runs ? launch_attention_d<ROPE, true, 64>(G, grid, st, a) : launch_attention_d<ROPE, false, 64>(G, grid, st, a);
-    else runs ? launch_attention_d<ROPE, true, 32>(G, grid, st, a) : launch_attention_d<ROPE, false, 32>(G, grid, st, a);
+    if (grid.x > 64) runs ? launch_attention_parts<ROPE, true, true>(grid, st, a) : launch_attention_parts<ROPE, false, true>(grid, st, a);
+    else runs ? launch_attention_parts<ROPE, true, false>(grid, st, a) : launch_attention_parts<ROPE, false, false>(grid, st, a);
 }
 
 // ---------------------------------------------------------------- argmax ---

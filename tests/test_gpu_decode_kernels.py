@@ -244,6 +244,31 @@ def test_attention_parts_of_several_chunks(torch, lib, nh, nkv, d, parts):
         assert torch.equal(two, out) and torch.equal(k1, k2) and torch.equal(v1, v2), p
 
 
+@pytest.mark.parametrize("nh,nkv,d", [(8, 1, 128), (4, 2, 64), (9, 3, 32)])
+def test_attention_many_parts_of_one_chunk(torch, lib, nh, nkv, d):
+    """Up to 3 kv heads: more than 64 parts of one chunk each (85 at 3), the
+    merge with two parts' (m, l) per lane, on both sides of its 64th and at the
+    last part."""
+    rng = np.random.default_rng(nkv)
+    cap = 85 * 64
+    scale = float(np.float32(d ** -0.5))
+    dev = torch.device("cuda")
+    kc_np = rng.normal(0, 1, (nkv, cap, d)).astype(np.float16)
+    vc_np = rng.normal(0, 1, (nkv, cap, d)).astype(np.float16)
+    q_np = rng.normal(0, 1, nh * d).astype(np.float32)
+    kc, vc, tq = (torch.from_numpy(a).to(dev) for a in (kc_np, vc_np, q_np))
+    out = torch.empty(nh * d, device=dev)
+    scratch = torch.zeros(lib.q4_attention_scratch_floats(nh, d, cap), device=dev)
+    for p in (0, 2304, 4095, 4096, 4160, cap - 1):
+        pos = torch.tensor([p], dtype=torch.int64, device=dev)
+        rc = lib.q4_attention_dev(tq.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr(), out.data_ptr(),
+                                  scratch.data_ptr(), nh, nkv, d, cap, scale, sp(torch))
+        assert rc == 0, q4.last_error(lib)
+        ref = attention_ref(q_np, kc_np, vc_np, p, nh, nkv, scale)
+        assert oracle.normwise_rel(out.cpu().numpy(), ref) < ATTN_TOL, p
+        assert int(scratch[-512 * 32:].view(torch.int32).abs().sum().item()) == 0, p
+
+
 def test_attention_long_context(torch, lib):
     """Contexts past one round of the merge's loads (36 chunks of 64
     positions): up to 79 chunks, the ones past the first round merged by
