@@ -536,7 +536,9 @@ struct Workspace {
     size_t cap[7] = {0, 0, 0, 0, 0, 0, 0};      // bytes, in the order above
     bool in_graph[7] = {false, false, false, false, false, false, false};
     bool fixed = false;
-    bool prefill_reserved = false;              // part and sk once sized for every plan (prefill_workspace)
+    // (column blocks, columns, n_in; 0 columns: gate/up) -> rows up to which part
+    // and sk hold every plan (prefill_reserve)
+    std::map<std::tuple<int, int, int>, int> reserved;
     std::vector<void*> retired;
 };
 enum WsBuf { kWsPlanes, kWsXsum, kWsXscale, kWsTmp, kWsXbf, kWsPart, kWsSk };
@@ -1254,8 +1256,15 @@ bool sk_ok(int P, long tiles, long T, int cus) {
 // Q4_GEMM_PLAN="rows:<bm>:<S>" (or "dp:", 128 and 256 rows only) or "sk:<P>"
 // sets the plan instead (for tests
 // and measurement).
-// nblocks: 256-column blocks of the launch; ncols: its columns.
-int plan_prefill(int m, int nblocks, int ncols, int n_in, PrefillPlan* out) {
+// nblocks: 256-column blocks of the launch; ncols: its columns.  room, flags:
+// the bytes of partials to plan within, and whether stream-K's flags are there.
+size_t sk_part_bytes(int P) { return static_cast<size_t>(P) * 256 * 256 * 4; }
+
+size_t plan_part_bytes(const PrefillPlan& p, int m, int ncols) {
+    return p.sk_p > 0 ? sk_part_bytes(p.sk_p) : p.S > 1 ? static_cast<size_t>(p.S) * m * ncols * 4 : 0;
+}
+
+int plan_prefill(int m, int nblocks, int ncols, int n_in, PrefillPlan* out, size_t room = SIZE_MAX, bool flags = true) {
     const int cus = num_cus();
     const int G = n_in / 64;
     const long tiles256 = static_cast<long>((m + 255) / 256) * nblocks;
@@ -1289,7 +1298,7 @@ int plan_prefill(int m, int nblocks, int ncols, int n_in, PrefillPlan* out) {
         const long tiles = static_cast<long>((m + bm - 1) / bm) * nblocks;
         // (splits past two rounds only add partials)
         for (int S = 1; S <= 32 && G / S >= 2 && (S == 1 || tiles * S <= 2L * cus); S++) {
-            if (!splits_ok(S)) continue;
+            if (!splits_ok(S) || plan_part_bytes(PrefillPlan{bm, S, 0}, m, ncols) > room) continue;
             const double est = prefill_dp_us(bm, tiles * S, (G + S - 1) / S, cus) +
                                (S > 1 ? static_cast<double>(S) * m * ncols * 8.0 / 4.5e6 + 3.0 + 0.2 * S : 0.0);
             if (est < best) {
@@ -1299,7 +1308,7 @@ int plan_prefill(int m, int nblocks, int ncols, int n_in, PrefillPlan* out) {
         }
     }
     // (few tiles: every owner would add many partials)
-    for (int P = 8; P <= cus && tiles256 * 5 >= cus; P += 8) {
+    for (int P = 8; P <= cus && tiles256 * 5 >= cus && flags && sk_part_bytes(P) <= room; P += 8) {
         if (!sk_ok(P, tiles256, T, cus) || sk_groups(P, tiles256) != 8) continue;
         const long Tg = (tiles256 + 7) / 8 * G, Pg = P / 8;
         const long L = (Tg + Pg - 1) / Pg, Lmin = Tg / Pg;
@@ -1736,30 +1745,59 @@ int sk_flags(Workspace& ws, hipStream_t st) {
     return 0;
 }
 
-// Room for a prefill plan's partial sums (stream-K: 256 KiB per workgroup;
-// split-K: S M N floats) and, for stream-K, its flags.  A stream's first
-// prefill call outside a capture reserves what any plan takes -- two tiles of
-// 256 x 256 per CU, 128 MiB on 256 CUs, and the flags -- because which plan
-// and how much a call needs is not monotonic in its rows: a captured call may
-// split where the larger one run before it did not.  Where that much memory
-// is not to be had, a call takes what it needs.
-int prefill_workspace(Workspace& ws, size_t part_bytes, bool flags, hipStream_t st) {
-    if (!ws.prefill_reserved) {
-        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-        HIP_TRY(hipStreamIsCapturing(st, &cs));
-        if (cs == hipStreamCaptureStatusNone) {
-            ws.prefill_reserved = true;
-            const size_t most = static_cast<size_t>(num_cus()) * 2 * 256 * 256 * 4;
-            if (grow(ws, ws.part, kWsPart, std::max(part_bytes, most), st, "prefill") || sk_flags(ws, st))
-                (void)hipGetLastError();
-        }
+bool stream_capturing(hipStream_t st) {
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return hipStreamIsCapturing(st, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone;
+}
+
+// Partials and flags for every prefill plan of up to m rows of one shape, m
+// rounded up to a power of two (so that calls of rising sizes seldom grow them):
+// which plan and how much a call needs is not monotonic in its rows, and a
+// captured call may split where the larger one run before it did not.
+// need(r0, r1, &flags): the most that calls of r0 to r1 rows take, flags set if
+// one takes the flags; asked for steps of 16 rows up to 64 and 64 rows past them,
+// in which no tile count changes.  Where the memory is not to be had, a call
+// takes what it needs itself.  At 512 rows, hidden 3584 and intermediate 18944,
+// q/k/v, o and down take 27, 28 and 63 MiB: past 128 rows 64 MiB at once, as each
+// growth waits for the stream (0.4 ms of a stage's first prompt).  Any plan fits
+// two tiles of 256 x 256 per CU, 128 MiB on 256 CUs.
+template <class F>
+void prefill_reserve(Workspace& ws, std::tuple<int, int, int> shape, int m, hipStream_t st, F need) {
+    static std::mutex mu;                                          // of every stream's `reserved`
+    {
+        std::lock_guard<std::mutex> lock(mu);
+        const auto it = ws.reserved.find(shape);
+        if (it != ws.reserved.end() && it->second >= m) return;
     }
+    if (stream_capturing(st)) return;
+    int rows = 64;
+    while (rows < m && rows < 4096) rows *= 2;                     // (larger calls have no splits)
+    size_t most = 0;
+    bool flags = false;
+    for (int r0 = 1, step; r0 <= rows; r0 += step) {
+        step = r0 < 64 ? 16 : 64;
+        most = std::max(most, need(r0, r0 + step - 1, &flags));
+    }
+    size_t bytes = !most ? 0 : size_t{1} << (m > 128 ? 26 : 20);
+    while (bytes < most) bytes *= 2;
+    if ((bytes && grow(ws, ws.part, kWsPart, bytes, st, "prefill")) || (flags && sk_flags(ws, st)))
+        (void)hipGetLastError();
+    std::lock_guard<std::mutex> lock(mu);
+    if (ws.reserved.size() >= 256) ws.reserved.clear();
+    ws.reserved[shape] = std::max(rows, m);
+}
+
+// Room for one plan: part_bytes of partials (stream-K: 256 KiB per workgroup;
+// split-K: S M N floats) and, for stream-K, its flags.
+int prefill_workspace(Workspace& ws, size_t part_bytes, bool flags, hipStream_t st) {
     if (part_bytes)
         if (int rc = grow(ws, ws.part, kWsPart, part_bytes, st, "prefill")) return rc;
     return flags ? sk_flags(ws, st) : 0;
 }
 
-size_t sk_part_bytes(int P) { return static_cast<size_t>(P) * 256 * 256 * 4; }
+bool prefill_fits(const Workspace& ws, size_t part_bytes, bool flags) {
+    return part_bytes <= ws.cap[kWsPart] && (!flags || ws.sk);
+}
 
 // q4_gemm_bf16_multi_dev on x given in fp32 (x, rounded to bf16 into the
 // workspace first) or already in bf16 (xb).
@@ -1811,8 +1849,20 @@ int gemm_bf16_multi(int count, const uint32_t* const* w, const uint16_t* const* 
     if ((rc = plan_prefill(m, nblocks, ncols, n_in, &plan))) return rc;
     const size_t mk = static_cast<size_t>(m) * n_in, mn = static_cast<size_t>(m) * ncols;
     if (!xb_in && (rc = grow(*ws, ws->xbf, kWsXbf, mk * 2, st, "prefill"))) return rc;
-    const size_t part_bytes = plan.sk_p > 0 ? sk_part_bytes(plan.sk_p) : plan.S > 1 ? plan.S * mn * 4 : 0;
-    if ((rc = prefill_workspace(*ws, part_bytes, plan.sk_p > 0, st))) return rc;
+    const bool forced = getenv("Q4_GEMM_PLAN") != nullptr;
+    if (!forced)
+        prefill_reserve(*ws, {nblocks, ncols, n_in}, m, st, [&](int r0, int r1, bool* flags) {
+            // more rows never take more splits here (a split costs by the row)
+            PrefillPlan p0, p1;
+            if (plan_prefill(r0, nblocks, ncols, n_in, &p0) || plan_prefill(r1, nblocks, ncols, n_in, &p1)) return size_t{0};
+            *flags = *flags || p0.sk_p > 0 || p1.sk_p > 0;
+            return std::max(plan_part_bytes(p0, r1, ncols), plan_part_bytes(p1, r1, ncols));
+        });
+    // a captured call cannot grow the workspace: the best plan that fits it
+    if (!forced && !prefill_fits(*ws, plan_part_bytes(plan, m, ncols), plan.sk_p > 0) && stream_capturing(st) &&
+        (rc = plan_prefill(m, nblocks, ncols, n_in, &plan, ws->cap[kWsPart], ws->sk != nullptr)))
+        return rc;
+    if ((rc = prefill_workspace(*ws, plan_part_bytes(plan, m, ncols), plan.sk_p > 0, st))) return rc;
     const uint16_t* xb = xb_in;
     if (!xb) {
         const long n8 = static_cast<long>(mk / 8);
@@ -1891,22 +1941,24 @@ int q4_gemm_bf16in_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate
     // 172), 192 at 512 (169; 176), stream-K at 1000 (299).
     // Q4_PAIR_PLAN=dp (256 rows), rows:<bm> or sk:<P> chooses.
     const int cus = num_cus(), G = n_in / 64;
-    const long nblocks = (n_inter + 127) / 128, tiles = static_cast<long>((m + 255) / 256) * nblocks;
-    const long T = tiles * G;
-    int bm = 256, P = 0;
-    double best = 1e30;
-    for (int h : {256, 192, 128, 64}) {
-        const double est = prefill_dp_us(h, (m + h - 1) / h * nblocks, G, cus);
-        if (est < best) {
-            best = est;
-            bm = h;
+    const long nblocks = (n_inter + 127) / 128;
+    auto plan = [&](int rows, int* height) {                       // stream-K's workgroups, 0: tiles of *height rows
+        double best = 1e30;
+        for (int h : {256, 192, 128, 64}) {
+            const double est = prefill_dp_us(h, (rows + h - 1) / h * nblocks, G, cus);
+            if (est < best) {
+                best = est;
+                *height = h;
+            }
         }
-    }
-    if (tiles > cus) {
-        const int p = static_cast<int>(std::min<long>(cus >= 8 ? cus / 8 * 8 : cus, T));
-        if (1.9 * static_cast<double>(T) / p + 53.0 < best) P = p;
-    }
-    if (const char* env = getenv("Q4_PAIR_PLAN")) {
+        const long tiles = (rows + 255) / 256 * nblocks;
+        const int p = static_cast<int>(std::min<long>(cus >= 8 ? cus / 8 * 8 : cus, tiles * G));
+        return tiles > cus && 1.9 * static_cast<double>(tiles * G) / p + 53.0 < best ? p : 0;
+    };
+    int bm = 256, P = plan(m, &bm);
+    const long tiles = (m + 255) / 256 * nblocks, T = tiles * G;
+    const char* env = getenv("Q4_PAIR_PLAN");
+    if (env) {
         char tail = 0;
         int p = 0;
         if (std::strcmp(env, "dp") == 0) P = 0, bm = 256;
@@ -1915,12 +1967,21 @@ int q4_gemm_bf16in_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate
         else return fail(Q4_EARG, "Q4_PAIR_PLAN=%s: expected dp, rows:<bm> or sk:<P> with P in [1, %ld]", env,
                          std::min<long>(cus, T));
     }
-    Workspace* ws = nullptr;
-    if (P > 0 || tiles > cus) {                        // (tiles of less than 256 rows need none themselves)
-        if ((rc = stream_workspace(st, &ws))) return rc;
-        if ((rc = prefill_workspace(*ws, P > 0 ? sk_part_bytes(P) : 0, P > 0, st))) return rc;
+    if (P == 0 && (env || tiles <= cus)) return gemm_w4_pair(xb, gm, h, m, n_in, bm, st);
+    Workspace* ws;
+    if ((rc = stream_workspace(st, &ws))) return rc;
+    if (!env) {
+        prefill_reserve(*ws, {static_cast<int>(nblocks), 0, n_in}, m, st, [&](int, int r1, bool* flags) {
+            int height;
+            const int p = plan(r1, &height);
+            *flags = *flags || p > 0;
+            return p > 0 ? sk_part_bytes(p) : size_t{0};
+        });
+        // a captured call cannot grow the workspace: tiles where stream-K's is not there
+        if (P > 0 && !prefill_fits(*ws, sk_part_bytes(P), true) && stream_capturing(st)) P = 0;
+        if (P == 0) return gemm_w4_pair(xb, gm, h, m, n_in, bm, st);
     }
-    if (P == 0) return gemm_w4_pair(xb, gm, h, m, n_in, bm, st);
+    if ((rc = prefill_workspace(*ws, sk_part_bytes(P), true, st))) return rc;
     return gemm_w4_sk_pair(xb, gm, static_cast<float*>(ws->part), ws->sk, sk_ctl(*ws), h, m, n_in, P,
                            sk_groups(P, tiles), st);
 }

@@ -153,7 +153,10 @@ int q4_mlp_dev(const uint32_t *gate_w, const uint16_t *gate_s, const uint16_t *g
  * gs must be 64; w and x 16-byte aligned.  Uses a per-stream workspace (the
  * bf16 copy of x and, when K is split over workgroups, the partial sums)
  * that grows on first use: run the largest call once on a stream before
- * capturing it in a graph. */
+ * capturing it in a graph.  The partial sums are reserved for calls of up to
+ * that many rows of the shape, rounded up to a power of two (64 MiB for the
+ * layers of a 7B model at 512 rows, never more than 128); a captured call whose
+ * split finds too few takes the fastest tiling that they do hold. */
 int q4_gemm_bf16_dev(const uint32_t *w, const uint16_t *scales, const uint16_t *biases,
                      const float *x, float *out, int m, int n_out, int n_in, int gs,
                      void *stream);

@@ -294,3 +294,70 @@ def test_smaller_calls_under_capture_after_the_largest(n_out, n_in, warm):
             g.replay()
             torch.cuda.synchronize()
             assert torch.equal(out, e), m
+
+
+@pytest.mark.gpu
+def test_partials_reserved_by_the_call():
+    """A stream holds the partial sums that its calls can take, not those of
+    the largest plan there is: a 17-row call of a small matrix under 2 MiB, and
+    five streams not five times 128 MiB."""
+    import torch
+    n_out, n_in = 512, 3584
+    (tw, ts, tb, tx), exact = _operands(977, 17, n_out, n_in)
+    q4.gemm_bf16_dev(tw, ts, tb, tx)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(5)]
+    outs = [torch.empty((17, n_out), device="cuda") for _ in streams]
+    free = torch.cuda.mem_get_info()[0]
+    for s, o in zip(streams, outs):
+        q4.gemm_bf16_dev(tw, ts, tb, tx, out=o, stream=s)
+    torch.cuda.synchronize()
+    # a split of 64 rows takes at most 32 planes of 64 x 512 floats, 4 MiB, x and flags less than one more
+    assert free - torch.cuda.mem_get_info()[0] <= 5 * (6 << 20)
+    for o in outs:
+        assert oracle.normwise_rel(o.cpu().numpy(), exact) < EXACT_OPERAND_TOL
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m", [17, 300, 512])
+def test_captured_calls_without_room_for_their_plan(monkeypatch, m):
+    """A captured call of a shape that the stream has not run (bf16 x: no copy
+    of it): the tiling that fits the stream's workspace, the result within the
+    bar; the paired gate/up form, which would take stream-K at 512 rows, equal to
+    its unsplit form bit for bit."""
+    import torch
+    n_out, n_in = 18944, 5120
+    g = torch.Generator(device="cuda")
+    g.manual_seed(m)
+    mats = []
+    for _ in range(2):
+        w = torch.randint(-2 ** 31, 2 ** 31, (n_out, n_in // 8), dtype=torch.int64, device="cuda", generator=g)
+        s = (torch.randn((n_out, n_in // 64), device="cuda", generator=g) * 0.01).abs().half()
+        mats.append((w.to(torch.int32), s, (-7.5 * s.float()).half()))
+    x = torch.randn((m, n_in), device="cuda", generator=g).bfloat16()
+    small = [t[:64].contiguous() for t in mats[0]]
+    want_h = torch.empty((m, n_out), dtype=torch.bfloat16, device="cuda")
+    monkeypatch.setenv("Q4_PAIR_PLAN", "dp")
+    q4.gemm_bf16_gate_up_silu_dev(*mats, x, h=want_h)
+    monkeypatch.delenv("Q4_PAIR_PLAN")
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(stream):
+        q4.gemm_bf16_multi_dev([small], x[:1], stream=stream)      # the stream's first call, a small one
+    torch.cuda.synchronize()
+    out, h = torch.empty((m, 512), device="cuda"), torch.zeros_like(want_h)
+    part = [t[:512].contiguous() for t in mats[0]]
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        q4.gemm_bf16_multi_dev([part], x, outs=[out], stream=stream)
+        q4.gemm_bf16_gate_up_silu_dev(*mats, x, h=h, stream=stream)
+    eager = q4.gemm_bf16_multi_dev([part], x)[0]
+    for _ in range(2):
+        out.fill_(float("nan"))
+        h.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert oracle.normwise_rel(out.cpu().numpy(), eager.cpu().numpy()) < 2 * EXACT_OPERAND_TOL
+        assert torch.equal(h, want_h)
+    assert q4.prefill_errors() == 0
