@@ -113,11 +113,12 @@ def test_gate_up_silu_epilogue_equals_separate_calls(torch, lib, monkeypatch, m,
     assert torch.equal(_bits(got), _bits(again))
 
 
-# the default plan of a 512-token prompt (296 tiles: stream-K over the
-# CUs), and forced stream-K plans on small shapes: 8 and 5 workgroups
-# (fewer than the tiles: ranges of several tiles), 64 (more than the
-# tiles: several partials per tile), 3 over a single tile row
-@pytest.mark.parametrize("m,n_inter,n_in,plan", [(512, 18944, 3584, None), (300, 1000, 1024, "sk:8"),
+# forced stream-K plans: 296 tiles of a 512-token prompt over 256 workgroups
+# in 8 groups (the launch of the default plan at wider n_in, below), and on
+# small shapes 8 and 5 workgroups (fewer than the tiles: ranges of several
+# tiles), 64 (more than the tiles: several partials per tile), 3 over a
+# single tile row
+@pytest.mark.parametrize("m,n_inter,n_in,plan", [(512, 18944, 3584, "sk:256"), (300, 1000, 1024, "sk:8"),
                                                  (300, 1000, 1024, "sk:5"), (300, 1000, 1024, "sk:64"),
                                                  (37, 200, 512, "sk:3")])
 def test_gate_up_silu_stream_k(torch, lib, monkeypatch, m, n_inter, n_in, plan):
@@ -154,6 +155,27 @@ def test_gate_up_silu_stream_k(torch, lib, monkeypatch, m, n_inter, n_in, plan):
     err = oracle.normwise_rel(got.float().cpu().numpy(), ref)
     print(f"normwise error vs float64: {err:.2e}", flush=True)
     assert err < 8e-3                             # bf16 output rounding, 2^-8 relative at most
+
+
+def test_gate_up_silu_default_plan(torch, lib, monkeypatch):
+    """The plan of the call itself, told apart by its bits: tiles of one
+    workgroup each at n_in 3584 (512 and 1000 rows), stream-K over every CU at
+    5120, where its fixed cost weighs less."""
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("plans of 256 CUs")
+    for m, n_in, stream_k in ((512, 3584, False), (1000, 3584, False), (512, 5120, True)):
+        print(f"default plan m={m} k={n_in}", flush=True)
+        gate, up = _mats(torch, 950, (18944, 18944), n_in)
+        xb = torch.from_numpy(synth.activations(951 + m, m, n_in)).cuda().to(torch.bfloat16)
+        h = {}
+        for plan in (None, "dp", "sk:256"):
+            _pair_plan(monkeypatch, plan)
+            h[plan] = _bits(q4.gemm_bf16_gate_up_silu_dev(gate, up, xb))
+        _pair_plan(monkeypatch, None)
+        torch.cuda.synchronize()
+        assert lib.q4_prefill_errors(_sp(torch)) == 0
+        assert not torch.equal(h["dp"], h["sk:256"])
+        assert torch.equal(h[None], h["sk:256" if stream_k else "dp"]), (m, n_in)
 
 
 def test_gate_up_silu_argument_errors(torch, lib):
