@@ -178,13 +178,16 @@ __device__ __forceinline__ void pa_split(float x, _Float16& hi, _Float16& lo) {
 
 // Two values of p, times 2^15, as hi + lo: hi the nearest fp16 value, lo the
 // rest.  (Vector conversions: the packed one, where a product converted alone
-// becomes a half-register write of its own.)
+// becomes a half-register write of its own; opaque, so that lo is the rest of
+// the very value that the MFMA takes and not of a second conversion.)
 constexpr float kPScale = 32768.0f;
 constexpr float kPDrop = 32.0f;                    // see the softmax of a tile
 typedef float pa_f2 __attribute__((ext_vector_type(2)));
 typedef _Float16 pa_h2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ void pa_split_p(const float (&x)[2], pa_h2& hi, pa_h2& lo) {
-    hi = __builtin_convertvector((pa_f2{x[0], x[1]}), pa_h2);
+    uint32_t h = __builtin_bit_cast(uint32_t, __builtin_convertvector((pa_f2{x[0], x[1]}), pa_h2));
+    asm("" : "+v"(h));
+    hi = __builtin_bit_cast(pa_h2, h);
     lo = __builtin_convertvector(
         (pa_f2{__fsub_rn(x[0], static_cast<float>(hi[0])), __fsub_rn(x[1], static_cast<float>(hi[1]))}), pa_h2);
 }
