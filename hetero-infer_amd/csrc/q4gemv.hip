@@ -1936,9 +1936,11 @@ int q4_gemm_bf16in_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate
     // estimated time, or past one round of 256-row tiles stream-K over one
     // workgroup per CU, so that a last partial round does not double the time
     // (about 1.9 us a step and 53 us of partials, restarts and imbalance).
-    // n_inter 18944, n_in 3584: 64 rows up to 64 (50 us; 256 rows take 84),
-    // 128 up to 128 (57), 256 up to 256 (90), 128 up to 384 (138; stream-K
-    // 172), 192 at 512 (169; 176), stream-K at 1000 (299).
+    // Measured, n_inter 18944, n_in 3584: 64 rows up to 64 (50 us; 256 rows take
+    // 84), 128 up to 128 (57), 256 up to 256 (90), 128 at 300 (126; stream-K 167),
+    // 192 at 512 (168; 176), 256 at 600 (204; 227) and 1000 (295; 300): stream-K
+    // at no row count up to 1536.  n_in 5120, whose steps weigh more: stream-K at
+    // 512 (223; 192 rows 236) and 1000 (414; 256 rows 414).
     // Q4_PAIR_PLAN=dp (256 rows), rows:<bm> or sk:<P> chooses.
     const int cus = num_cus(), G = n_in / 64;
     const long nblocks = (n_inter + 127) / 128;

@@ -191,14 +191,14 @@ int q4_gemm_bf16in_multi_dev(int count, const uint32_t *const *w, const uint16_t
  * each tile holds the same 128 rows of both matrices, so the SiLU * mul is
  * the GEMM's epilogue.  With a tile per workgroup the fp32 sums are those of
  * q4_gemm_bf16in_multi_dev on {gate, up} without split-K (bit for bit,
- * whatever the tile's height); where many rows would leave a last partial
- * round of tiles (past about 600 rows at n_inter 18944) the tiles'
- * K steps are shared out stream-K over one workgroup per CU and a tile's
- * partial sums are added in a fixed order, which may move a value by one
- * bf16 unit.  Q4_PAIR_PLAN=dp, rows:<bm> or sk:<P> forces a form.  gs must be
+ * whatever the tile's height).  Where a last partial round of tiles would
+ * cost more (512 rows of n_inter 18944 at n_in 5120; at n_in 3584 no count up
+ * to 1536) the tiles' K steps are shared out stream-K over one workgroup per
+ * CU and a tile's partial sums are added in a fixed order, which may move a
+ * value by one bf16 unit.  Q4_PAIR_PLAN=dp, rows:<bm> or sk:<P> forces a form.  gs must be
  * 64; w and x 16-byte aligned.  The stream-K form uses the calling
  * stream's workspace, which grows on first use (run the largest call once
- * before capturing it in a graph). */
+ * before capturing it in a graph; a captured call without it runs the tiles). */
 int q4_gemm_bf16in_gate_up_silu_dev(const uint32_t *gate_w, const uint16_t *gate_s, const uint16_t *gate_b,
                                     const uint32_t *up_w, const uint16_t *up_s, const uint16_t *up_b,
                                     const uint16_t *xb, uint16_t *h, int m, int n_inter, int n_in, int gs,
