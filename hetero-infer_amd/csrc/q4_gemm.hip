@@ -24,9 +24,10 @@
 // swizzle, byte selects in the dequant and the next step's operands read under
 // the last slice, in 4 waves of 64 columns): gate/up + down of a prompt chunk
 // 308 -> 270 us, down 111 -> 94, o 45 -> 37, 1000 rows 546 -> 446; one 256-row
-// tile per CU over K = 18944 took 2.02 us a step, 1064 TFLOP/s (MFMAs and
-// barriers alone 1.52: the clock drops as the CUs fill).  8 waves of 32
-// columns: a lone tile's step 1.50 -> 1.31 us at 256 rows, 1.25 -> 1.09 at 192.
+// tile per CU over K = 18944 took 2.02 us a step (MFMAs and barriers alone 1.52:
+// the clock drops as the CUs fill).  8 waves of 32
+// columns (the present form): a lone tile's step 1.50 -> 1.31 us at 256 rows,
+// 1.25 -> 1.09 at 192; with a tile on every CU 2.0 to 2.2 (988 TFLOP/s at 2.17).
 // B is dequantised in registers right before the MFMA that consumes it:
 // one packed word (word ks + 4 (lane/32) of the row: a lane's four words of
 // a step are one 16-byte read) is exactly one lane's 8-value B fragment of K

@@ -308,11 +308,11 @@ def test_one_row_five_item_ring(lib, gs):
 
 
 def test_matrix_core_tile_variants(lib):
-    """3..8 rows on the matrix cores, bit-exact vs the oracle, for the
-    variants the Qwen shapes leave out: group counts not a multiple of 8
-    (per-group scale/bias loads; 13 and 44 groups), 16-row tiles with a
-    partial last tile (N = 300), 32-row tiles of 8 waves (N = 9000) and of 4
-    waves (N = 16400, a partial last tile)."""
+    """3..8 rows on the matrix cores, bit-exact vs the oracle, at what the
+    Qwen shapes leave out: group counts that are odd (13: scales and biases
+    copied one group at a time) and not a multiple of a 16-group window (8, 13
+    and 44), a partial last 16-row tile (N = 300, 9000), fewer tiles than CUs
+    (N = 48) and several per workgroup (N = 9000, 16400)."""
     import torch
     o = oracle.Oracle()
     for k_in, n_out in ((832, 300), (2816, 48), (512, 9000), (832, 16400)):
@@ -330,8 +330,8 @@ def test_matrix_core_tile_variants(lib):
 def test_matrix_core_group_count_bounds(lib):
     """The matrix-core path at one group (K = 64: a window holds a single
     group, every other group slot past the end) and at 64 and 65 groups
-    (K = 4096, 4160), for 16-row and 32-row tiles, with rows past M zero in
-    the prepared x.  Bit-exact vs the oracle."""
+    (K = 4096, 4160), with one tile per workgroup and several, rows past M
+    zero in the prepared x.  Bit-exact vs the oracle."""
     import torch
     o = oracle.Oracle()
     for k_in, n_out in ((64, 40), (4096, 3584), (4096, 9000), (4160, 200)):
