@@ -35,7 +35,7 @@ struct PromptAttnArgs {
 
 // ---------------------------------------------------------------------
 // On the matrix cores (v_mfma_f32_16x16x32_f16).  A workgroup takes one kv
-// head, 16 consecutive query rows and up to 4 of the kv head's query heads,
+// head, 16 consecutive query rows and 2 or 4 of the kv head's query heads,
 // in KS groups of one wave per head: group k walks the tiles k, k + KS, ...
 // of 64 positions, its tile's K rows (k_s, row-major) and V rows (vt_s,
 // transposed: [dim][pos]) staged in LDS once for its heads, the next tile's
@@ -65,10 +65,12 @@ struct PromptAttnArgs {
 // thousands of small p to make the output: from p below the running maximum,
 // unscaled and so to 2^-25, 6e-5 of them was lost 10 nats below that key and
 // 0.19 at 18; now 2e-6, as with fp32 probabilities, in the same time (45 us
-// against 46 for the case below).
+// against 46 for the case below; 3 to 4 % more at head_dim 64).
 // q is multiplied by scale * log2(e) first and the softmax taken with exp2,
 // which is exp of the scaled score.  Workgroups of the last rows, which see
-// the most positions, are launched first.
+// the most positions, are launched first, over all kv heads (block rows are the
+// grid's slowest dimension): with heads the slowest, the last heads' longest rows
+// made a second round as long as the first (700 rows, 28 heads 26 -> 20 us).
 //
 // Bound by the matrix and vector ALUs of the few waves there are: 16 rows of
 // 28 heads are 28 waves, 512 rows 896, so the groups put two waves on every
@@ -202,7 +204,7 @@ __device__ __forceinline__ float pa_rows4(float x, F f) {
 }
 
 template <int HPW, int KS, int D, bool BF>
-__global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(HPW == 1 ? 1 : 2, 2))) void prompt_attn_kernel(PromptAttnArgs a) {
+__global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(2, 2))) void prompt_attn_kernel(PromptAttnArgs a) {
     constexpr int NT = 64 * HPW, KT = D / 32, DT = D / 16;
     using S = PaShape<D, NT>;
     // a wave's maximum, sum and outputs, when the groups are merged
@@ -215,10 +217,12 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
     const int kg = wave / HPW;                                  // the wave's group
     const int tid = threadIdx.x - kg * NT;                      // thread of the group
     const int G = a.nh / a.nkv;
-    const int h = blockIdx.z * HPW + wave % HPW;                // query head of the kv head
+    // (7 heads are 4 and 3: an XCD, workgroups modulo 8, gets some of each)
+    const int part = gridDim.y == 2 ? blockIdx.y ^ (blockIdx.z & 1) : blockIdx.y;
+    const int h = part * HPW + wave % HPW;                // query head of the kv head
     const int c = lane & 15, qd = lane >> 4;
-    const int kvh = blockIdx.y;
-    const int r0 = (static_cast<int>(gridDim.x) - 1 - static_cast<int>(blockIdx.x)) * kMRows;
+    const int kvh = blockIdx.x;
+    const int r0 = (static_cast<int>(gridDim.z) - 1 - static_cast<int>(blockIdx.z)) * kMRows;
     const int last_row = (r0 + kMRows < a.rows ? r0 + kMRows : a.rows) - 1;
     const int64_t wg_last = a.pos0 + last_row;
     const int r = r0 + c;                                      // lane's query row
@@ -387,7 +391,7 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
     l = pa_rows4(l, [](float x, float y) { return __fadd_rn(x, y); });
 
     // merge the groups: group 0 rescales every part to the common maximum
-    if (n_tiles > 1) {
+    if (KS > 1 && n_tiles > 1) {
         __syncthreads();                                           // the last tiles are read
         float* parts = reinterpret_cast<float*>(lds);
         if (kg > 0) {
@@ -436,29 +440,57 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(H
     }
 }
 
-template <int HPW, int D>
-void launch_prompt(const PromptAttnArgs& a, bool bf, hipStream_t st) {
-    constexpr int KS = HPW <= 2 ? 4 : 2;                       // 4 to 8 waves: two per SIMD, 256 registers each
-    const dim3 grid((a.rows + kMRows - 1) / kMRows, a.nkv, (a.nh / a.nkv + HPW - 1) / HPW);
-    if (bf) hipLaunchKernelGGL((prompt_attn_kernel<HPW, KS, D, true>), grid, dim3(64 * HPW * KS), 0, st, a);
-    else hipLaunchKernelGGL((prompt_attn_kernel<HPW, KS, D, false>), grid, dim3(64 * HPW * KS), 0, st, a);
+template <int HPW, int KS, int D>
+void launch_prompt(PromptAttnArgs a, bool bf, hipStream_t st) {
+    constexpr int kMost = 65535 * kMRows;                      // the grid's z
+    const int parts = (a.nh / a.nkv + HPW - 1) / HPW;
+    for (int left = a.rows; left > 0; left -= a.rows) {
+        a.rows = left < kMost ? left : kMost;
+        const dim3 grid(a.nkv, parts, (a.rows + kMRows - 1) / kMRows);
+        if (bf) hipLaunchKernelGGL((prompt_attn_kernel<HPW, KS, D, true>), grid, dim3(64 * HPW * KS), 0, st, a);
+        else hipLaunchKernelGGL((prompt_attn_kernel<HPW, KS, D, false>), grid, dim3(64 * HPW * KS), 0, st, a);
+        const size_t at = static_cast<size_t>(a.rows) * a.nh * D;
+        a.q += at;
+        a.out = static_cast<char*>(a.out) + at * (bf ? 2 : 4);
+        a.pos0 += a.rows;
+    }
 }
 
-// Query heads per workgroup: pairs (in four groups, a quarter of the tiles
-// each) while those workgroups fit the chip at one per CU, else the fewest
-// workgroups of at most 4 heads, as even as they come (in two groups), which
-// read each K and V operand for more heads.  Pairs / fours, 28 heads of 4 kv
-// heads: 17 rows after 4000 positions 57 / 75 us, 100 after 2000 37 / 43, 256
-// after 1000 (256 workgroups of pairs) 25 / 29, 300 after 3000 (304) 94 / 60,
-// 512 after 1536 69 / 45.
+// Query heads per workgroup and groups of waves, by the tiles of the last row
+// and the workgroups per CU (us at head_dim 128; a wave without a head still
+// stages its share of the tiles).
+// Pairs of heads while those workgroups fit the chip at one per CU, and always
+// for 1 or 2 heads per kv head: a group per tile up to two tiles, four groups
+// from seven on (17 rows of 28 heads: 1 tile 6.9 / 7.4 / 8.6 us with 1 / 2 / 4
+// groups, 2 tiles 8.8 / 8.0 / 9.9, 6 tiles 2 groups 12.1 and 4 12.9, 8 tiles 13.7
+// and 13.2, 63 tiles 69 and 56).  1 or 2 heads and up to three tiles: fours, the
+// extra waves staging (one head, 1 tile 5.7 against 6.2 us, 3 tiles 8.4 against
+// 9.0).  1 or 2 heads past one pair per CU: what a CU holds two workgroups of,
+// pairs in two groups (700 rows, 8 heads 17.1 us; one per CU in four groups
+// 19.9) or, at head_dim 128 past 16 tiles or from two pairs per CU on, fours (700
+// after 1000 positions 42.1 against 46.3; 1500 39.0 against 51.3).
+// Else fours, which read each K and V operand for more heads (300 rows after
+// 3000, 28 heads 94 -> 60 us, 512 after 1536 69 -> 43): two groups; one, two
+// workgroups per CU, for up to three tiles, or past one workgroup per CU for up
+// to eight tiles (300 rows, 64 heads of 8 kv heads 15.3 against 16.4 us) or from
+// two per CU on (700 rows 30.4 against 38.6; with fewer and more tiles the other
+// way, 700 rows of 32 heads 24.6 against 21.4).
 template <int D>
 void launch_prompt_heads(const PromptAttnArgs& a, bool bf, hipStream_t st) {
-    const int G = a.nh / a.nkv, parts = (G + 3) / 4;
+    const int G = a.nh / a.nkv, cus = num_cus();
+    const int64_t tiles = (a.pos0 + a.rows - 1) / kPTile + 1;
     const int64_t blocks = static_cast<int64_t>((a.rows + kMRows - 1) / kMRows) * a.nkv;
-    if (G == 1) return launch_prompt<1, D>(a, bf, st);
-    if (G == 2 || blocks * ((G + 1) / 2) <= num_cus()) return launch_prompt<2, D>(a, bf, st);
-    if ((G + parts - 1) / parts == 3) return launch_prompt<3, D>(a, bf, st);
-    return launch_prompt<4, D>(a, bf, st);
+    const bool fit = blocks * ((G + 1) / 2) <= cus;
+    if (G <= 2 && tiles <= 3) return launch_prompt<4, 1, D>(a, bf, st);
+    if (G <= 2 || fit) {
+        if (!fit && D == 128 && (tiles > 16 || blocks >= 2 * cus)) return launch_prompt<4, 1, D>(a, bf, st);
+        if (tiles == 1) return launch_prompt<2, 1, D>(a, bf, st);
+        if (tiles <= 6 || !fit) return launch_prompt<2, 2, D>(a, bf, st);
+        return launch_prompt<2, 4, D>(a, bf, st);
+    }
+    const int64_t wgs = blocks * ((G + 3) / 4);
+    if (tiles <= 3 || (wgs > cus && tiles <= 8) || wgs >= 2 * cus) return launch_prompt<4, 1, D>(a, bf, st);
+    return launch_prompt<4, 2, D>(a, bf, st);
 }
 
 int launch_failed(const char* what) {

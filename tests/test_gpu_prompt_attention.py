@@ -96,16 +96,19 @@ def test_planted_mistakes_exceed_the_bar():
 
 
 # The tiles of a row block go to 2 or 4 groups of waves and its heads to
-# workgroups of 1 to 4: fewer tiles than groups, a last round of some groups
+# workgroups of 2 or 4: fewer tiles than groups, a last round of some groups
 # only, rows that see none of a group's positions, heads that leave a
-# workgroup's last waves idle, few and many workgroups (pairs of heads while
-# they fit the 256 CUs).  The bar is the one above: the groups' sums are
+# workgroup's last waves idle, few and many workgroups; and every form that
+# launch_prompt_heads picks by tiles, heads and workgroups per CU (256).  The bar is the one above: the groups' sums are
 # merged by one more rescaling, 2 fp32 roundings against the up to 40 of the
 # tiles' running ones.
 @pytest.mark.gpu
 @pytest.mark.parametrize("nh,nkv,d,rows,pos0", [
     (7, 1, 128, 5, 62), (7, 1, 64, 16, 112), (5, 1, 128, 20, 250), (10, 2, 64, 700, 0), (12, 2, 32, 700, 60),
-    (28, 4, 128, 330, 15), (16, 8, 64, 17, 600), (3, 3, 128, 40, 127), (24, 3, 64, 48, 300), (15, 5, 128, 2, 2500)],
+    (28, 4, 128, 330, 15), (16, 8, 64, 17, 600), (3, 3, 128, 40, 127), (24, 3, 64, 48, 300), (15, 5, 128, 2, 2500),
+    (28, 4, 128, 37, 0), (8, 4, 128, 17, 110), (4, 4, 64, 30, 120), (4, 4, 32, 30, 270), (6, 3, 128, 40, 330),
+    (5, 5, 64, 17, 500), (8, 8, 64, 520, 0), (16, 8, 128, 520, 0), (8, 8, 128, 530, 800), (8, 8, 32, 540, 1600), (64, 8, 128, 300, 0),
+    (64, 8, 64, 512, 100), (9, 3, 32, 700, 0), (15, 3, 64, 600, 0), (8, 1, 128, 16, 0)],
     ids=lambda v: str(v))
 def test_prompt_attention_groups_and_heads(nh, nkv, d, rows, pos0):
     import torch
