@@ -201,9 +201,12 @@ constexpr int mf_wait_copies(int n) {                            // s_waitcnt vm
 
 // Sizes of an instance.  EVEN: an even group count and 4-byte aligned scales
 // and biases, copied two groups at a time; else one at a time, zero-extended.
-// The ring's depth hardly matters (2, 4 and 8 windows within 2 %: the copies
-// and the compute of a window set the pace, not the weights), so it is kept
-// short: every slot is a copy of the loop's code.
+// The ring's depth hardly matters to a long K (the copies and the compute of a
+// window set the pace, not the weights), and every slot is a copy of the
+// loop's code, which runs cold in a short call: 3 rows, prep included, with 4
+// and 2 windows 9.2 and 8.3 us at 896 -> 200, 11.0 and 9.4 at 896 -> 4864, 19.0
+// and 17.8 at 3584 -> 18944, 18.0 and 17.4 at 18944 -> 3584 (the form before the
+// wave jobs: 8.0, 10.4, 20.1, 24.3).
 constexpr int kMfWaves = 8;                                       // compute waves
 template <bool PAIR, int MB, bool EVEN>
 struct MfShape {
@@ -211,7 +214,7 @@ struct MfShape {
     static constexpr int win = 2 * kMfWaves;                      // groups per window
     static constexpr int chain = MB / 4;                          // chain waves: 16 MB lanes
     static constexpr int threads = 64 * (kMfWaves + chain + 2);
-    static constexpr int depth = PAIR && MB == 16 ? 2 : 4;        // windows of weights in a wave's ring (128 VGPRs)
+    static constexpr int depth = 2;                               // windows of weights in a wave's ring
     static constexpr int xslots = PAIR && MB == 16 ? 2 : 3;       // windows of x in LDS (160 KB)
     static constexpr int sbslots = PAIR && MB == 16 ? 6 : 8;      // and of scales and biases
     static constexpr int xbytes = win * MB * 128;                 // x operand of a window
