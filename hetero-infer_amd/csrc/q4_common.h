@@ -273,6 +273,10 @@ struct GemmMats {
     int count;
 };
 
+// Groups of scales and biases that a copy of the prefill GEMM takes: 8, 2 or 1,
+// by the group count and the matrices' alignment.
+int w4_groups(const GemmMats& gm, int K);
+
 // The prefill GEMM (q4_gemm.hip), data-parallel: tiles of height bm (256, 192,
 // 128 or 64) over every block of gm, S splits of kt_split K steps.  part null:
 // each matrix's output directly; else split z into part + z M ldp at the

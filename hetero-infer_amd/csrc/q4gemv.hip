@@ -536,9 +536,9 @@ struct Workspace {
     size_t cap[7] = {0, 0, 0, 0, 0, 0, 0};      // bytes, in the order above
     bool in_graph[7] = {false, false, false, false, false, false, false};
     bool fixed = false;
-    // (column blocks, columns, n_in; 0 columns: gate/up) -> rows up to which part
-    // and sk hold every plan (prefill_reserve)
-    std::map<std::tuple<int, int, int>, int> reserved;
+    // (column blocks, columns, n_in, groups a copy; 0 columns: gate/up) -> rows up
+    // to which part and sk hold every plan (prefill_reserve)
+    std::map<std::tuple<int, int, int, int>, int> reserved;
     std::vector<void*> retired;
 };
 enum WsBuf { kWsPlanes, kWsXsum, kWsXscale, kWsTmp, kWsXbf, kWsPart, kWsSk };
@@ -1221,18 +1221,42 @@ struct PrefillPlan {
     int bm = 256, S = 1, sk_p = 0, sk_nx = 1;
 };
 
+// Extra us of a K step in a tile of bm rows whose scales and biases are copied
+// 2 groups or 1 group at a time (sg; w4_groups) instead of 8: those copies'
+// requests, more under the longer steps of high tiles, and with 1 the more the
+// longer the rows of G groups are.
+double prefill_copy_us(int bm, int sg, int G) {
+    const double e = sg == 8 ? 0.0 : sg == 2 ? 0.13 : 0.003 * std::min(G, 150);
+    return e * (bm == 64 ? 1.0 : bm == 128 ? 0.85 : bm == 192 ? 0.5 : 0.35);
+}
+
 // Estimated us of wgs data-parallel workgroups of kts K steps each, from
-// timings over 17 to 1000 rows (K 3584 and 18944, N 3584 to 18944): a step of
-// a lone tile takes 0.77 / 0.89 / 1.09 / 1.31 us at 64 / 128 / 192 / 256
-// rows (dequantising the tile's 256 columns and the copies are most of the
-// low ones), up to 35 % more as the CUs fill (the clock drops), and a round
-// 3 us of pipeline fill and stores.  One workgroup per CU, two of 64 rows
-// (72 KiB of LDS), which then take up to 75 % longer.
-double prefill_dp_us(int bm, long wgs, int kts, int cus) {
-    const double t0 = bm == 64 ? 0.77 : bm == 128 ? 0.89 : bm == 192 ? 1.09 : 1.31, grow = bm == 64 ? 0.75 : 0.35;
-    const long cap = static_cast<long>(cus) * (bm == 64 ? 2 : 1), full = wgs / cap, rest = wgs % cap;
-    const double us = full * (kts * t0 * (1.0 + grow) + 3.0);
-    return rest ? us + kts * t0 * (1.0 + grow * static_cast<double>(rest) / cap) + 3.0 : us;
+// timings over 17 to 1000 rows (K 832 to 18944, N 896 to 25724): a step of a
+// lone tile takes 0.77 / 0.89 / 1.09 / 1.31 us at 64 / 128 / 192 / 256 rows
+// (dequantising the tile's 256 columns and the copies are most of the low
+// ones), up to 35 % more (64 rows: 26) as the CUs fill (the clock drops), and a
+// round 3 us of pipeline fill and stores.  One workgroup per CU; two of 64 rows
+// (60 to 72 KiB of LDS), whose step is that of a CU with two as soon as some
+// have two: 1.36 to 1.76 us as the others get theirs, and up to 2.8 and 3.5 us
+// with copies of 2 and 1 groups, whose requests then are the bound (434 rows of 3392
+// -> 8768, 53 groups: 483 workgroups of 64 rows 185 us, 207 of 192 rows 80).
+// Against the fastest plan of 134 shapes the ones picked take 0.4 % more on
+// average and 11 % at most (without the copies and the second workgroup 9 % and
+// 131 %).
+double prefill_dp_us(int bm, long wgs, int kts, int cus, int sg, int G) {
+    const double t0 = bm == 64 ? 0.77 : bm == 128 ? 0.89 : bm == 192 ? 1.09 : 1.31, extra = prefill_copy_us(bm, sg, G);
+    if (bm == 64) {
+        const long full = wgs / (2L * cus), rest = wgs % (2L * cus);
+        const double us = full * (kts * (sg == 8 ? 1.5 : sg == 2 ? 2.6 : 3.4) + 3.0);   // (rounds overlap)
+        if (!rest) return us;
+        const double u = static_cast<double>(rest) / cus;
+        const double step = u <= 1.0 ? t0 * (1.0 + 0.26 * u) + extra
+                            : sg == 8 ? 1.36 + 0.4 * (u - 1.0) : sg == 2 ? 1.45 + 1.35 * (u - 1.0) : 1.5 + 0.0032 * G + 1.9 * (u - 1.0);
+        return us + kts * step + 3.0;
+    }
+    const long full = wgs / cus, rest = wgs % cus;
+    const double us = full * (kts * (t0 * 1.35 + extra) + 3.0);
+    return rest ? us + kts * (t0 * (1.0 + 0.35 * static_cast<double>(rest) / cus) + extra) + 3.0 : us;
 }
 
 // XCD groups of a stream-K launch of P workgroups over `tiles` tiles: one per
@@ -1256,15 +1280,17 @@ bool sk_ok(int P, long tiles, long T, int cus) {
 // Q4_GEMM_PLAN="rows:<bm>:<S>" (or "dp:", 128 and 256 rows only) or "sk:<P>"
 // sets the plan instead (for tests
 // and measurement).
-// nblocks: 256-column blocks of the launch; ncols: its columns.  room, flags:
-// the bytes of partials to plan within, and whether stream-K's flags are there.
+// nblocks: 256-column blocks of the launch; ncols: its columns; sg: groups a
+// copy of scales takes (w4_groups).  room, flags: the bytes of partials to plan
+// within, and whether stream-K's flags are there.
 size_t sk_part_bytes(int P) { return static_cast<size_t>(P) * 256 * 256 * 4; }
 
 size_t plan_part_bytes(const PrefillPlan& p, int m, int ncols) {
     return p.sk_p > 0 ? sk_part_bytes(p.sk_p) : p.S > 1 ? static_cast<size_t>(p.S) * m * ncols * 4 : 0;
 }
 
-int plan_prefill(int m, int nblocks, int ncols, int n_in, PrefillPlan* out, size_t room = SIZE_MAX, bool flags = true) {
+int plan_prefill(int m, int nblocks, int ncols, int n_in, int sg, PrefillPlan* out, size_t room = SIZE_MAX,
+                 bool flags = true) {
     const int cus = num_cus();
     const int G = n_in / 64;
     const long tiles256 = static_cast<long>((m + 255) / 256) * nblocks;
@@ -1299,8 +1325,8 @@ int plan_prefill(int m, int nblocks, int ncols, int n_in, PrefillPlan* out, size
         // (splits past two rounds only add partials)
         for (int S = 1; S <= 32 && G / S >= 2 && (S == 1 || tiles * S <= 2L * cus); S++) {
             if (!splits_ok(S) || plan_part_bytes(PrefillPlan{bm, S, 0}, m, ncols) > room) continue;
-            const double est = prefill_dp_us(bm, tiles * S, (G + S - 1) / S, cus) +
-                               (S > 1 ? static_cast<double>(S) * m * ncols * 8.0 / 4.5e6 + 3.0 + 0.2 * S : 0.0);
+            const double est = prefill_dp_us(bm, tiles * S, (G + S - 1) / S, cus, sg, G) +
+                               (S > 1 ? static_cast<double>(S) * m * ncols * 8.0 / 4.5e6 + 3.5 + 0.2 * S : 0.0);
             if (est < best) {
                 best = est;
                 best_plan = PrefillPlan{bm, S, 0};
@@ -1313,7 +1339,7 @@ int plan_prefill(int m, int nblocks, int ncols, int n_in, PrefillPlan* out, size
         const long Tg = (tiles256 + 7) / 8 * G, Pg = P / 8;
         const long L = (Tg + Pg - 1) / Pg, Lmin = Tg / Pg;
         const long partials = (G + Lmin - 1) / Lmin - 1;            // per owner, at most
-        const double est = static_cast<double>(L + 4) * 1.7 + static_cast<double>(partials) * 5.0 + 28.0;
+        const double est = static_cast<double>(L + 4) * (1.7 + prefill_copy_us(256, sg, G)) + static_cast<double>(partials) * 5.0 + 28.0;
         if (est < best) {
             best = est;
             best_plan = PrefillPlan{256, 1, P, 8};
@@ -1762,7 +1788,7 @@ bool stream_capturing(hipStream_t st) {
 // growth waits for the stream (0.4 ms of a stage's first prompt).  Any plan fits
 // two tiles of 256 x 256 per CU, 128 MiB on 256 CUs.
 template <class F>
-void prefill_reserve(Workspace& ws, std::tuple<int, int, int> shape, int m, hipStream_t st, F need) {
+void prefill_reserve(Workspace& ws, std::tuple<int, int, int, int> shape, int m, hipStream_t st, F need) {
     static std::mutex mu;                                          // of every stream's `reserved`
     {
         std::lock_guard<std::mutex> lock(mu);
@@ -1846,21 +1872,22 @@ int gemm_bf16_multi(int count, const uint32_t* const* w, const uint16_t* const* 
     Workspace* ws;
     if ((rc = stream_workspace(st, &ws))) return rc;
     PrefillPlan plan;
-    if ((rc = plan_prefill(m, nblocks, ncols, n_in, &plan))) return rc;
+    const int sg = w4_groups(gm, n_in);
+    if ((rc = plan_prefill(m, nblocks, ncols, n_in, sg, &plan))) return rc;
     const size_t mk = static_cast<size_t>(m) * n_in, mn = static_cast<size_t>(m) * ncols;
     if (!xb_in && (rc = grow(*ws, ws->xbf, kWsXbf, mk * 2, st, "prefill"))) return rc;
     const bool forced = getenv("Q4_GEMM_PLAN") != nullptr;
     if (!forced)
-        prefill_reserve(*ws, {nblocks, ncols, n_in}, m, st, [&](int r0, int r1, bool* flags) {
+        prefill_reserve(*ws, {nblocks, ncols, n_in, sg}, m, st, [&](int r0, int r1, bool* flags) {
             // more rows never take more splits here (a split costs by the row)
             PrefillPlan p0, p1;
-            if (plan_prefill(r0, nblocks, ncols, n_in, &p0) || plan_prefill(r1, nblocks, ncols, n_in, &p1)) return size_t{0};
+            if (plan_prefill(r0, nblocks, ncols, n_in, sg, &p0) || plan_prefill(r1, nblocks, ncols, n_in, sg, &p1)) return size_t{0};
             *flags = *flags || p0.sk_p > 0 || p1.sk_p > 0;
             return std::max(plan_part_bytes(p0, r1, ncols), plan_part_bytes(p1, r1, ncols));
         });
     // a captured call cannot grow the workspace: the best plan that fits it
     if (!forced && !prefill_fits(*ws, plan_part_bytes(plan, m, ncols), plan.sk_p > 0) && stream_capturing(st) &&
-        (rc = plan_prefill(m, nblocks, ncols, n_in, &plan, ws->cap[kWsPart], ws->sk != nullptr)))
+        (rc = plan_prefill(m, nblocks, ncols, n_in, sg, &plan, ws->cap[kWsPart], ws->sk != nullptr)))
         return rc;
     if ((rc = prefill_workspace(*ws, plan_part_bytes(plan, m, ncols), plan.sk_p > 0, st))) return rc;
     const uint16_t* xb = xb_in;
@@ -1936,18 +1963,18 @@ int q4_gemm_bf16in_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate
     // estimated time, or past one round of 256-row tiles stream-K over one
     // workgroup per CU, so that a last partial round does not double the time
     // (about 1.9 us a step and 53 us of partials, restarts and imbalance).
-    // Measured, n_inter 18944, n_in 3584: 64 rows up to 64 (50 us; 256 rows take
-    // 84), 128 up to 128 (57), 256 up to 256 (90), 128 at 300 (126; stream-K 167),
-    // 192 at 512 (168; 176), 256 at 600 (204; 227) and 1000 (295; 300): stream-K
+    // Measured, n_inter 18944, n_in 3584: 64 rows up to 64 (49 us; 256 rows take
+    // 79), 128 up to 128 (57), 192 up to 192 (75; 64 rows 91), 256 up to 256 (91),
+    // 128 at 300 (126; stream-K 167), 192 at 512 (168; 176), 256 at 600 (204; 227) and 1000 (295; 300): stream-K
     // at no row count up to 1536.  n_in 5120, whose steps weigh more: stream-K at
     // 512 (223; 192 rows 236) and 1000 (414; 256 rows 414).
     // Q4_PAIR_PLAN=dp (256 rows), rows:<bm> or sk:<P> chooses.
-    const int cus = num_cus(), G = n_in / 64;
+    const int cus = num_cus(), G = n_in / 64, sg = w4_groups(gm, n_in);
     const long nblocks = (n_inter + 127) / 128;
     auto plan = [&](int rows, int* height) {                       // stream-K's workgroups, 0: tiles of *height rows
         double best = 1e30;
         for (int h : {256, 192, 128, 64}) {
-            const double est = prefill_dp_us(h, (rows + h - 1) / h * nblocks, G, cus);
+            const double est = prefill_dp_us(h, (rows + h - 1) / h * nblocks, G, cus, sg, G);
             if (est < best) {
                 best = est;
                 *height = h;
@@ -1955,7 +1982,7 @@ int q4_gemm_bf16in_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate
         }
         const long tiles = (rows + 255) / 256 * nblocks;
         const int p = static_cast<int>(std::min<long>(cus >= 8 ? cus / 8 * 8 : cus, tiles * G));
-        return tiles > cus && 1.9 * static_cast<double>(tiles * G) / p + 53.0 < best ? p : 0;
+        return tiles > cus && (1.9 + prefill_copy_us(256, sg, G)) * static_cast<double>(tiles * G) / p + 53.0 < best ? p : 0;
     };
     int bm = 256, P = plan(m, &bm);
     const long tiles = (m + 255) / 256 * nblocks, T = tiles * G;
@@ -1973,7 +2000,7 @@ int q4_gemm_bf16in_gate_up_silu_dev(const uint32_t* gate_w, const uint16_t* gate
     Workspace* ws;
     if ((rc = stream_workspace(st, &ws))) return rc;
     if (!env) {
-        prefill_reserve(*ws, {static_cast<int>(nblocks), 0, n_in}, m, st, [&](int, int r1, bool* flags) {
+        prefill_reserve(*ws, {static_cast<int>(nblocks), 0, n_in, sg}, m, st, [&](int, int r1, bool* flags) {
             int height;
             const int p = plan(r1, &height);
             *flags = *flags || p > 0;
