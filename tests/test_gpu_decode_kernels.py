@@ -269,6 +269,31 @@ def test_attention_many_parts_of_one_chunk(torch, lib, nh, nkv, d):
         assert int(scratch[-512 * 32:].view(torch.int32).abs().sum().item()) == 0, p
 
 
+@pytest.mark.parametrize("nh,nkv,d", [(6, 3, 128), (28, 4, 64)])
+def test_attention_merge_rounds(torch, lib, nh, nkv, d):
+    """Part counts on both sides of each round of the merge: 36 at first, 32
+    in each later one, up to 8 in the last.  The values are the position in
+    one dimension and 1 in the others, so that a part left out or taken twice
+    shows in both; equal scores make the exact result the positions' mean."""
+    dev = torch.device("cuda")
+    cap = 110 * 64
+    kc = torch.zeros(nkv, cap, d, dtype=torch.float16, device=dev)
+    vc = torch.ones(nkv, cap, d, dtype=torch.float16, device=dev)
+    vc[:, :, 0] = (torch.arange(cap, device=dev) // 64).to(torch.float16)
+    tq = torch.ones(nh * d, device=dev)
+    out = torch.empty(nh * d, device=dev)
+    scratch = torch.zeros(lib.q4_attention_scratch_floats(nh, d, cap), device=dev)
+    for parts in (35, 36, 37, 43, 44, 45, 52, 53, 67, 68, 69, 75, 76, 77, 84, 85):
+        pos = torch.tensor([parts * 64 - 1], dtype=torch.int64, device=dev)
+        rc = lib.q4_attention_dev(tq.data_ptr(), kc.data_ptr(), vc.data_ptr(), pos.data_ptr(), out.data_ptr(),
+                                  scratch.data_ptr(), nh, nkv, d, cap, 0.125, sp(torch))
+        assert rc == 0, q4.last_error(lib)
+        got = out.view(nh, d).cpu().numpy().astype(np.float64)
+        # every weight is 1: whole numbers up to 2^24 in fp32, then one division
+        assert np.array_equal(got[:, 1:], np.ones((nh, d - 1))), parts
+        assert np.abs(got[:, 0] - (parts - 1) / 2).max() <= parts * 2.0 ** -23, parts
+
+
 def test_attention_long_context(torch, lib):
     """Contexts past one round of the merge's loads (36 chunks of 64
     positions): up to 79 chunks, the ones past the first round merged by
