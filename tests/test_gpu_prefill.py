@@ -86,6 +86,25 @@ def _operands(seed, m, n_out, n_in):
     return dev, exact
 
 
+@pytest.mark.parametrize("m,n_out,n_in,splits", [(190, 8768, 3392, 5), (434, 8768, 3392, 3), (512, 8768, 3392, 3),
+                                                 (512, 3584, 3584, 4)])
+def test_gemm_bf16_default_plan(monkeypatch, m, n_out, n_in, splits):
+    """The splits the call itself takes, told by the order of its sums: with
+    an odd group count (53; scales copied a group at a time) a few splits of
+    high tiles, as two 64-row workgroups to a CU took twice as long."""
+    import torch
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("plans of 256 CUs")
+    print(f"default plan m={m} n={n_out} k={n_in}", flush=True)
+    (tw, ts, tb, tx), _ = _operands(705, m, n_out, n_in)
+    got = {}
+    for s in (None, *range(1, 7)):
+        _plan(monkeypatch, s and f"rows:192:{s}")
+        got[s] = q4.gemm_bf16_dev(tw, ts, tb, tx)
+    torch.cuda.synchronize()
+    assert [s for s in range(1, 7) if torch.equal(got[None], got[s])] == [splits]
+
+
 # Stream-K plans: P workgroups over tiles x G iterations, in 8 XCD groups
 # when P is a multiple of 8 and there are at least 8 tiles (one group
 # otherwise).  P = tiles gives every workgroup one whole tile (no partials);
