@@ -41,8 +41,8 @@
 //
 // Measured (Qwen2.5-7B shapes, graph replays, against the earlier form: x
 // operand in the register ring, a launch per matrix and per 8 rows): MLP
-// block 61.5 -> 50.5 us at 3..8 rows, 115 -> 64 at 16; q/k/v at 16 rows 57
-// -> 15; down_proj at 16 rows 49 -> 25.  What bounds it now is a window's
+// block 60 -> 47 us at 3..8 rows, 114 -> 62 at 16; q/k/v at 16 rows 58 ->
+// 14.5; down_proj at 16 rows 48.5 -> 23.4.  What bounds it now is a window's
 // instructions and LDS traffic: with the copies and the weights' loads taken
 // out it still needs 0.5 us a window (0.75 paired) where the weights alone
 // need 0.43 (0.86), and the two overlap only in part across the barrier.
