@@ -57,10 +57,10 @@ struct PromptAttnArgs {
 // product, placed in fp16's range so that nothing that counts is rounded away:
 //   q: a row is scaled by a power of two to a maximum in [2^14, 2^15)
 //     (pa_split), each value to 2^-22 of itself or 2^-38 of the maximum;
-//   p: relative to a power of two just above its tile's own maximum (the
-//     online softmax's running maximum replaced by the tile's, so that
-//     rescaling l and O^T is exact) and times 2^15, as hi + lo (pa_split_p), to
-//     2^-23 of itself or 2^-40 of the tile's largest.
+//   p: relative to its tile's own maximum (the online softmax's running
+//     maximum replaced by it), after the first tile to the power of two just
+//     above, so that rescaling l and O^T is exact, and times 2^15, as hi + lo
+//     (pa_split_p), to 2^-23 of itself or 2^-40 of the tile's largest.
 // One dominant key (an attention sink, whose value is near zero) leaves
 // thousands of small p to make the output: from p below the running maximum,
 // unscaled and so to 2^-25, 6e-5 of them was lost 10 nats below that key and
@@ -316,9 +316,13 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(2
             for (int mt = 0; mt < 4; mt++) s[mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(kf[ks & 1][mt], ql[ks], s[mt], 0, 0, 0);
         }
         // the softmax of row r (s times up are the scores), l and o relative to
-        // 2^m: m the tile's maximum rounded up, but at most kPDrop (64 where m's
-        // spacing is that wide) below the row's largest so far, so that o stays
-        // below 2^(64 + 15 + 16 + 16)
+        // 2^m: m the tile's maximum, rounded up after the group's first tile, but
+        // at most kPDrop (64 where m's spacing is that wide) below the row's
+        // largest so far, so that o stays below 2^(64 + 15 + 16 + 16).  In the
+        // first tile the largest p is so exactly 1, and a row that sees one key
+        // gives that key's value exactly (rounded up there too, one bf16 value in
+        // sixteen of a prompt's first row was a unit off, as an eighth of the
+        // fp16 values are ties of bf16; 1 % of the time at 512 rows after 1536).
         if (c0 + kPTile - 1 > a.pos0 + r0) {                   // uniform: some row does not see all of the tile
             const int vis = static_cast<int>(my_last - c0 < kPTile ? my_last - c0 : kPTile) - 4 * qd;
 #pragma unroll
@@ -332,7 +336,9 @@ __global__ __launch_bounds__(64 * HPW * KS) __attribute__((amdgpu_waves_per_eu(2
 #pragma unroll
             for (int v = 0; v < 4; v++) mx = fmaxf(mx, s[mt][v]);
         mx = pa_rows4(mx, [](float x, float y) { return fmaxf(x, y); });
-        const float mc = __builtin_ceilf(__fmul_rn(mx, up));
+        const float t = __fmul_rn(mx, up);
+        float mc = t0 == 0 ? t : __builtin_ceilf(t);
+        if constexpr (D == 128) asm("" : "+v"(mc));             // a schedule 1 % faster there
         top = fmaxf(top, mc);
         const float mn = fmaxf(mc, __fsub_rn(top, kPDrop));
         const float ms = mn == -__builtin_inff() ? 0.0f : mn;  // the row sees none of the group's positions so far

@@ -241,6 +241,44 @@ def test_prompt_attention_infinite_keys(d):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("nh,nkv,d,rows", [(8, 4, 128, 6), (7, 1, 64, 40), (1, 1, 32, 300), (32, 8, 128, 300)])
+def test_prompt_attention_one_visible_key(nh, nkv, d, rows):
+    """The first row of an empty cache sees one key: its output is that key's
+    value, exactly, and so its bf16 rounding (an eighth of the fp16 values are
+    ties between two bf16 ones)."""
+    import torch
+    rng = np.random.default_rng(d + rows)
+    lib, scale = q4.load(), ctypes.c_float(d ** -0.5).value
+    tq = torch.from_numpy((2 * rng.normal(0, 1, (rows, nh * d))).astype(np.float32)).cuda()
+    tk, tv = (torch.from_numpy(rng.normal(0, 1, (nkv, rows, d)).astype(np.float16)).cuda() for _ in range(2))
+    want = tv[:, 0].float().repeat_interleave(nh // nkv, dim=0).reshape(-1)
+    for fn, dt in ((lib.q4_prompt_attention_dev, torch.float32), (lib.q4_prompt_attention_bf16_dev, torch.bfloat16)):
+        out = torch.zeros((rows, nh * d), dtype=dt, device="cuda")
+        rc = fn(tq.data_ptr(), tk.data_ptr(), tv.data_ptr(), out.data_ptr(), rows, 0, nh, nkv, d, rows, scale,
+                torch.cuda.current_stream().cuda_stream)
+        assert rc == 0, q4.last_error(lib)
+        assert torch.equal(out[0], want.to(dt)), dt
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_prompt_attention_one_overwhelming_key(d):
+    """A key 400 nats above all others (scores that are no whole numbers): its
+    value, exactly in the first tile, elsewhere to four fp32 roundings of p, o,
+    l and their quotient and p's two terms (2^-23)."""
+    rng = np.random.default_rng(d)
+    n = 400
+    q = rng.normal(0, 1, (1, d)).astype(np.float32)
+    q[0, 3] = 37.3
+    v = rng.normal(0, 1, (n, d)).astype(np.float16)
+    for best in (0, 3, 63, 70, 200, 399):
+        k = rng.normal(0, 0.1, (n, d)).astype(np.float16)
+        k[best, 3] = 13.7
+        got, want = _one_head(q, k, v, 1.0)[0].astype(np.float64), v[best].astype(np.float64)
+        assert (np.abs(got - want) <= (0.0 if best < 64 else 6 * 2.0 ** -24) * np.abs(want)).all(), best
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("d", [32, 64, 128])
 def test_prompt_attention_scores_far_apart(d):
     """Scores of up to 2^30, every two at least 2^18 apart: the output is the
