@@ -65,7 +65,7 @@ struct PromptAttnArgs {
 // thousands of small p to make the output: from p below the running maximum,
 // unscaled and so to 2^-25, 6e-5 of them was lost 10 nats below that key and
 // 0.19 at 18; now 2e-6, as with fp32 probabilities, in the same time (45 us
-// against 46 for the case below; 3 to 4 % more at head_dim 64).
+// against 46 for the case below; 1 to 2 % more at head_dim 64).
 // q is multiplied by scale * log2(e) first and the softmax taken with exp2,
 // which is exp of the scaled score.  Workgroups of the last rows, which see
 // the most positions, are launched first, over all kv heads (block rows are the
